@@ -33,6 +33,13 @@ int qtt_hip_check(qtt_ctx* ctx, hipError_t e, const char* what) {
   } while (0)
 
 double* qtt_scratch(qtt_ctx* ctx, size_t bytes) {
+  if (ctx->scratch_stream && ctx->scratch_stream != ctx->stream) {
+    if (hipStreamWaitEvent(ctx->stream, ctx->scratch_ev, 0) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    ctx->scratch_stream = nullptr;
+  }
   if (bytes <= ctx->scratch_bytes) return ctx->d_scratch;
   if (ctx->d_scratch) {
     (void)hipStreamSynchronize(ctx->stream);
@@ -48,6 +55,16 @@ double* qtt_scratch(qtt_ctx* ctx, size_t bytes) {
   }
   ctx->scratch_bytes = sz;
   return ctx->d_scratch;
+}
+
+int qtt_scratch_queued(qtt_ctx* ctx) {
+  if (!ctx->scratch_ev) {
+    const int rc = qtt_hip_check(ctx, hipEventCreateWithFlags(&ctx->scratch_ev, hipEventDisableTiming), "scratch event");
+    if (rc) return rc;
+  }
+  const int rc = qtt_hip_check(ctx, hipEventRecord(ctx->scratch_ev, ctx->stream), "scratch event");
+  if (!rc) ctx->scratch_stream = ctx->stream;
+  return rc;
 }
 
 // ---------------------------------------------------------------------------
@@ -300,6 +317,7 @@ static void ctx_free(qtt_ctx* ctx) {
   (void)hipStreamSynchronize(ctx->stream);
   if (ctx->d_scratch) (void)hipFree(ctx->d_scratch);
   if (ctx->d_sync) (void)hipFree(ctx->d_sync);
+  if (ctx->scratch_ev) (void)hipEventDestroy(ctx->scratch_ev);
   if (ctx->d_flag) (void)hipFree(ctx->d_flag);
   if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
   delete ctx;
@@ -493,6 +511,7 @@ void qtt_net_destroy(qtt_net* n) {
   if (n->d_pack32) (void)hipFree(n->d_pack32);
   if (n->d_desc) (void)hipFree(n->d_desc);
   if (n->d_env) (void)hipFree(n->d_env);
+  tree_state_free(n->tree);
   qtt_ctx* c = n->ctx;
   delete n;
   ctx_release(c);

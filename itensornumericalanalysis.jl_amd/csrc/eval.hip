@@ -12,6 +12,7 @@
 // the one its digit selects.  The per-lane vectors live in LDS ([i][lane]
 // layout, conflict free).
 #include "qtt_internal.h"
+#include "tree.h"
 
 #include <cstring>
 
@@ -500,62 +501,6 @@ __global__ void pack_split_kernel(const double* __restrict__ pack, int64_t n, fl
     float l = (float)(a - (double)h);
     out[2 * e] = h;
     out[2 * e + 1] = l;
-  }
-}
-
-// Generic tree evaluation: one thread per point, per-vertex vectors in a
-// global buffer laid out [vector element][thread] (coalesced).  Used for tree
-// topologies; the vertex contraction sums over all child index combinations.
-__global__ void __launch_bounds__(256)
-eval_tree_kernel(const double* __restrict__ data, const int64_t* __restrict__ off,
-                 const int* __restrict__ bond, TopoView t, const int64_t* __restrict__ voff,
-                 const double* __restrict__ xs, int64_t npts, double* __restrict__ out,
-                 int* __restrict__ flag, double* __restrict__ vs, int64_t nthr) {
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= nthr) return;
-  const int nc = t.ncoord;
-  for (int64_t p = gid; p < npts; p += nthr) {
-    bool bad = false;
-    for (int c = 0; c < nc; ++c) {
-      double x = xs[p * nc + c];
-      if (!(x >= 0.0)) bad = true;
-    }
-    if (bad) {
-      out[p] = __builtin_nan("");
-      flag[0] = 1;
-      continue;
-    }
-    for (int v = t.nv - 1; v >= 0; --v) {
-      const int c = t.vcoord[v];
-      int d = 0;
-      if (c >= 0) {
-        bool b2 = false;
-        uint64_t kk = digit_word(xs[p * nc + c], t.ndigits[c], b2);
-        d = (int)((kk >> (t.ndigits[c] - t.vdigit[v])) & 1u);
-      }
-      const int m = t.nch[v];
-      const int* ch = t.chs + t.choff[v];
-      int64_t pc = 1;
-      for (int k = 0; k < m; ++k) pc *= bond[ch[k]];
-      const int sd = t.sdim[v];
-      for (int pp = 0; pp < bond[v]; ++pp) {
-        const double* base = data + off[v] + ((int64_t)pp * sd + d) * pc;
-        double acc = 0.0;
-        for (int64_t j = 0; j < pc; ++j) {
-          double wgt = base[j];
-          int64_t r = j;
-          for (int k = m - 1; k >= 0 && wgt != 0.0; --k) {
-            const int b = bond[ch[k]];
-            const int idx = (int)(r % b);
-            r /= b;
-            wgt *= vs[(voff[ch[k]] + idx) * nthr + gid];
-          }
-          acc += wgt;
-        }
-        vs[(voff[v] + pp) * nthr + gid] = acc;
-      }
-    }
-    out[p] = vs[voff[0] * nthr + gid];
   }
 }
 
@@ -1185,7 +1130,18 @@ int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, doub
   TopoView tv = net->view();
   int64_t maxb = 1;
   for (int v = 0; v < t.nv; v++) maxb = std::max(maxb, net->bond[v]);
+  // a stream that is being captured takes only kernels that need no scratch
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  (void)hipStreamIsCapturing(ctx->stream, &cap);
+  const bool capturing = cap != hipStreamCaptureStatusNone;
   if (t.chain && t.ncoord <= QTT_MAX_COORD) {
+    // bonds over 32: matrix products over many rows (tree.hip).  100,003 points
+    // of a 24-site chain of bond 96: 24 us, 0.30 ms when the call also packs the
+    // cores and builds the tables, against 41.1 ms for the LDS-vector kernel,
+    // which stays for captured streams.  (Bonds over 160, which that kernel
+    // cannot take, stay refused.)
+    if (precision == QTT_F64 && maxb > 32 && maxb <= 160 && !ctx->force_lds_eval && !capturing)
+      return launch_eval_tree(ctx, net, xs, npts, out);
     int rc = precision == QTT_F64 ? ensure_pack(ctx, net) : ensure_pack32(ctx, net);
     if (rc) return rc;
     if (precision == QTT_F64 && maxb <= 32 && !ctx->force_lds_eval) {
@@ -1235,28 +1191,8 @@ int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, doub
   }
   if (precision != QTT_F64)
     return qtt_fail(ctx, QTT_EINVAL, "evaluate: float32 paths are implemented for chains only");
-  // generic tree path
-  std::vector<int64_t> voff(t.nv);
-  int64_t tot = 0;
-  for (int v = 0; v < t.nv; v++) {
-    voff[v] = tot;
-    tot += net->bond[v];
-  }
-  int64_t nthr = std::min<int64_t>(npts, 65536);
-  while (nthr > 256 && (size_t)tot * nthr * sizeof(double) > (size_t(1) << 31)) nthr /= 2;
-  size_t bytes = (size_t)tot * nthr * sizeof(double) + t.nv * sizeof(int64_t) + 64;
-  double* scr = qtt_scratch(ctx, bytes);
-  if (!scr) return qtt_fail(ctx, QTT_ENOMEM, "evaluate: scratch");
-  int64_t* d_voff = (int64_t*)(scr + (size_t)tot * nthr);
-  int rc = qtt_hip_check(ctx, hipMemcpyAsync(d_voff, voff.data(), t.nv * sizeof(int64_t), hipMemcpyHostToDevice, ctx->stream), "voff");
-  if (rc) return rc;
-  int bs = 256;
-  int64_t nb = (nthr + bs - 1) / bs;
-  eval_tree_kernel<<<dim3((unsigned)nb), bs, 0, ctx->stream>>>(net->d_data, net->d_off, net->d_bond, tv, d_voff, xs, npts, out,
-                                                               ctx->flags(), scr, nthr);
-  rc = qtt_hip_check(ctx, hipGetLastError(), "eval_tree_kernel");
-  if (rc) return rc;
-  return qtt_hip_check(ctx, hipStreamSynchronize(ctx->stream), "eval_tree sync");
+  if (capturing) return qtt_fail(ctx, QTT_EHIP, "evaluate: a tree cannot be evaluated on a captured stream");
+  return launch_eval_tree(ctx, net, xs, npts, out);
 }
 
 // f_i at its own points for a batch of networks.  Float64 chains with bonds

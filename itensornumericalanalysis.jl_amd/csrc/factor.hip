@@ -4157,6 +4157,7 @@ int truncate_batch_finish(qtt_ctx* ctx, TruncStaged& st, qtt_net* const* nets, d
     nets[i]->pack_valid = false;
     nets[i]->pack32_valid = false;
     nets[i]->env_valid = false;
+    tree_state_stale(nets[i]->tree);
     if (errs) errs[i] = im->herr[i];
   }
   int fl[2];

@@ -38,6 +38,10 @@ struct qtt_ctx {
   bool closed = false;
   double* d_scratch = nullptr;
   size_t scratch_bytes = 0;
+  // the last queued work that uses the scratch without the host waiting for
+  // it (qtt_scratch_queued): scratch_ev follows it on scratch_stream
+  hipEvent_t scratch_ev = nullptr;
+  hipStream_t scratch_stream = nullptr;
   int* d_sync = nullptr;  // counters of the dataflow kernels, zero between launches
   int sync_cap = 0;
   int cus = 256;
@@ -83,6 +87,10 @@ struct HostTopo {
   bool chain = false;
 };
 
+struct TreeState;  // packed cores and tables of the tree evaluate (tree.hip)
+void tree_state_free(TreeState* s);
+void tree_state_stale(TreeState* s);  // the cores changed
+
 struct qtt_net {
   qtt_ctx* ctx = nullptr;
   HostTopo t;
@@ -112,6 +120,7 @@ struct qtt_net {
   int64_t env_elems = 0;
   int env_tb = -1;
   bool env_valid = false;
+  TreeState* tree = nullptr;
   // Networks made by one apply batch share two device allocations (cores;
   // offsets, topology and bonds): d_data, d_off, d_topo and d_bond point into
   // them, and the last network destroyed frees them.  Null: own allocations.
@@ -135,7 +144,10 @@ struct qtt_mpo {
 int qtt_fail(qtt_ctx* ctx, int code, const std::string& msg);
 TopoView topo_view(const int* d_topo, const HostTopo& t);
 int qtt_hip_check(qtt_ctx* ctx, hipError_t e, const char* what);
+// the context's scratch, ordered on its stream after queued work of other
+// streams that uses it
 double* qtt_scratch(qtt_ctx* ctx, size_t bytes);
+int qtt_scratch_queued(qtt_ctx* ctx);
 // a checked HostTopo from the C-ABI description; a new network with these
 // bonds (cores uninitialised)
 int topo_from_abi(qtt_ctx* ctx, const qtt_topology* tp, HostTopo& t);

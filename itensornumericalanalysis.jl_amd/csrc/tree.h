@@ -1,0 +1,8 @@
+// Batched contraction of a tree network at many points, vertex by vertex
+// (tree.hip; used by the evaluate of trees and wide chains).
+#pragma once
+#include "qtt_internal.h"
+
+// Evaluate float64 networks of any tree (nv >= 1, any coordinates): device
+// points and values, queued on the context's stream.
+int launch_eval_tree(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, double* out);

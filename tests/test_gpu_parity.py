@@ -191,6 +191,48 @@ def test_eval_tree(q, po, eng, rng):
     assert rel_l2(q.evaluate(f, xs), oracle_eval(po, f, xs)) < TOL
 
 
+@pytest.mark.parametrize("npts", [1, 7, 129, 3000])
+@pytest.mark.parametrize("case", ["chain33", "chain97", "star", "comb_odd", "six_coordinates", "one_vertex",
+                                  "no_digit"])
+def test_eval_vertex_products(q, po, eng, rng, case, npts):
+    # the row-tiled vertex products: bonds around the 16-wide tiles and column
+    # groups, vertices with several input legs, point counts with no table, some
+    # tables and tables on both sides, vertices without a digit, one vertex
+    grid = lambda n: q.named_grid((n, 1))
+    bond = {"chain33": 33, "chain97": 97, "star": 5, "comb_odd": 19}.get(case, 7)
+    if case == "chain33":
+        s = q.continuous_siteinds(grid(13), map_dimension=2)
+    elif case == "chain97":
+        s = q.continuous_siteinds(grid(9))
+    elif case == "star":
+        g = q.NamedGraph(list(range(8)), [(0, i) for i in range(1, 5)] + [(4, 5), (5, 6), (6, 7)])
+        s = q.continuous_siteinds(g, [[5, 0, 1], [2, 7, 4, 3, 6]])
+    elif case == "comb_odd":
+        s = q.continuous_siteinds(q.named_comb_tree((3, 4)), [[(i, j) for j in range(1, 5)] for i in range(1, 4)])
+    elif case == "six_coordinates":
+        s = q.continuous_siteinds(grid(12), map_dimension=6)
+    elif case == "one_vertex":
+        s = q.continuous_siteinds(grid(1), [[], [], [], [], [(1, 1)]])
+    else:
+        s = q.continuous_siteinds(q.named_comb_tree((3, 3)), [[(1, 3), (1, 2)], [(3, 2), (2, 3)]])
+    f = q.random_itn(s, link_space=bond, rng=rng, normalize_cores=True)
+    xs = rng.uniform(0, 1, (npts, s.dimension()))
+    xs[::5] = np.floor(4 * xs[::5]) / 4
+    xs[-1] = 1.0
+    ref = oracle_eval(po, f, xs)
+    y = q.evaluate(f, xs)
+    # a sum of products through n vertices of K terms each: error below
+    # n sqrt(K) eps of the largest value
+    assert np.max(np.abs(y - ref)) < TOL * np.max(np.abs(ref))
+    # the kept tables serve the next call; a smaller call needs smaller ones
+    assert np.array_equal(q.evaluate(f, xs), y)
+    assert np.allclose(q.evaluate(f, xs[:3]), y[:3], rtol=0, atol=TOL * np.max(np.abs(ref)))
+    bad = xs[:1].copy()
+    bad[0, 0] = -1.0
+    with pytest.raises(q.DigitMapError):
+        q.evaluate(f, bad)
+
+
 def test_eval_edge_points(q, po, eng):
     L = 10
     s = q.continuous_siteinds(q.named_grid((L, 1)))
