@@ -69,12 +69,14 @@ struct TreeJob {
   int kc, kper;      // chunks of k blocks (one workgroup each) and blocks per chunk
   int dmode;         // digit of a row: 0 none (slice 0), 1 bit dshift of the row, 2 of a point's coordinate
   int dshift, coord, nc, ndig;
-  int unit0;         // first workgroup of this vertex
   TreeLeg leg[TREE_MAX_IN];
 };
 
+// (the arguments lie in host memory: unit0, the vertices' first workgroups,
+// apart from the jobs, so that a workgroup finds its vertex with one load)
 struct TreeJobs {
   int n;
+  int unit0[TREE_JOBS];
   TreeJob job[TREE_JOBS];
 };
 static_assert(sizeof(TreeJobs) <= 4096, "kernel arguments");
@@ -204,10 +206,11 @@ __global__ void __launch_bounds__(256) tree_vertex_kernel(TreeJobs js) {
   __shared__ int rows[TREE_ROWS + 32];
   __shared__ int cnt[2];
   int jj = 0;
-  while (jj + 1 < js.n && (int)blockIdx.x >= js.job[jj + 1].unit0) ++jj;
+#pragma unroll
+  for (int i = 1; i < TREE_JOBS; ++i) jj += (i < js.n && (int)blockIdx.x >= js.unit0[i]) ? 1 : 0;
   const TreeJob& J = js.job[jj];
   const int tid = threadIdx.x;
-  int unit = (int)blockIdx.x - J.unit0;
+  int unit = (int)blockIdx.x - js.unit0[jj];
   const int kc = unit % J.kc;
   unit /= J.kc;
   const int ng = unit % J.ngrp, rb = unit / J.ngrp;
@@ -644,7 +647,7 @@ struct Level {
       J.out = part + part_used;
       part_used += n * J.kc;
     }
-    J.unit0 = units;
+    js.unit0[js.n] = units;
     units += (int)((R + TREE_ROWS - 1) / TREE_ROWS) * p.ngrp * J.kc;
     js.job[js.n++] = J;
     return QTT_OK;

@@ -331,6 +331,37 @@ def _compare_networks(q, po, g_dev, ref_cores, f, rng, tol=TOL, npts=4000):
     return float(np.max(np.abs(y - yr)) / np.max(np.abs(yr)))
 
 
+@pytest.mark.parametrize("case", ["one_vertex", "chain_small", "chain_33_16", "chain_130_150", "comb", "comb_48_17",
+                                  "star", "no_digit"])
+def test_inner_vertex_products(q, po, eng, rng, case):
+    # bonds around the 16-wide tiles and the 128-wide slabs, several children
+    # (mode products before the closing one), one vertex, vertices without a
+    # digit; positive cores, so the sum does not cancel
+    ba, bb = {"chain_small": (3, 2), "chain_33_16": (33, 16), "chain_130_150": (130, 150), "comb": (20, 33),
+              "comb_48_17": (48, 17)}.get(case, (7, 5))
+    grid = lambda n: q.named_grid((n, 1))
+    if case == "one_vertex":
+        s = q.continuous_siteinds(grid(1))
+    elif case.startswith("chain"):
+        s = q.continuous_siteinds(grid(8), map_dimension=2)
+    elif case.startswith("comb"):
+        s = q.continuous_siteinds(q.named_comb_tree((3, 3)), [[(i, j) for j in range(1, 4)] for i in range(1, 4)])
+    elif case == "star":
+        g = q.NamedGraph(list(range(7)), [(0, i) for i in range(1, 5)] + [(4, 5), (4, 6)])
+        s = q.continuous_siteinds(g, [[5, 0, 1, 2], [3, 6, 4]])
+    else:
+        s = q.continuous_siteinds(q.named_comb_tree((3, 3)), [[(1, 3), (1, 2)], [(3, 2)]])
+    nets = []
+    for bond in (ba, bb):
+        f = q.random_itn(s, link_space=bond, rng=rng)
+        f.set_cores([np.abs(c) / c.size ** 0.5 for c in f.cores])
+        nets.append(f)
+    t = nets[0].topo
+    ref = po.inner(t.parent, t.sdim, nets[0].cores, nets[1].cores)
+    # sums of positive terms: relative error at most (vertices x terms) eps
+    assert abs(q.inner(*nets) - ref) <= TOL * abs(ref)
+
+
 def test_apply_exact_matches_oracle(q, po, eng, rng):
     s = q.continuous_siteinds(q.named_comb_tree((2, 5)))
     f = q.random_itn(s, link_space=3, rng=rng)
