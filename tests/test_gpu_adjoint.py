@@ -130,3 +130,77 @@ def test_apply_grad_chain_rule(q, po, eng, rng):
     rg = po.eval_grad(t.parent, t.sdim, C, t.vcoord, t.vdigit, t.Lc, xs, yb)
     rfb, _ = po.contract_adjoint(t.parent, t.sdim, op.cores, f.cores, rg, want_w=False)
     assert _rel(fb, rfb) < 1e-11
+
+
+@pytest.mark.parametrize("npts", [1, 6, 130, 4500])
+@pytest.mark.parametrize("case", ["bond1", "bond17", "bond33", "bond53", "odd_2d", "no_digit", "one_vertex", "six_coordinates"])
+def test_gradient_chain_rows(q, po, eng, rng, case, npts):
+    # chains by rows: no tables, tables and per-point sites between them, tables
+    # on both sides; bonds around the 16-wide tiles, vertices without a digit
+    grid = lambda n: q.named_grid((n, 1))
+    bond = int(case[4:]) if case.startswith("bond") else 9
+    if case == "odd_2d":
+        s = q.continuous_siteinds(grid(27), map_dimension=2)
+    elif case == "no_digit":
+        s = q.continuous_siteinds(grid(14), [[(j, 1) for j in (3, 2, 6, 5)], [(j, 1) for j in (9, 8, 11, 13)]])
+    elif case == "one_vertex":
+        s = q.continuous_siteinds(grid(1))
+    elif case == "six_coordinates":
+        s = q.continuous_siteinds(grid(12), map_dimension=6)
+    else:
+        s = q.continuous_siteinds(grid(11))
+    f = q.random_itn(s, link_space=bond, rng=rng, normalize_cores=True)
+    f.set_cores([c * math.sqrt(c.shape[0] * c.shape[1]) for c in f.cores])
+    xs = rng.uniform(0, 1, (npts, s.dimension()))
+    xs[-1] = 1.0
+    yb = rng.standard_normal(npts)
+    t = f.topo
+    ref = po.eval_grad(t.parent, t.sdim, f.cores, t.vcoord, t.vdigit, t.Lc, xs, yb)
+    g = q.eval_grad(f, xs, yb)
+    assert _rel(g, ref) < TOL
+    assert all(np.array_equal(a, b) for a, b in zip(g, q.eval_grad(f, xs, yb)))
+
+
+@pytest.mark.parametrize("bond", [7, 30])
+@pytest.mark.parametrize("spread", ["one_point", "few_points", "one_cell"])
+def test_gradient_chain_long_runs(q, po, eng, rng, bond, spread):
+    # many points on the same table rows: runs of equal entries over many groups
+    s = q.continuous_siteinds(q.named_grid((16, 1)), map_dimension=2)
+    f = q.random_itn(s, link_space=bond, rng=rng, normalize_cores=True)
+    n = 5000
+    if spread == "one_point":
+        xs = np.tile([[0.3, 0.8]], (n, 1))
+    elif spread == "few_points":
+        xs = rng.uniform(0, 1, (3, 2))[rng.integers(0, 3, n)]
+    else:
+        xs = 0.5 + rng.uniform(0, 2.0 ** -7, (n, 2))
+    yb = rng.uniform(0.5, 1.5, n)
+    t = f.topo
+    ref = po.eval_grad(t.parent, t.sdim, f.cores, t.vcoord, t.vdigit, t.Lc, xs, yb)
+    assert _rel(q.eval_grad(f, xs, yb), ref) < TOL
+
+
+def test_gradient_chain_unused_slices(q, po, eng, rng):
+    # core entries that no point's digits select may be anything, infinite
+    # included; a point outside the domain counts for nothing and is reported
+    s = q.continuous_siteinds(q.named_grid((14, 1)), map_dimension=2)
+    f = q.random_itn(s, link_space=6, rng=rng, std=0.5)
+    xs = rng.uniform(0, 0.5, (3000, 2))
+    yb = rng.standard_normal(3000)
+    t = f.topo
+    ref = po.eval_grad(t.parent, t.sdim, f.cores, t.vcoord, t.vdigit, t.Lc, xs, yb)
+    cores = [c.copy() for c in f.cores]
+    cores[0][:, 1] = np.inf
+    cores[1][2, 1] = np.nan
+    h = q.ITensorNetworkFunction(s, cores)
+    g = q.eval_grad(h, xs, yb)
+    for v in range(t.nv):
+        used = g[v][:, :1] if v < 2 else g[v]
+        want = ref[v][:, :1] if v < 2 else ref[v]
+        assert np.all(np.isfinite(used))
+        assert np.linalg.norm(used - want) < TOL * max(np.linalg.norm(want), 1e-3)
+    assert all(np.all(g[v][:, 1] == 0) for v in range(2))
+    xs[5, 1] = np.nan
+    from itensornumericalanalysis_jl_amd import _capi
+    with pytest.raises(_capi.EngineError):
+        q.eval_grad(f, xs, yb)
