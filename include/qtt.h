@@ -45,7 +45,8 @@ extern "C" {
 #define QTT_EHIP 4
 #define QTT_ENOCONV 5
 
-/* arithmetic of the bulk contractions: the exact contraction and the mode
+/* arithmetic of the bulk contractions (evaluate takes all three and computes in
+ * float64, the fastest of them here): the exact contraction and the mode
  * products of the truncation sweep (its QR, SVD and cutoff are always FP64, and
  * so is the apply of a kept Q: a QR move of a matrix beyond LDS keeps its
  * reflectors and the move consuming that core applies them in FP64) */

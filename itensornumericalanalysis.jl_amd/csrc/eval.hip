@@ -33,10 +33,6 @@ __device__ inline double bitsel(double a, double b, uint64_t mask) {
   return __longlong_as_double((long long)((ua & ~mask) | (ub & mask)));
 }
 
-__device__ inline float bitself(float a, float b, uint32_t mask) {
-  return __uint_as_float((__float_as_uint(a) & ~mask) | (__float_as_uint(b) & mask));
-}
-
 // pack chain site k as P[r][lpad][2] (lpad = bond[k] rounded up to 4, zero padded)
 __global__ void pack_chain_kernel(const double* __restrict__ data, const int64_t* __restrict__ off,
                                   const int* __restrict__ bond, const int* __restrict__ sdim,
@@ -388,111 +384,6 @@ eval_chain_reg2_kernel(const double* __restrict__ pack, const int64_t* __restric
   if (bad0 || bad1) flag[0] = 1;
 }
 
-// float32 variants of the chain kernel.  SPLIT keeps each operand as a
-// (hi, lo) float pair and accumulates in float-float (Dekker/Knuth error-free
-// transformations), PLAIN is ordinary float32.
-struct ff {
-  float h, l;
-};
-
-// The error-free transformations need every + and * rounded on its own:
-// contraction into FMA (hipcc's default) would silently drop the low word.
-__device__ inline ff two_sum(float a, float b) {
-#pragma clang fp contract(off)
-  float s = a + b;
-  float bb = s - a;
-  float e = (a - (s - bb)) + (b - bb);
-  return {s, e};
-}
-
-__device__ inline ff ff_fma(float ah, float al, float bh, float bl, ff c) {
-  // c + (ah + al) * (bh + bl), dropping al * bl
-#pragma clang fp contract(off)
-  float p = ah * bh;
-  float pe = __builtin_fmaf(ah, bh, -p);
-  pe = __builtin_fmaf(ah, bl, pe);
-  pe = __builtin_fmaf(al, bh, pe);
-  ff s = two_sum(c.h, p);
-  float e = s.l + c.l + pe;
-  float h = s.h + e;
-  return {h, e - (h - s.h)};
-}
-
-template <bool SPLIT>
-__global__ void __launch_bounds__(256)
-eval_chain_f32_kernel(const float* __restrict__ pack, const int64_t* __restrict__ poff,
-                      const int* __restrict__ bond, TopoView t, const double* __restrict__ xs,
-                      int64_t npts, double* __restrict__ out, int* __restrict__ flag, int vstride) {
-  extern __shared__ float ldsf[];
-  const int tid = threadIdx.x;
-  const int bs = blockDim.x;
-  const int64_t p = (int64_t)blockIdx.x * bs + tid;
-  const bool active = p < npts;
-  const int nc = t.ncoord;
-  bool bad = false;
-  uint64_t kw[QTT_MAX_COORD] = {0, 0, 0, 0};
-#pragma unroll
-  for (int c = 0; c < QTT_MAX_COORD; ++c)
-    if (c < nc) kw[c] = digit_word(active ? xs[p * nc + c] : 0.0, t.ndigits[c], bad);
-  // vectors as (hi, lo) pairs: [i][lane][2]
-  float* v = ldsf + 2 * tid;
-  float* w = ldsf + (size_t)2 * vstride * bs + 2 * tid;
-  v[0] = 1.0f;
-  v[1] = 0.0f;
-  for (int k = t.nv - 1; k >= 0; --k) {
-    const int chil = bond[k];
-    const int chir = (k == t.nv - 1) ? 1 : bond[k + 1];
-    const int c = t.vcoord[k];
-    int d = 0;
-    if (c >= 0) {
-      const uint64_t kk = c == 0 ? kw[0] : c == 1 ? kw[1] : c == 2 ? kw[2] : kw[3];
-      d = (int)((kk >> (t.ndigits[c] - t.vdigit[k])) & 1u);
-    }
-    // packed float layout: [r][lpad][s][hi, lo]
-    const float* __restrict__ P = pack + 2 * poff[k];
-    const int lpad = (chil + 3) & ~3;
-    for (int l0 = 0; l0 < chil; l0 += 4) {
-      ff a0[4], a1[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a0[i] = a1[i] = {0.0f, 0.0f};
-      const float* __restrict__ q = P + 4 * l0;
-      for (int r = 0; r < chir; ++r) {
-        const float vh = v[(size_t)2 * r * bs];
-        const float vl = SPLIT ? v[(size_t)2 * r * bs + 1] : 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (SPLIT) {
-            a0[i] = ff_fma(q[4 * i], q[4 * i + 1], vh, vl, a0[i]);
-            a1[i] = ff_fma(q[4 * i + 2], q[4 * i + 3], vh, vl, a1[i]);
-          } else {
-            a0[i].h = __builtin_fmaf(q[4 * i], vh, a0[i].h);
-            a1[i].h = __builtin_fmaf(q[4 * i + 2], vh, a1[i].h);
-          }
-        }
-        q += 4 * lpad;
-      }
-      const uint32_t fmask = 0u - (uint32_t)d;
-      float sh[4], sl[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        sh[i] = bitself(a0[i].h, a1[i].h, fmask);
-        sl[i] = bitself(a0[i].l, a1[i].l, fmask);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (l0 + i < chil) {
-          w[(size_t)2 * (l0 + i) * bs] = sh[i];
-          w[(size_t)2 * (l0 + i) * bs + 1] = sl[i];
-        }
-    }
-    float* tmp = v;
-    v = w;
-    w = tmp;
-  }
-  if (active) out[p] = bad ? __builtin_nan("") : (double)v[0] + (double)v[1];
-  if (bad) flag[0] = 1;
-}
-
 // float32 (hi, lo) pack of the float64 pack: [r][lpad][s] -> [r][lpad][s][2]
 __global__ void pack_split_kernel(const double* __restrict__ pack, int64_t n, float* __restrict__ out) {
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
@@ -501,6 +392,88 @@ __global__ void pack_split_kernel(const double* __restrict__ pack, int64_t n, fl
     float l = (float)(a - (double)h);
     out[2 * e] = h;
     out[2 * e + 1] = l;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// A few points (chains of bonds <= 32): CHI lanes per point, a lane per entry of
+// the vector.  With a lane per point one wavefront walks all sites, each row
+// of each behind scalar loads (40 sites of bond 16: 190 us whether 1 or 30,000
+// points); here a site is CHI multiply-adds per lane, the vector through LDS,
+// and the rows of the next sites, known from the digits alone, are on their
+// way meanwhile.  The sums run in the order of chain1_site, so the values are
+// bit for bit those of the other kernels.  The cores are read where they lie
+// (no packed copy).  What bounds it with more points: each lane reads its own
+// core row, 64 accesses per load.
+// ---------------------------------------------------------------------------
+template <int CHI>
+__global__ void __launch_bounds__(64)
+eval_chain_few_kernel(const double* __restrict__ data, const int64_t* __restrict__ off, const int* __restrict__ bond,
+                      TopoView t, const double* __restrict__ xs, int64_t npts, double* __restrict__ out,
+                      int* __restrict__ flag) {
+  typedef double f64x2 __attribute__((ext_vector_type(2)));
+  constexpr int D = CHI == 32 ? 2 : 3;  // sites in flight
+  __shared__ __align__(16) double vec[64 / CHI][CHI + 2];
+  const int lane = threadIdx.x, l = lane % CHI;
+  const int64_t p = (int64_t)blockIdx.x * (64 / CHI) + lane / CHI;
+  const bool active = p < npts;
+  const int nv = t.nv, nc = t.ncoord;
+  bool bad = false;
+  uint64_t kw[QTT_MAX_COORD] = {0, 0, 0, 0};
+#pragma unroll
+  for (int c = 0; c < QTT_MAX_COORD; ++c)
+    if (c < nc) kw[c] = digit_word(active ? xs[p * nc + c] : 0.0, t.ndigits[c], bad);
+  double a[D][CHI];
+  auto fetch = [&](int i, double (&x)[CHI]) {  // the row of site nv-1-i for this lane's entry and digit
+    const int k = max(nv - 1 - i, 0);
+    const int chil = bond[k], chir = k == nv - 1 ? 1 : bond[k + 1];
+    const int c = t.vcoord[k];
+    int d = 0;
+    if (c >= 0) {
+      const uint64_t w = c == 0 ? kw[0] : c == 1 ? kw[1] : c == 2 ? kw[2] : kw[3];
+      d = (int)((w >> (t.ndigits[c] - t.vdigit[k])) & 1u);
+    }
+    const bool on = l < chil;
+    const double* T = data + off[k] + ((int64_t)(on ? l : 0) * t.sdim[k] + d) * chir;
+    if (chir & 1) {
+#pragma unroll
+      for (int e = 0; e < CHI; ++e) x[e] = (on && e < chir) ? T[e] : 0.0;
+    } else {  // (cores start at multiples of 16 bytes)
+#pragma unroll
+      for (int e = 0; e < CHI; e += 2) {
+        f64x2 q = {0.0, 0.0};
+        if (on && e < chir) q = *(const f64x2*)(T + e);
+        x[e] = q.x;
+        x[e + 1] = q.y;
+      }
+    }
+  };
+  double* v = vec[lane / CHI];
+  v[l] = l == 0 ? 1.0 : 0.0;
+#pragma unroll
+  for (int i = 0; i < D; ++i) fetch(i, a[i]);
+  for (int i0 = 0; i0 < nv; i0 += D) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      if (i0 + j < nv) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (one wavefront's LDS operations complete in order)
+        double s = 0.0;
+#pragma unroll
+        for (int e = 0; e < CHI; e += 2) {
+          const f64x2 q = *(const f64x2*)(v + e);
+          s = __builtin_fma(a[j][e], q.x, s);
+          s = __builtin_fma(a[j][e + 1], q.y, s);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        v[l] = s;
+        fetch(i0 + j + D, a[j]);
+      }
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  if (l == 0 && active) {
+    if (bad) flag[0] = 1;
+    out[p] = bad ? __builtin_nan("") : v[0];
   }
 }
 
@@ -964,14 +937,15 @@ static EnvPlan env_plan(const qtt_net* net, int tb) {
   return p;
 }
 
-// Digit sites per table when nothing is tuned: enough points that a table
-// row is reused about 32 times, at most 16.
-static int default_table_bits(int64_t npts) {
-  if (npts < (int64_t(1) << 15)) return 0;
-  int lg = 0;
-  while ((int64_t(1) << (lg + 1)) <= npts) ++lg;
-  return std::min(16, lg - 5);
-}
+// Digit sites per table when nothing is tuned: 12, from 2^15 points (below,
+// values are bit for bit those of the batch kernels, which take no tables).  Two
+// tables of 2^12 rows stay in an XCD's L2 and are built in one short launch;
+// larger ones save two sites per digit (20 us per site at 10^6 points of bond 16)
+// but their rows come from beyond the L2.  10^6 points, 40 sites of bond 16,
+// repeated / first call: 10 digits 408 / 541 us, 12 digits 337 / 468, 14 digits
+// 403 / 561, 16 digits 296 / 751, 18 digits 171 / 760.  (qtt_tune_eval weighs
+// the repeated calls alone.)
+static int default_table_bits(int64_t npts) { return npts < (int64_t(1) << 15) ? 0 : 12; }
 
 static EnvTableArgs env_table_args(const qtt_net* net, const EnvPlan& pl, bool left, double* tab) {
   const HostTopo& t = net->t;
@@ -1124,12 +1098,26 @@ int tune_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, double
   return QTT_OK;
 }
 
+// Points up to which CHI lanes per point (eval_chain_few_kernel) beat one: the
+// lane-per-point kernel takes the same time for 1 to 30,000 points, the other
+// grows with them.  Measured us, few against one lane per point: bond 5, 12
+// sites 9.0 / 13.5 at 1 point, 11.6 / 14.2 at 16,384; bond 8, 28 sites 16 / 38
+// and 35 / 38; bond 16, 40 sites 27 / 189 at 1, 84 / 197 at 8,192, 190 / 190 at
+// 16,384; bond 32, 24 sites 24 / 398, 91 / 405 at 4,096, 401 / 400 at 16,384.
+static int64_t few_points(int64_t maxb) { return maxb <= 8 ? 16384 : 12288; }
+
 int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, double* out,
                 int precision) {
   const HostTopo& t = net->t;
   TopoView tv = net->view();
   int64_t maxb = 1;
   for (int v = 0; v < t.nv; v++) maxb = std::max(maxb, net->bond[v]);
+  // The float32 precisions are for chains, and are computed in float64 as well:
+  // vector FP64 runs at the rate of (unpacked) FP32 here, and the float64 kernels
+  // with their tables are far ahead of float-float arithmetic (200,003 points
+  // of 40 sites of bond 15: 1530 us in float-float, 135 us in float64).
+  if (precision != QTT_F64 && !(t.chain && t.ncoord <= QTT_MAX_COORD))
+    return qtt_fail(ctx, QTT_EINVAL, "evaluate: float32 paths are implemented for chains only");
   // a stream that is being captured takes only kernels that need no scratch
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   (void)hipStreamIsCapturing(ctx->stream, &cap);
@@ -1140,11 +1128,22 @@ int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, doub
     // cores and builds the tables, against 41.1 ms for the LDS-vector kernel,
     // which stays for captured streams.  (Bonds over 160, which that kernel
     // cannot take, stay refused.)
-    if (precision == QTT_F64 && maxb > 32 && maxb <= 160 && !ctx->force_lds_eval && !capturing)
+    if (maxb > 32 && maxb <= 160 && !ctx->force_lds_eval && !capturing)
       return launch_eval_tree(ctx, net, xs, npts, out);
-    int rc = precision == QTT_F64 ? ensure_pack(ctx, net) : ensure_pack32(ctx, net);
+    if (maxb <= 32 && npts <= few_points(maxb) && !ctx->force_lds_eval && !ctx->eval_ppl &&
+        ctx->eval_tbits < 0 && !ctx->eval_tuned.count(eval_tune_key(maxb, npts))) {
+#define QTT_FEW_LAUNCH(C)                                                                                     \
+  eval_chain_few_kernel<C><<<dim3((unsigned)((npts + 64 / C - 1) / (64 / C))), 64, 0, ctx->stream>>>(         \
+      net->d_data, net->d_off, net->d_bond, tv, xs, npts, out, ctx->flags())
+      if (maxb <= 8) QTT_FEW_LAUNCH(8);
+      else if (maxb <= 16) QTT_FEW_LAUNCH(16);
+      else QTT_FEW_LAUNCH(32);
+#undef QTT_FEW_LAUNCH
+      return qtt_hip_check(ctx, hipGetLastError(), "eval_chain_few_kernel");
+    }
+    int rc = ensure_pack(ctx, net);
     if (rc) return rc;
-    if (precision == QTT_F64 && maxb <= 32 && !ctx->force_lds_eval) {
+    if (maxb <= 32 && !ctx->force_lds_eval) {
       // tuned shape if qtt_tune_eval measured one for this bond class and point
       // count; else two points per lane for bonds <= 16 (register room) when
       // there are enough points to fill the GPU at half the workgroup count
@@ -1160,7 +1159,7 @@ int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, doub
       if (ctx->eval_tbits >= 0) tb = ctx->eval_tbits;
       return launch_eval_env(ctx, net, xs, npts, out, maxb, ppl, wg, tb);
     }
-    // LDS: two vectors of maxb entries per lane (double, or a float pair)
+    // LDS: two vectors of maxb entries per lane
     const size_t per_lane = 2 * size_t(maxb) * sizeof(double);
     int bs = 256;
     while (bs > 64 && per_lane * bs > 160 * 1024) bs /= 2;
@@ -1170,27 +1169,14 @@ int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, doub
     if (nb > INT32_MAX) return qtt_fail(ctx, QTT_EINVAL, "evaluate: too many points");
     const size_t lds = per_lane * bs;
     if (lds > 64 * 1024) {
-      const void* fn = precision == QTT_F64 ? (const void*)eval_chain_f64_kernel
-                       : precision == QTT_F32_SPLIT ? (const void*)eval_chain_f32_kernel<true>
-                                                    : (const void*)eval_chain_f32_kernel<false>;
-      rc = qtt_hip_check(ctx, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+      rc = qtt_hip_check(ctx, hipFuncSetAttribute((const void*)eval_chain_f64_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
                          "evaluate LDS attribute");
       if (rc) return rc;
     }
-    if (precision == QTT_F64) {
-      eval_chain_f64_kernel<<<dim3((unsigned)nb), bs, lds, ctx->stream>>>(
-          net->d_pack, net->d_pack_off, net->d_bond, tv, xs, npts, out, ctx->flags(), (int)maxb);
-    } else if (precision == QTT_F32_SPLIT) {
-      eval_chain_f32_kernel<true><<<dim3((unsigned)nb), bs, lds, ctx->stream>>>(
-          (const float*)net->d_pack32, net->d_pack_off, net->d_bond, tv, xs, npts, out, ctx->flags(), (int)maxb);
-    } else {
-      eval_chain_f32_kernel<false><<<dim3((unsigned)nb), bs, lds, ctx->stream>>>(
-          (const float*)net->d_pack32, net->d_pack_off, net->d_bond, tv, xs, npts, out, ctx->flags(), (int)maxb);
-    }
+    eval_chain_f64_kernel<<<dim3((unsigned)nb), bs, lds, ctx->stream>>>(
+        net->d_pack, net->d_pack_off, net->d_bond, tv, xs, npts, out, ctx->flags(), (int)maxb);
     return qtt_hip_check(ctx, hipGetLastError(), "eval_chain kernel");
   }
-  if (precision != QTT_F64)
-    return qtt_fail(ctx, QTT_EINVAL, "evaluate: float32 paths are implemented for chains only");
   if (capturing) return qtt_fail(ctx, QTT_EHIP, "evaluate: a tree cannot be evaluated on a captured stream");
   return launch_eval_tree(ctx, net, xs, npts, out);
 }
@@ -1209,7 +1195,7 @@ int launch_eval_batch(qtt_ctx* ctx, int n, qtt_net* const* nets, const double* c
     const HostTopo& t = net->t;
     int64_t maxb = 1;
     for (int v = 0; v < t.nv; v++) maxb = std::max(maxb, net->bond[v]);
-    if (precision != QTT_F64 || !t.chain || t.ncoord > QTT_MAX_COORD || maxb > 32 || ctx->force_lds_eval) {
+    if (!t.chain || t.ncoord > QTT_MAX_COORD || maxb > 32 || ctx->force_lds_eval) {
       int rc = launch_eval(ctx, net, xs[i], npts[i], out[i], precision);
       if (rc) return rc;
       continue;

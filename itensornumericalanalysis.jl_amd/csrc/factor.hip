@@ -40,18 +40,18 @@ extern "C" int qtt_debug_times(unsigned long long* out, int n) {
   return (int)hipMemcpyFromSymbol(out, HIP_SYMBOL(qtt_phase_t), (size_t)n * 8 * sizeof(unsigned long long));
 }
 #define QTT_PHASE(step, phase) \
-  do { if (threadIdx.x == 0) qtt_phase_mark((step), (phase), wall_clock64()); } while (0)
+  do { if (threadIdx.x == 0 && blockIdx.x == 0) qtt_phase_mark((step), (phase), wall_clock64()); } while (0)
 // the move's shape in the two spare slots of its record
 #define QTT_SHAPE(step, rows, b, tr) \
-  do { if (threadIdx.x == 0 && (step) < 8192) { qtt_phase_t[(step) * 8 + 6] = (rows); qtt_phase_t[(step) * 8 + 7] = (b) | ((tr) << 20); } } while (0)
+  do { if (threadIdx.x == 0 && blockIdx.x == 0 && (step) < 8192) { qtt_phase_t[(step) * 8 + 6] = (rows); qtt_phase_t[(step) * 8 + 7] = (b) | ((tr) << 20); } } while (0)
 // Jacobi sweeps (low 16 bits) and calls (high bits) of the step opened last
 __device__ unsigned long long qtt_phase_sweeps[8192];
 extern "C" int qtt_debug_sweeps(unsigned long long* out, int n) {
   return (int)hipMemcpyFromSymbol(out, HIP_SYMBOL(qtt_phase_sweeps), (size_t)n * sizeof(unsigned long long));
 }
 #define QTT_SWEEPS(s) \
-  do { if (threadIdx.x == 0 && qtt_phase_step < 8192) qtt_phase_sweeps[qtt_phase_step] += (unsigned long long)(s) + (1ull << 16); } while (0)
-#define QTT_SWEEPS_CLEAR(step) do { if (threadIdx.x == 0 && (step) < 8192) qtt_phase_sweeps[step] = 0; } while (0)
+  do { if (threadIdx.x == 0 && blockIdx.x == 0 && qtt_phase_step < 8192) qtt_phase_sweeps[qtt_phase_step] += (unsigned long long)(s) + (1ull << 16); } while (0)
+#define QTT_SWEEPS_CLEAR(step) do { if (threadIdx.x == 0 && blockIdx.x == 0 && (step) < 8192) qtt_phase_sweeps[step] = 0; } while (0)
 #endif
 // Cycle counters inside the Jacobi rounds and QR panels (-DQTT_JACOBI_TIMING,
 // on top of the phase timestamps); each mark is a read-modify-write of global
