@@ -3169,33 +3169,63 @@ __device__ bool jacobi_coop(double* X, int n, int b, double* J, CoopJob* job, in
 }
 
 // One-sided Jacobi of a wide matrix X (n x b, n <= b, ld b, global memory)
-// preconditioned by two QRs (Drmac and Veselic; here without pivoting):
-// X^T = Q1 R1 and R1^T = Q2 R2, so X = Q2 R2 Q1^T.  The rounds run on the rows
-// of R2 (n x n) with J starting from Q2^T; X's rotated rows are then
-// (J R2) Q1^T, formed as (Q1 (J R2)^T)^T.  A truncation sweep's wide matrices
-// are numerically rank deficient (their smallest singular values are round-off
-// of the bigger ones) and their rows keep rotating for many sweeps unless
-// preconditioned: on a 256 x 384 matrix of the 3D comb operate a CPU replay of
-// the block rounds takes 35 sweeps on X, 8 on R2.  A (b x n) receives X^T and
-// keeps Q1's reflectors; Tg1, Tg2 the panels' T of the two QRs; Mq (b x n) is
-// scratch.  Same result as the Jacobi on X up to round-off (the rotations act
-// on the same row space).
+// preconditioned by two QRs (Drmac and Veselic; here with the rows sorted by
+// norm instead of pivoting): (P X)^T = Q1 R1 and R1^T = Q2 R2, so P X = Q2 R2
+// Q1^T.  The rounds run on the rows of R2 (n x n) with J starting from Q2^T P;
+// X's rotated rows are then (J R2) Q1^T, formed as (Q1 (J R2)^T)^T.  A
+// truncation sweep's wide matrices are graded, many numerically rank deficient
+// (their smallest singular values are round-off of the bigger ones): on a 256 x
+// 384 matrix of the 3D comb operate a CPU replay of the block rounds takes 35
+// sweeps on X, 8 on R2; on the 64 x 270 matrices of the kernel-operator batch
+// 13 sweeps on X, 8 on R2, 7 with the rows sorted.  And a round on R2 touches n
+// entries per row instead of b: with R2 and J in LDS (2 n^2 doubles; n <= 96)
+// a round costs about 1.2 us on one workgroup, rows of 285 in global memory 7
+// us (a 64 x 285 move of that batch: 5.5 ms -> 0.88 ms, the whole step of 512
+// functions 142 -> 85 ms).  A (b x n) receives X^T and keeps Q1's reflectors; Tg1, Tg2 the
+// panels' T of the two QRs; Mq (b x n) is scratch, sig and ord n doubles / ints.
+// Same result as the Jacobi on X up to round-off (the rotations act on the same
+// row space).
 __device__ __noinline__ bool jacobi_precond(double* X, int n_in, int b_in, double* A, double* J, double* tau,
-                                            double* Tg1, double* Tg2, double* Mq, lds_f64* pnl, int pnl_cap,
-                                            CoopJob* job, int nwg_in, double* red, int* iflag, double cut,
-                                            int max_sweeps) {
-  const int tid = threadIdx.x, bs = blockDim.x;
-  const int n = uni(n_in), b = uni(b_in), nwg = uni(nwg_in);
-  // A = X^T: tiled transposes shared with the helper workgroups
-  if (tid == 0) {
-    job->type = 10;
-    job->U = X;
-    job->D = A;
-    job->Au = 1;
-    job->rb = n;
-    job->Bu = b;
+                                            double* Tg1, double* Tg2, double* Mq, double* sig, int* ord, lds_f64* pnl,
+                                            int pnl_cap_in, CoopJob* job, int nwg_in, double* red, int* iflag,
+                                            double cut, int max_sweeps) {
+  const int tid = threadIdx.x, bs = blockDim.x, lane = tid & 63, wv = tid >> 6, nwv = bs >> 6;
+  const int n = uni(n_in), b = uni(b_in), nwg = uni(nwg_in), pnl_cap = uni(pnl_cap_in);
+  const bool coop = job != nullptr && nwg > 1;
+  // rows by decreasing norm: Mq <- P X (row r at its rank)
+  for (int r = wv; r < n; r += nwv) {
+    double s = 0.0;
+    for (int c = lane; c < b; c += 64) s = __builtin_fma(X[(int64_t)r * b + c], X[(int64_t)r * b + c], s);
+    s = sum64(s);
+    if (lane == 0) sig[r] = s == s ? s : -1.0;  // an order in any case: NaN rows last
   }
-  coop_post_run(job, nwg, iflag, pnl, (int)min<int64_t>((int64_t)((n + 63) >> 6) * ((b + 63) >> 6), nwg));
+  __syncthreads();
+  for (int r = tid; r < n; r += bs) {
+    const double s = sig[r];
+    int k = 0;
+    for (int j = 0; j < n; ++j) k += (sig[j] > s || (sig[j] == s && j < r)) ? 1 : 0;
+    ord[k] = r;
+  }
+  __syncthreads();
+  for (int r = wv; r < n; r += nwv) {
+    const double* src = X + (int64_t)ord[r] * b;
+    for (int c = lane; c < b; c += 64) Mq[(int64_t)r * b + c] = src[c];
+  }
+  __syncthreads();
+  // A = (P X)^T: tiled transposes, shared with the helper workgroups
+  if (coop) {
+    if (tid == 0) {
+      job->type = 10;
+      job->U = Mq;
+      job->D = A;
+      job->Au = 1;
+      job->rb = n;
+      job->Bu = b;
+    }
+    coop_post_run(job, nwg, iflag, pnl, (int)min<int64_t>((int64_t)((n + 63) >> 6) * ((b + 63) >> 6), nwg));
+  } else {
+    gather_tiles(Mq, A, 1, n, b, 0, 1, pnl);
+  }
   __syncthreads();
   if (b * PLD <= 8 * TALL_REGION) qr_panel(A, b, n, n, tau, Tg1, pnl, job, nwg, iflag);
   else qr_tall(A, b, n, n, tau, Tg1, pnl, job, nwg, iflag);
@@ -3208,14 +3238,45 @@ __device__ __noinline__ bool jacobi_precond(double* X, int n_in, int b_in, doubl
   if (n * PLD <= 8 * TALL_REGION) qr_panel(X, n, n, n, tau, Tg2, pnl, job, nwg, iflag);
   else qr_tall(X, n, n, n, tau, Tg2, pnl, job, nwg, iflag);
   __syncthreads();
-  // J <- Q2^T: Q2 formed and written transposed (rows of Q2 as columns, bx = n)
-  q_form_tall(X, n, n, n, Tg2, Mq, J, n, nullptr, 0, nullptr, 0, pnl, job, nwg, iflag);
+  // J <- Q2^T P: Q2's columns are J's rows, entry c standing for row ord[c] of X
+  q_form_tall(X, n, n, n, Tg2, Mq, Mq, 1, nullptr, 0, nullptr, 0, pnl, job, nwg, iflag);
+  for (int c = wv; c < n; c += nwv)
+    for (int i = lane; i < n; i += 64) J[(int64_t)i * n + ord[c]] = Mq[(int64_t)c * n + i];
   for (int e = tid; e < n * n; e += bs) {  // X <- R2 (upper triangle of the second QR)
     const int i = e / n, j = e - i * n;
     if (j < i) X[e] = 0.0;
   }
   __syncthreads();
-  const bool cv = jacobi_coop(X, n, n, J, job, nwg, red, iflag, pnl, pnl_cap, cut, false, max_sweeps);
+  bool cv;
+  const int ld = n | 1;  // odd row strides in LDS: the rows of a round fall in different banks
+  if (n <= 96 && 2 * n * ld + 160 <= pnl_cap) {
+    lds_f64 *Xl = pnl, *Jl = pnl + n * ld;
+    for (int e = tid; e < n * n; e += bs) {
+      const int i = e / n, j = e - i * n;
+      Xl[i * ld + j] = X[e];
+      Jl[i * ld + j] = J[e];
+    }
+    __syncthreads();
+    lds_i32* fl = (lds_i32*)iflag;
+    if (n <= 32) cv = jacobi_rows_reg<8>(Xl, ld, n, n, Jl, ld, fl, red, cut, 0, max_sweeps);
+    else if (n <= 64) cv = jacobi_rows_reg<16>(Xl, ld, n, n, Jl, ld, fl, red, cut, 0, max_sweeps);
+    else cv = jacobi_rows_reg<32>(Xl, ld, n, n, Jl, ld, fl, red, cut, 0, max_sweeps);
+    __syncthreads();
+    for (int e = tid; e < n * n; e += bs) {
+      const int i = e / n, j = e - i * n;
+      X[e] = Xl[i * ld + j];
+      J[e] = Jl[i * ld + j];
+    }
+    __syncthreads();
+  } else if (coop) {
+    cv = jacobi_coop(X, n, n, J, job, nwg, red, iflag, pnl, pnl_cap, cut, false, max_sweeps);
+  } else {
+    lds_i32* fl = (lds_i32*)iflag;
+    if (n <= 128) cv = jacobi_rows_reg<32, 4, double>(X, n, n, n, J, n, fl, red, cut, 0, max_sweeps);
+    else if (n <= 256) cv = jacobi_rows_reg<32, 8, double>(X, n, n, n, J, n, fl, red, cut, 0, max_sweeps);
+    else if (n <= 384) cv = jacobi_rows_reg<32, 12, double>(X, n, n, n, J, n, fl, red, cut, 0, max_sweeps);
+    else cv = jacobi_rows_reg<64, 8, double>(X, n, n, n, J, n, fl, red, cut, 0, max_sweeps);
+  }
   // X (n x b) <- (J R2) Q1^T: Q1 applied to [(J R2)^T; 0], written transposed (bx = b)
   q_form_tall(A, b, n, n, Tg1, Mq, X, b, X, n, nullptr, n, pnl, job, nwg, iflag);
   return cv;
@@ -3490,11 +3551,13 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
       }
       return cv;
     };
-    // wide matrices of at least 192 rows on the global workspace with helper
-    // workgroups: the QR-preconditioned rounds (3D comb operate: 256 x 384
-    // moves 25.3 -> 12.7 ms; at 128 x 128 the two QRs cost what the saved
-    // sweeps do)
-    const bool precond = !REG && gws && job && nwg > 1 && !tall && n >= 192 && b <= 512 && pnl != nullptr;
+    // Wide or square matrices on the global workspace: the QR-preconditioned
+    // rounds, from 12 rows (below, the two QRs cost what the rounds do) where R2 and J fit LDS;
+    // with helper workgroups again from 192 (3D comb operate: 256 x 384 moves 25.3
+    // -> 12.7 ms; at 128 x 128 the two QRs cost what the saved sweeps do); alone,
+    // where the rounds run in global memory, whenever the lanes hold a row.
+    const bool precond = !REG && gws && pnl != nullptr && !tall && n >= 12 &&
+                         (n <= 96 || (job && nwg > 1 ? n >= 192 && b <= 512 : n <= 512));
     // A tall move that can drop nothing (cutoff <= 0: at most exactly zero singular
     // values would go; maxdim >= n) and whose R has no zero on its diagonal
     // (nonsingular, so none of its singular values is zero) keeps all n: Q R
@@ -3514,8 +3577,8 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
       __syncthreads();
     }
     bool conv = keep_all ? true
-                : precond ? jacobi_precond(X, n, b, Rb, Jb, tau, vbuf, vbuf + ((int64_t)n + PNB) * PNB, gY, pnl,
-                                           pnl_cap, job, nwg, red, iflag, cutoff, max_sweeps)
+                : precond ? jacobi_precond(X, n, b, Rb, Jb, tau, vbuf, vbuf + ((int64_t)n + PNB) * PNB, gY, sig, perm,
+                                           pnl, pnl_cap, job, nwg, red, iflag, cutoff, max_sweeps)
                           : jacobi(cutoff, true);
     row_norms<G>(X, n, b, sig);
     __syncthreads();

@@ -462,6 +462,27 @@ def test_truncate_preconditioned_wide_moves(q, po, eng, rng):
     assert err == pytest.approx(rerr, rel=1e-9)
 
 
+@pytest.mark.parametrize("maxdim", [16, 17, 24, 32, 33, 48, 49, 66])
+def test_truncate_preconditioned_batch_moves(q, po, eng, rng, maxdim):
+    # kernel-operator products of bonds up to 180 and 270 (batched: no helper
+    # workgroups), whose wide SVD moves have 2 maxdim rows: 32 and 64 (the lane
+    # groups of the rounds in LDS), 96 (the last that fits LDS), 98 and 132
+    # (rounds in global memory), and those next to them.  The sum of a function
+    # with itself is rank deficient: half of its rows are round-off.
+    s = q.continuous_siteinds(q.named_grid((13, 1)))
+    op = q.fredholm_operator(s)
+    f = q.random_itn(s, link_space=60, rng=rng, std=1.0 / math.sqrt(60))
+    h = q.random_itn(s, link_space=45, rng=rng, std=1.0 / math.sqrt(45))
+    fs = [f, q.builders.add_host(h, h)]
+    gs = q.operate_batch([op] * 2, fs, maxdim=maxdim)
+    gs = gs[0] if isinstance(gs, tuple) else gs
+    for fi, g in zip(fs, gs):
+        t = fi.topo
+        ref, _ = po.truncate(t.parent, t.sdim, po.contract(t.parent, t.sdim, op.cores, fi.cores), 0.0, maxdim)
+        assert list(g.bonds()) == [c.shape[0] for c in ref]
+        assert _compare_networks(q, po, g, ref, fi, rng) < 1e-11
+
+
 # ------------------------------------------------------------------ comb tree (config-3 shape, reduced)
 def test_comb_operate_and_integrate(q, po, eng, rng):
     from itensornumericalanalysis_jl_amd import workloads
