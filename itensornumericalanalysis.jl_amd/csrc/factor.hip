@@ -66,10 +66,10 @@ extern "C" int qtt_debug_jacobi(unsigned long long* out) {
 #define QTT_JT(i)                                                   \
   do {                                                              \
     const unsigned long long c_ = clock64();                        \
-    if (threadIdx.x == 0) qtt_jac_t[i] += c_ - jt_last_;            \
+    if (threadIdx.x == 0 && blockIdx.x == 0) qtt_jac_t[i] += c_ - jt_last_; \
     jt_last_ = c_;                                                  \
   } while (0)
-#define QTT_JC(i) do { if (threadIdx.x == 0) qtt_jac_t[i] += 1; } while (0)
+#define QTT_JC(i) do { if (threadIdx.x == 0 && blockIdx.x == 0) qtt_jac_t[i] += 1; } while (0)
 // cycles of thread 0 per segment of a blocked-QR panel
 __device__ unsigned long long qtt_pnl_t[16];
 extern "C" int qtt_debug_panel(unsigned long long* out) {
@@ -82,7 +82,7 @@ extern "C" int qtt_debug_panel(unsigned long long* out) {
 #define QTT_PT(i)                                                   \
   do {                                                              \
     const unsigned long long c_ = clock64();                        \
-    if (threadIdx.x == 0) qtt_pnl_t[i] += c_ - pt_last_;            \
+    if (threadIdx.x == 0 && blockIdx.x == 0) qtt_pnl_t[i] += c_ - pt_last_; \
     pt_last_ = c_;                                                  \
   } while (0)
 #else
@@ -1407,6 +1407,10 @@ constexpr int PLD = PNB + 1;  // row stride of a panel staged in LDS: odd, so no
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) f64x2 lds_f64x2;
+// Global memory by its address space: through a plain pointer argument the loads
+// of a function that is not inlined are flat ones, which count as LDS accesses
+// too, so every wait for LDS also waits for the loads in flight.
+typedef __attribute__((address_space(1))) double glb_f64;
 
 // ---------------------------------------------------------------------------
 // Blocked Householder QR for matrices too tall for an LDS panel.
@@ -1718,10 +1722,235 @@ __device__ __forceinline__ void wy_p3_unit2(double* M, int ldm, int mr, int col0
 constexpr int64_t WY_COOP_MIN = int64_t(1) << 15;  // entries of a row-chunk (two-job) shared update
 constexpr int64_t WY_COLS_MIN = int64_t(1) << 13;  // entries of a column-tile (one-job) shared update
 
+// A panel's reflector entry (row r, column j) without a branch: the address is
+// clamped into V (mr >= 1 rows, nb >= 1 columns) and the implied entries (unit
+// diagonal, zeros above, past row mr or column nb) are selected afterwards, so
+// the loads of a pipelined loop need no wait at a join.
+__device__ __forceinline__ double vsel(const double* V, int ldv, int r, int j, int mr, int nb) {
+  const double x = V[(int64_t)min(max(r, 0), mr - 1) * ldv + min(j, nb - 1)];
+  return (j < nb && r < mr) ? (r > j ? x : (r == j ? 1.0 : 0.0)) : 0.0;
+}
+
+// A 16 x 16 block of reflectors as MFMA operand A (lane: row li, column
+// 4 q + lk): loaded with the columns across the lanes (two 128-byte lines per 16
+// lanes at most, where loading it in operand order touches 16) and turned round
+// in 272 doubles of LDS of this wavefront's own.
+__device__ __forceinline__ void block_to_a(lds_f64* S, const double (&v)[4], double (&a)[4]) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) S[(4 * q + lk) * PLD + li] = v[q];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) a[q] = S[li * PLD + 4 * q + lk];
+}
+
+// W partials of one row chunk [rs, re) and two 16-column tiles from col0 and
+// col0 + 16 (columns past c1: whatever column c1 - 1 gives): w1 = V1^T M, w2 =
+// V2^T M, and g = V2^T V1 (TWO).  The reflectors are read once for both tiles,
+// the next 16 rows while this 16's MFMAs run.
+template <bool TWO>
+__device__ __forceinline__ void wyu_p1(const double* M, int ldm, int mr, int col0, int c1, const double* V1, int nb1,
+                                       const double* V2, int nb2, int ldv, int rs, int re, f64x4 (&w1)[2],
+                                       f64x4 (&w2)[2], f64x4& g) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int ca = min(col0 + li, c1 - 1), cb = min(col0 + 16 + li, c1 - 1);
+  double v1[4], v2[4], ba[4], bb[4];
+  auto load = [&](int r, double (&x1)[4], double (&x2)[4], double (&ya)[4], double (&yb)[4]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int rr = r + 4 * q + lk, rc = min(rr, mr - 1);
+      const bool in = rr < re;
+      const double t1 = vsel(V1, ldv, rr, li, mr, nb1);
+      x1[q] = in ? t1 : 0.0;
+      if constexpr (TWO) {
+        const double t2 = vsel(V2, ldv, rr - PNB, li, mr - PNB, nb2);
+        x2[q] = in ? t2 : 0.0;
+      }
+      const double ma = M[(int64_t)rc * ldm + ca], mb = M[(int64_t)rc * ldm + cb];
+      ya[q] = in ? ma : 0.0;
+      yb[q] = in ? mb : 0.0;
+    }
+  };
+  const f64x4 zero = {0.0, 0.0, 0.0, 0.0};
+  w1[0] = w1[1] = w2[0] = w2[1] = g = zero;
+  load(rs, v1, v2, ba, bb);
+  for (int r = rs; r < re; r += 16) {
+    double n1[4], n2[4], na[4], nb[4];
+    load(r + 16, n1, n2, na, nb);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      w1[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(v1[q], ba[q], w1[0], 0, 0, 0);
+      w1[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(v1[q], bb[q], w1[1], 0, 0, 0);
+      if constexpr (TWO) {
+        w2[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(v2[q], ba[q], w2[0], 0, 0, 0);
+        w2[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(v2[q], bb[q], w2[1], 0, 0, 0);
+        g = __builtin_amdgcn_mfma_f64_16x16x4f64(v2[q], v1[q], g, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      v1[q] = n1[q];
+      if constexpr (TWO) v2[q] = n2[q];
+      ba[q] = na[q];
+      bb[q] = nb[q];
+    }
+  }
+}
+
+// One or two panels' update in one pass over M, on this workgroup alone:
+//   M[0:mr, c0:c1] <- (I - V1 op(T1) V1^T) M                               (one)
+//   M <- (I - V2 T2^T V2^T)(I - V1 T1^T V1^T) M          (two, a QR's: trans)
+//   M <- (I - V1 T1 V1^T)(I - V2 T2 V2^T) M              (two, forming Q: rev)
+// M global (ldm); V1: the first panel's reflectors (rows from 0), V2: the
+// second's (rows from 16, so zero above), both with leading dimension ldv.  With
+// W1 = V1^T M, W2 = V2^T M and G = V2^T V1 from one pass over the rows: U of the
+// panel applied first, the other's W corrected by G, its U; then M -= V1 U1 + V2
+// U2 in a second pass, so M is read twice and written once per 32 columns of V.
+// All products are FP64 MFMA tiles (v_mfma_f64_16x16x4f64: lane l holds
+// A[l % 16][l / 16], B[l / 16][l % 16] and D[l / 16 + 4 e][l % 16] in element e;
+// D is B's layout of four steps, so the 16 x 16 products chain in registers, a
+// tile per wavefront without barriers).  M is a matrix of some 100 KB to a few MB
+// in this XCD's L2, and a load costs its access per line that 16 lanes touch: in
+// the second pass a wavefront keeps a 16-row block of V (turned round in LDS)
+// for four or eight column tiles; with V read in operand order per tile (64
+// accesses a load) a 570 x 285 QR took 1.65 ms, so 1.25 ms.  Matrices
+// of up to QC_ROWS rows that one workgroup factors go through qr_cols / q_cols.  L: 14336 doubles of LDS.
+template <bool TWO>
+__device__ __noinline__ void wy_update(double* M, int ldm_in, int mr_in, int c0_in, int c1_in, const double* V1,
+                                       const double* V2, int ldv_in, int nb1_in, int nb2_in, const lds_f64* T1,
+                                       const lds_f64* T2, lds_f64* L, bool trans, bool rev) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
+  const int li = lane & 15, lk = lane >> 4;
+  const int ldm = uni(ldm_in), mr = uni(mr_in), c0 = uni(c0_in), c1 = uni(c1_in), ldv = uni(ldv_in),
+            nb1 = uni(nb1_in), nb2 = uni(nb2_in);
+  lds_f64* P1 = L;              // partials [tile * nch + chunk][e * 64 + lane], 16 of them
+  lds_f64* P2 = L + 16 * 256;
+  lds_f64* PG = L + 32 * 256;   // partials of G, 8 of them
+  lds_f64* U1 = L + 40 * 256;   // -U1 [tile][j][c], 8 tiles
+  lds_f64* U2 = L + 48 * 256;
+  lds_f64* S = L + wv * (2 * 16 * PLD);  // the second pass: over P1 and P2
+  // equal groups of at most 8 tiles
+  const int ntile = (c1 - c0 + 15) >> 4, ngrp = (ntile + 7) >> 3, per = (ntile + ngrp - 1) / ngrp;
+  int ng = 0;  // chunks of G
+  for (int tg = 0; tg < ntile; tg += per) {
+    const int cg = c0 + 16 * tg, nct = min(per, ntile - tg), npr = (nct + 1) >> 1;
+    const int nch = max(1, min(8 / npr, (mr + 15) >> 4));
+    const int chunk = (((mr + nch - 1) / nch) + 15) & ~15;
+    for (int u = wv; u < npr * nch; u += nwv) {
+      const int p = u / nch, h = u - p * nch;
+      f64x4 w1[2], w2[2], g;
+      wyu_p1<TWO>(M, ldm, mr, cg + p * 32, c1, V1, nb1, V2, nb2, ldv, h * chunk, min(mr, (h + 1) * chunk), w1, w2, g);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        if (2 * p + t < nct) {
+          const int o = ((2 * p + t) * nch + h) * 256 + lane;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            P1[o + e * 64] = w1[t][e];
+            if constexpr (TWO) P2[o + e * 64] = w2[t][e];
+          }
+        }
+      }
+      if (TWO && tg == 0 && p == 0) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) PG[h * 256 + e * 64 + lane] = g[e];
+      }
+    }
+    if (tg == 0) ng = nch;
+    __syncthreads();
+    for (int t = wv; t < nct; t += nwv) {  // a tile per wavefront, its sums and products in registers
+      f64x4 w1 = {0.0, 0.0, 0.0, 0.0}, w2 = {0.0, 0.0, 0.0, 0.0};
+      for (int h = 0; h < nch; ++h) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          w1[e] += P1[(t * nch + h) * 256 + e * 64 + lane];
+          if constexpr (TWO) w2[e] += P2[(t * nch + h) * 256 + e * 64 + lane];
+        }
+      }
+      // the panel applied first (V1, or V2 if rev): U_f = op(T_f) W_f; then
+      // W_s <- W_s - (V_s^T V_f) U_f and U_s = op(T_s) W_s for the second, with
+      // V_s^T V_f = G (or G^T if rev); op(T) = T^T if trans.  U kept negated.
+      const lds_f64* Tf = TWO && rev ? T2 : T1;
+      f64x4 wf = TWO && rev ? w2 : w1, uf = {0.0, 0.0, 0.0, 0.0}, us = uf;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int j = 4 * q + lk;
+        uf = __builtin_amdgcn_mfma_f64_16x16x4f64(trans ? Tf[j * PNB + li] : Tf[li * PNB + j], wf[q], uf, 0, 0, 0);
+      }
+      uf = -uf;
+      if constexpr (TWO) {
+        const lds_f64* Ts = rev ? T1 : T2;
+        f64x4 ws = rev ? w1 : w2;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int j = 4 * q + lk, gi = rev ? j : li, gj = rev ? li : j;  // G[gi][gj], in D's layout in PG
+          double gs = 0.0;
+          for (int h = 0; h < ng; ++h) gs += PG[h * 256 + (gi >> 2) * 64 + (gi & 3) * 16 + gj];
+          ws = __builtin_amdgcn_mfma_f64_16x16x4f64(gs, uf[q], ws, 0, 0, 0);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int j = 4 * q + lk;
+          us = __builtin_amdgcn_mfma_f64_16x16x4f64(trans ? Ts[j * PNB + li] : Ts[li * PNB + j], ws[q], us, 0, 0, 0);
+        }
+        us = -us;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        U1[t * 256 + e * 64 + lane] = TWO && rev ? us[e] : uf[e];
+        if constexpr (TWO) U2[t * 256 + e * 64 + lane] = rev ? uf[e] : us[e];
+      }
+    }
+    __syncthreads();
+    // M -= V1 U1 + V2 U2: a wavefront takes a 16-row block and half of the tiles
+    // (all, up to four), the next block's reflectors in flight
+    const int nrb = (mr + 15) >> 4, nh = nct > 4 ? 2 : 1, hw = (nct + nh - 1) / nh;
+    double v1[4], v2[4];
+    auto loadv = [&](int x) {
+      const int rb = (x / nh) * 16;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        v1[q] = vsel(V1, ldv, rb + 4 * q + lk, li, mr, nb1);
+        if constexpr (TWO) v2[q] = vsel(V2, ldv, rb + 4 * q + lk - PNB, li, mr - PNB, nb2);
+      }
+    };
+    if (wv < nrb * nh) loadv(wv);
+    for (int x = wv; x < nrb * nh; x += nwv) {
+      const int rb = (x / nh) * 16, t0 = (x - (x / nh) * nh) * hw, t1 = min(nct, t0 + hw);
+      double a1[4], a2[4], cn[4];
+      block_to_a(S, v1, a1);
+      if constexpr (TWO) block_to_a(S + 16 * PLD, v2, a2);
+      loadv(x + nwv);  // past the last block: rows clamped, not used
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        cn[q] = M[(int64_t)min(rb + lk + 4 * q, mr - 1) * ldm + min(cg + t0 * 16 + li, c1 - 1)];
+      for (int t = t0; t < t1; ++t) {
+        const int col = cg + t * 16 + li;
+        f64x4 cm = {cn[0], cn[1], cn[2], cn[3]};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) cn[q] = M[(int64_t)min(rb + lk + 4 * q, mr - 1) * ldm + min(col + 16, c1 - 1)];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          cm = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[q], U1[t * 256 + q * 64 + lane], cm, 0, 0, 0);
+        if constexpr (TWO) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            cm = __builtin_amdgcn_mfma_f64_16x16x4f64(a2[q], U2[t * 256 + q * 64 + lane], cm, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int rr = rb + lk + 4 * e;
+          if (col < c1 && rr < mr) M[(int64_t)rr * ldm + col] = cm[e];
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
 __device__ __noinline__ void tall_wy(double* M, int ldm_in, int mr_in, int c0_in, int c1_in, const double* V,
                                      int ldv_in, int nb_in, const lds_f64* Tl, bool trans, lds_f64* L,
                                      CoopJob* job, int nwg_in, int* iflag) {
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nwv = blockDim.x >> 6;
+  const int tid = threadIdx.x, nwv = blockDim.x >> 6;
   const int ldm = uni(ldm_in), mr = uni(mr_in), c0 = uni(c0_in), c1 = uni(c1_in), ldv = uni(ldv_in),
             nb = uni(nb_in), nwg = uni(nwg_in);
   // helper workgroups only for a large trailing matrix: below WY_COOP_MIN
@@ -1751,61 +1980,52 @@ __device__ __noinline__ void tall_wy(double* M, int ldm_in, int mr_in, int c0_in
     if (threadIdx.x == 0) QTT_WY_COUNT_COLS;
     return;
   }
-  lds_f64* Pw = L;                  // partial W tiles: [unit][e * 64 + lane]
+  if (!coop) {
+    QTT_PT_INIT;
+    if (threadIdx.x == 0) QTT_WY_COUNT(coop);
+    wy_update<false>(M, ldm, mr, c0, c1, V, V, ldv, nb, 0, Tl, Tl, L, trans, false);
+    QTT_PT(10);
+    return;
+  }
   lds_f64* Wt = L + 32 * 256;       // W tiles [tile][j][c]
   lds_f64* Ut = Wt + 8 * 256;       // U tiles [tile][j][c]
   QTT_PT_INIT;
   if (threadIdx.x == 0) QTT_WY_COUNT(coop);
   for (int cg = c0; cg < c1; cg += 128) {
     const int nct = (min(128, c1 - cg) + 15) >> 4;  // 16-column tiles in this group
-    // row chunks per tile: enough units for every wavefront (of all workgroups with helpers)
-    const int nch = coop ? max(1, min(min((nwg * nwv + nct - 1) / nct, (mr + 63) / 64), COOP_PG_UNITS / nct))
-                         : max(1, min(32 / nct, (mr + 63) / 64));
-    const int nunit = nct * nch, chunk = (((mr + nch - 1) / nch) + 3) & ~3;
+    // row chunks per tile: enough units for every wavefront of all workgroups
+    const int nch = max(1, min(min((nwg * nwv + nct - 1) / nct, (mr + 63) / 64), COOP_PG_UNITS / nct));
+    const int chunk = (((mr + nch - 1) / nch) + 3) & ~3;
     // W = V^T M
-    if (coop) {
-      if (tid == 0) {
-        job->type = 6;
-        job->wy_M = M;
-        job->wy_ldm = ldm;
-        job->wy_mr = mr;
-        job->wy_cg = cg;
-        job->wy_c1 = c1;
-        job->wy_V = V;
-        job->wy_ldv = ldv;
-        job->nb = nb;
-        job->wy_nct = nct;
-        job->wy_nch = nch;
-        job->wy_chunk = chunk;
-      }
-      {
-        const int s = coop_post(job, iflag, nwg);
-        coop_wy_rows(job, 0, nwg);
-        coop_wait(job, s, nwg, iflag);
-      }
-    } else {
-      for (int u = wv; u < nunit; u += nwv) {
-        const int t = u / nch, h = u - t * nch;
-        const int rs = h * chunk, re = min(mr, rs + chunk);
-        const f64x4 acc = wy_p1_unit(M, ldm, mr, cg + t * 16, c1, V, ldv, nb, rs, re);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) Pw[u * 256 + e * 64 + lane] = acc[e];
-      }
-      __syncthreads();
+    if (tid == 0) {
+      job->type = 6;
+      job->wy_M = M;
+      job->wy_ldm = ldm;
+      job->wy_mr = mr;
+      job->wy_cg = cg;
+      job->wy_c1 = c1;
+      job->wy_V = V;
+      job->wy_ldv = ldv;
+      job->nb = nb;
+      job->wy_nct = nct;
+      job->wy_nch = nch;
+      job->wy_chunk = chunk;
+    }
+    {
+      const int s = coop_post(job, iflag, nwg);
+      coop_wy_rows(job, 0, nwg);
+      coop_wait(job, s, nwg, iflag);
     }
     // reduce the row chunks: W[t][j][c] with j = lane/16 + 4e, c = lane%16
     for (int x = tid; x < nct * 256; x += blockDim.x) {
       const int t = x >> 8, y = x & 255;
       const int e = y >> 6, ln = y & 63;
       double sum = 0.0;
-      if (coop)
-        for (int h = 0; h < nch; ++h) sum += job->Pg[(int64_t)(t * nch + h) * 256 + y];
-      else
-        for (int h = 0; h < nch; ++h) sum += Pw[(t * nch + h) * 256 + y];
+      for (int h = 0; h < nch; ++h) sum += job->Pg[(int64_t)(t * nch + h) * 256 + y];
       Wt[t * 256 + ((ln >> 4) + 4 * e) * 16 + (ln & 15)] = sum;
     }
     __syncthreads();
-    QTT_PT(coop ? 2 : 8);
+    QTT_PT(2);
     // U = op(T) W, stored negated for the update
     for (int x = tid; x < nct * 256; x += blockDim.x) {
       const int t = x >> 8, i = (x >> 4) & 15, c = x & 15;
@@ -1813,191 +2033,18 @@ __device__ __noinline__ void tall_wy(double* M, int ldm_in, int mr_in, int c0_in
 #pragma unroll
       for (int j = 0; j < PNB; ++j) sum = __builtin_fma(trans ? Tl[j * PNB + i] : Tl[i * PNB + j], Wt[t * 256 + j * 16 + c], sum);
       Ut[t * 256 + i * 16 + c] = -sum;
-      if (coop) job->Ug[t * 256 + i * 16 + c] = -sum;
+      job->Ug[t * 256 + i * 16 + c] = -sum;
     }
     __syncthreads();
-    QTT_PT(coop ? 3 : 9);
+    QTT_PT(3);
     // M -= V U, one (tile, 16-row block) at a time
-    const int nrb = (mr + 15) >> 4;
-    if (coop) {
-      if (tid == 0) job->type = 7;  // the other wy_* fields stay from the first phase
-      {
-        const int s = coop_post(job, iflag, nwg);
-        coop_wy_rows(job, 0, nwg);
-        coop_wait(job, s, nwg, iflag);
-      }
-    } else {
-      for (int x = wv; x < nct * nrb; x += nwv) {
-        const int t = x / nrb, rb = (x - t * nrb) * 16;
-        wy_p3_unit(M, ldm, mr, cg + t * 16, c1, V, ldv, nb, rb, (const lds_f64*)(Ut + t * 256));
-      }
-      __syncthreads();
+    if (tid == 0) job->type = 7;  // the other wy_* fields stay from the first phase
+    {
+      const int s = coop_post(job, iflag, nwg);
+      coop_wy_rows(job, 0, nwg);
+      coop_wait(job, s, nwg, iflag);
     }
-    QTT_PT(coop ? 5 : 10);
-  }
-}
-
-// Two panels' trailing update in one pass over M, on this workgroup alone:
-// M <- (I - V2 T2^T V2^T)(I - V1 T1^T V1^T) M for M[0:mr, c0:c1] (global,
-// ldm).  V1: the first panel's reflectors (rows from 0), V2: the second's
-// (rows from 16, so zero above), both with leading dimension ldv.  With
-// W1 = V1^T M and W2 = V2^T M read in the same pass, U1 = T1^T W1,
-// U2 = T2^T (W2 - G U1) with G = V2^T V1, and M -= V1 U1 + V2 U2 in a second
-// pass: M is read twice and written once per 32 columns instead of per 16.
-// L: LDS [0, 16384) for the partial and final tiles; T1, G: 256 doubles each.
-__device__ __forceinline__ void wy2_p1_unit(const double* M, int ldm, int mr, int col0, int c1, const double* V1,
-                                            int nb1, const double* V2, int nb2, int ldv, int rs, int re, f64x4& w1,
-                                            f64x4& w2) {
-  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-  const int col = col0 + li;
-  const bool con = col < c1;
-  f64x4 a1 = {0.0, 0.0, 0.0, 0.0}, a2 = {0.0, 0.0, 0.0, 0.0};
-  for (int r = rs; r < re; r += 16) {  // 16 rows (four steps) in flight per wait
-    double v1[4], v2[4], b[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int rr = r + 4 * q + lk;
-      const bool rin = rr < re;
-      v1[q] = rin ? vref(V1, ldv, rr, li, mr, nb1) : 0.0;
-      v2[q] = rin ? vref(V2, ldv, rr - PNB, li, mr - PNB, nb2) : 0.0;
-      b[q] = (rin && con) ? M[(int64_t)rr * ldm + col] : 0.0;
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(v1[q], b[q], a1, 0, 0, 0);
-      a2 = __builtin_amdgcn_mfma_f64_16x16x4f64(v2[q], b[q], a2, 0, 0, 0);
-    }
-  }
-  w1 = a1;
-  w2 = a2;
-}
-
-__device__ __noinline__ void tall_wy2(double* M, int ldm_in, int mr_in, int c0_in, int c1_in, const double* V1,
-                                      const double* V2, int ldv_in, int nb1_in, int nb2_in, const lds_f64* T1,
-                                      const lds_f64* T2, lds_f64* G, lds_f64* L, bool trans, bool rev) {
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nwv = blockDim.x >> 6;
-  const int li = lane & 15, lk = lane >> 4;
-  const int ldm = uni(ldm_in), mr = uni(mr_in), c0 = uni(c0_in), c1 = uni(c1_in), ldv = uni(ldv_in),
-            nb1 = uni(nb1_in), nb2 = uni(nb2_in);
-  lds_f64* P1 = L;                // [unit][e * 64 + lane], 16 units
-  lds_f64* P2 = L + 16 * 256;
-  lds_f64* W1 = L + 32 * 256;     // [tile][j][c], 8 tiles
-  lds_f64* W2 = L + 40 * 256;
-  lds_f64* U1 = L + 48 * 256;     // -U1 [tile][j][c]
-  lds_f64* U2 = L + 56 * 256;     // -U2
-  // G = V2^T V1 over the rows from 16: partials per wavefront in P1, summed
-  {
-    f64x4 g = {0.0, 0.0, 0.0, 0.0};
-    for (int r = PNB + 4 * wv; r < mr; r += 4 * nwv) {
-      const int rr = r + lk;
-      const double a = rr < mr ? vref(V2, ldv, rr - PNB, li, mr - PNB, nb2) : 0.0;
-      const double bb = rr < mr ? vref(V1, ldv, rr, li, mr, nb1) : 0.0;
-      g = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bb, g, 0, 0, 0);
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) P1[wv * 256 + e * 64 + lane] = g[e];
-    __syncthreads();
-    if (tid < 256) {  // element e of lane ln is G[ln / 16 + 4 e][ln % 16]
-      const int e = tid >> 6, ln = tid & 63;
-      double sum = 0.0;
-      for (int w = 0; w < nwv; ++w) sum += P1[w * 256 + tid];
-      G[((ln >> 4) + 4 * e) * 16 + (ln & 15)] = sum;
-    }
-    __syncthreads();
-  }
-  for (int cg = c0; cg < c1; cg += 128) {
-    const int nct = (min(128, c1 - cg) + 15) >> 4;
-    const int nch = max(1, min(16 / nct, (mr + 63) / 64));
-    const int nunit = nct * nch, chunk = (((mr + nch - 1) / nch) + 15) & ~15;
-    for (int u = wv; u < nunit; u += nwv) {
-      const int t = u / nch, h = u - t * nch;
-      const int rs = h * chunk, re = min(mr, rs + chunk);
-      f64x4 w1, w2;
-      wy2_p1_unit(M, ldm, mr, cg + t * 16, c1, V1, nb1, V2, nb2, ldv, rs, re, w1, w2);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        P1[u * 256 + e * 64 + lane] = w1[e];
-        P2[u * 256 + e * 64 + lane] = w2[e];
-      }
-    }
-    __syncthreads();
-    for (int x = tid; x < nct * 256; x += blockDim.x) {
-      const int t = x >> 8, y = x & 255;
-      const int e = y >> 6, ln = y & 63;
-      double s1 = 0.0, s2 = 0.0;
-      for (int h = 0; h < nch; ++h) {
-        s1 += P1[(t * nch + h) * 256 + y];
-        s2 += P2[(t * nch + h) * 256 + y];
-      }
-      const int o = t * 256 + ((ln >> 4) + 4 * e) * 16 + (ln & 15);
-      W1[o] = s1;
-      W2[o] = s2;
-    }
-    __syncthreads();
-    // the panel applied first (V1, or V2 if rev): U_f = op(T_f) W_f; then
-    // W_s <- W_s - (V_s^T V_f) U_f and U_s = op(T_s) W_s for the second, with
-    // V_s^T V_f = G (or G^T if rev); op(T) = T^T if trans.  U stored negated.
-    const lds_f64* Tf = rev ? T2 : T1;
-    const lds_f64* Ts = rev ? T1 : T2;
-    lds_f64* Wf = rev ? W2 : W1;
-    lds_f64* Ws = rev ? W1 : W2;
-    lds_f64* Uf = rev ? U2 : U1;
-    lds_f64* Us = rev ? U1 : U2;
-    for (int x = tid; x < nct * 256; x += blockDim.x) {
-      const int t = x >> 8, i = (x >> 4) & 15, c = x & 15;
-      double sum = 0.0;
-#pragma unroll
-      for (int j = 0; j < PNB; ++j)
-        sum = __builtin_fma(trans ? Tf[j * PNB + i] : Tf[i * PNB + j], Wf[t * 256 + j * 16 + c], sum);
-      Uf[t * 256 + i * 16 + c] = -sum;
-    }
-    __syncthreads();
-    for (int x = tid; x < nct * 256; x += blockDim.x) {  // Uf is stored negated
-      const int t = x >> 8, i = (x >> 4) & 15, c = x & 15;
-      double sum = Ws[t * 256 + i * 16 + c];
-#pragma unroll
-      for (int j = 0; j < PNB; ++j)
-        sum = __builtin_fma(rev ? G[j * 16 + i] : G[i * 16 + j], Uf[t * 256 + j * 16 + c], sum);
-      P2[t * 256 + i * 16 + c] = sum;
-    }
-    __syncthreads();
-    for (int x = tid; x < nct * 256; x += blockDim.x) {
-      const int t = x >> 8, i = (x >> 4) & 15, c = x & 15;
-      double sum = 0.0;
-#pragma unroll
-      for (int j = 0; j < PNB; ++j)
-        sum = __builtin_fma(trans ? Ts[j * PNB + i] : Ts[i * PNB + j], P2[t * 256 + j * 16 + c], sum);
-      Us[t * 256 + i * 16 + c] = -sum;
-    }
-    __syncthreads();
-    // M -= V1 U1 + V2 U2, one (tile, 16-row block) at a time
-    const int nrb = (mr + 15) >> 4;
-    for (int x = wv; x < nct * nrb; x += nwv) {
-      const int t = x / nrb, rb = (x - t * nrb) * 16;
-      const int col = cg + t * 16 + li;
-      const bool con = col < c1;
-      double b1[4], b2[4], a1[4], a2[4];
-      f64x4 cm;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        b1[q] = U1[t * 256 + (4 * q + lk) * 16 + li];
-        b2[q] = U2[t * 256 + (4 * q + lk) * 16 + li];
-        a1[q] = vref(V1, ldv, rb + li, 4 * q + lk, mr, nb1);
-        a2[q] = vref(V2, ldv, rb + li - PNB, 4 * q + lk, mr - PNB, nb2);
-        const int rr = rb + lk + 4 * q;
-        cm[q] = (con && rr < mr) ? M[(int64_t)rr * ldm + col] : 0.0;
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) cm = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[q], b1[q], cm, 0, 0, 0);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) cm = __builtin_amdgcn_mfma_f64_16x16x4f64(a2[q], b2[q], cm, 0, 0, 0);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int rr = rb + lk + 4 * e;
-        if (con && rr < mr) M[(int64_t)rr * ldm + col] = cm[e];
-      }
-    }
-    __syncthreads();
+    QTT_PT(5);
   }
 }
 
@@ -2022,6 +2069,71 @@ __device__ __noinline__ void qr_tall(double* W, int rows_in, int cols_in, int ld
   }
 }
 
+// D <- Y, n doubles in global memory: eight loads of a thread in flight.
+__device__ __noinline__ void copy_doubles(double* D_in, const double* Y_in, int64_t n) {
+  glb_f64* D = (glb_f64*)D_in;
+  const glb_f64* Y = (const glb_f64*)Y_in;
+  const int64_t bs = blockDim.x;
+  for (int64_t e0 = threadIdx.x; e0 < n; e0 += 8 * bs) {
+    double t[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = Y[min(e0 + u * bs, n - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (e0 + u * bs < n) D[e0 + u * bs] = t[u];
+  }
+}
+
+// Rows up to which a matrix is factored (or its Q formed) in column groups, and
+// the entries above which helper workgroups, where there are any, share it
+// instead: a 256 x 128 QR takes 281 us shared and 175 us on one workgroup; a
+// 768 x 384 one 989 us shared, which is about what one workgroup would need.
+constexpr int QC_ROWS = 1024;
+constexpr int64_t QC_SHARE = 40960;
+
+// Q or U of more than QC_ROWS rows, or shared with the helper workgroups, formed
+// in Mq (rows x ncol, global): the identity's columns (or J's), then the panels
+// applied in reverse, on this workgroup alone in pairs (one pass over Mq per two).
+__device__ __noinline__ void q_blocks(const double* W, int rows, int k, int ld, const double* Tg, double* Mq,
+                                      const double* Jb, int n, const int* perm, int ncol, lds_f64* L, CoopJob* job,
+                                      int nwg, int* iflag) {
+  const int tid = threadIdx.x, bs = blockDim.x;
+  const bool pairs = !(job != nullptr && nwg > 1) || (int64_t)rows * ncol < WY_COLS_MIN;
+  lds_f64* Tl = L + 8 * TALL_REGION + 16 * 128;
+  {  // a row per wavefront, the columns over its lanes (no divisions per entry)
+    const int lane = tid & 63, wv = tid >> 6, nwv = bs >> 6;
+    for (int r = wv; r < rows; r += nwv)
+      for (int c = lane; c < ncol; c += 64)
+        Mq[(int64_t)r * ncol + c] =
+            Jb ? (r < n ? Jb[(int64_t)(perm ? perm[c] : c) * n + r] : 0.0) : (r == c ? 1.0 : 0.0);
+  }
+  __syncthreads();
+  lds_f64* T1 = L + 8 * TALL_REGION + 512;  // the earlier panel's T of a pair
+  for (int p0 = ((k - 1) / PNB) * PNB; p0 >= 0;) {
+    const int nb = k - p0 < PNB ? k - p0 : PNB;
+    for (int e = tid; e < PNB * PNB; e += bs) Tl[e] = Tg[(p0 / PNB) * PNB * PNB + e];
+    if (pairs && p0 >= PNB) {
+      // panels pa = p0 - 16 (V1) and p0 (V2, 16 rows further), p0's applied first
+      const int pa = p0 - PNB;
+      for (int e = tid; e < PNB * PNB; e += bs) T1[e] = Tg[(pa / PNB) * PNB * PNB + e];
+      __syncthreads();
+      wy_update<true>(Mq + (int64_t)pa * ncol, ncol, rows - pa, Jb ? 0 : pa, ncol, W + (int64_t)pa * ld + pa,
+                      W + (int64_t)p0 * ld + p0, ld, PNB, nb, T1, Tl, L, false, true);
+      p0 = pa - PNB;
+    } else {
+      __syncthreads();
+      // Q: only columns >= p0 differ from the identity yet; U: every column
+      tall_wy(Mq + (int64_t)p0 * ncol, ncol, rows - p0, Jb ? 0 : p0, ncol, W + (int64_t)p0 * ld + p0, ld, nb, Tl,
+              false, L, job, nwg, iflag);
+      p0 -= PNB;
+    }
+  }
+}
+
+template <int NR, int NT>
+__device__ void q_cols(const double* W, int rows_in, int k_in, int ld_in, const double* Tg, double* Mq,
+                       const double* Jb, int n_in, const int* perm, int m_in, lds_f64* L);
+
 // x <- Q (rows x k) of qr_tall's reflectors, or with Jb x <- U = Q [J_perm^T; 0]
 // (rows x m; perm null: the rows of J in order), formed row-major in Mq
 // (global) and then written into the core Xc (rows split as (aa, bb), bb < bx).
@@ -2034,43 +2146,17 @@ __device__ __noinline__ void q_form_tall(const double* W, int rows_in, int k_in,
   const int rows = uni(rows_in), k = uni(k_in), ld = uni(ld_in), bx = uni(bx_in), n = uni(n_in), m = uni(m_in),
             nwg = uni(nwg_in);
   const int ncol = Jb ? m : k;
-  lds_f64* Tl = L + 8 * TALL_REGION + 16 * 128;
-  {  // a row per wavefront, the columns over its lanes (no divisions per entry)
-    const int lane = tid & 63, wv = tid >> 6, nwv = bs >> 6;
-    for (int r = wv; r < rows; r += nwv)
-      for (int c = lane; c < ncol; c += 64)
-        Mq[(int64_t)r * ncol + c] =
-            Jb ? (r < n ? Jb[(int64_t)(perm ? perm[c] : c) * n + r] : 0.0) : (r == c ? 1.0 : 0.0);
-  }
-  __syncthreads();
-  // panels in pairs (tall_wy2, one pass over Mq per two panels) where every
-  // update would run on this workgroup alone anyway
-  const bool pairs = !(job != nullptr && nwg > 1) || (int64_t)rows * ncol < WY_COLS_MIN;
-  lds_f64* T1 = L + 8 * TALL_REGION + 512;  // the earlier panel's T of a pair
-  lds_f64* Gp = L + 8 * TALL_REGION + 768;  // V_later^T V_earlier
-  for (int p0 = ((k - 1) / PNB) * PNB; p0 >= 0;) {
-    const int nb = k - p0 < PNB ? k - p0 : PNB;
-    for (int e = tid; e < PNB * PNB; e += bs) Tl[e] = Tg[(p0 / PNB) * PNB * PNB + e];
-    if (pairs && p0 >= PNB) {
-      // panels pa = p0 - 16 (V1) and p0 (V2, 16 rows further), p0's applied first
-      const int pa = p0 - PNB;
-      for (int e = tid; e < PNB * PNB; e += bs) T1[e] = Tg[(pa / PNB) * PNB * PNB + e];
-      __syncthreads();
-      tall_wy2(Mq + (int64_t)pa * ncol, ncol, rows - pa, Jb ? 0 : pa, ncol, W + (int64_t)pa * ld + pa,
-               W + (int64_t)p0 * ld + p0, ld, PNB, nb, T1, Tl, Gp, L, false, true);
-      p0 = pa - PNB;
-    } else {
-      __syncthreads();
-      // Q: only columns >= p0 differ from the identity yet; U: every column
-      tall_wy(Mq + (int64_t)p0 * ncol, ncol, rows - p0, Jb ? 0 : p0, ncol, W + (int64_t)p0 * ld + p0, ld, nb, Tl,
-              false, L, job, nwg, iflag);
-      p0 -= PNB;
-    }
-  }
+  // on this workgroup alone where every update would run here anyway or the
+  // matrix is small (see QC_SHARE)
+  const bool alone = !(job != nullptr && nwg > 1) || (int64_t)rows * ncol <= QC_SHARE;
+  if (alone && rows <= 256) q_cols<8, 2>(W, rows, k, ld, Tg, Mq, Jb, n, perm, ncol, L);
+  else if (alone && rows <= 640) q_cols<20, 2>(W, rows, k, ld, Tg, Mq, Jb, n, perm, ncol, L);
+  else if (alone && rows <= QC_ROWS) q_cols<32, 1>(W, rows, k, ld, Tg, Mq, Jb, n, perm, ncol, L);
+  else q_blocks(W, rows, k, ld, Tg, Mq, Jb, n, perm, ncol, L, job, nwg, iflag);
   // Xc[aa] (ncol x bx) = Mq[aa]^T (Mq[aa]: bx x ncol): tiled transposes, with
   // the helper workgroups for a large result
   if (bx == 1) {
-    for (int e = tid; e < rows * ncol; e += bs) Xc[e] = Mq[e];
+    if (Xc != Mq) copy_doubles(Xc, Mq, (int64_t)rows * ncol);
   } else if (job != nullptr && nwg > 1 && (int64_t)rows * ncol >= (int64_t(1) << 15)) {
     if (tid == 0) {
       job->type = 10;
@@ -2089,22 +2175,28 @@ __device__ __noinline__ void q_form_tall(const double* W, int rows_in, int k_in,
 }
 
 // ---------------------------------------------------------------------------
-// Panel factorization in registers (panels of up to 512 RPT rows, 512
-// threads): thread t holds rows t + 512 k (k < RPT) of the panel's PNB
-// columns.  Step j applies reflector j to those rows and, in the same pass,
-// forms this thread's share of what step j+1 needs: s_c = the sum over the
-// rows r > j+1 of a[r][j+1] a[r][c], for every column c -- for c > j+1 the
-// dot products with column j+1, for c == j+1 its norm^2, and for c <= j its
-// dot products with the earlier reflectors (stored in place), which give
-// column j+1 of T.  The 16 sums are reduced within each wavefront by four
-// halving exchanges (every lane ends with the sum of one column over its
-// quad) and across the wavefronts through LDS: one barrier per column.
-// Row j+1, read by every thread in step j+1, travels through LDS with them.
+// Panel factorization in registers (panels of up to 32 NR rows, 512 threads).
+// Lane (lk, li) of wavefront w holds column li of rows 32 q + 4 w + lk (q < NR):
+// 16 lanes are a row, so global loads and stores are whole rows, a column is
+// broadcast over its rows by one DPP move (row_newbcast), and every lane keeps
+// the sums of its own column only.  Step J applies reflector J and, in the same
+// pass, forms what step J + 1 needs: S_c = the sum over the rows r > J + 1 of
+// a[r][J + 1] a[r][c] for every column c -- for c > J + 1 the dot products with
+// column J + 1, for c == J + 1 its norm^2, and for c <= J its dot products with
+// the earlier reflectors, which give column J + 1 of T.  A sum is two lane swaps
+// in the wavefront, and the wavefronts' partials are added through LDS: one
+// barrier per column.  Reflectors stay unscaled until the end (their dot
+// products are scaled instead).
+//   Bound by instruction issue: 4 NR + some 60 instructions a column on each of
+// two wavefronts per SIMD.  With a row per thread (16 columns in registers, 16
+// sums reduced by 15 exchanges, 16 coefficients read lane by lane, staged
+// through LDS) a panel of a 570 x 285 QR took 20 us, now 12.
 // ---------------------------------------------------------------------------
 
-// column whose sum lane l holds after wave_sum16: 8 b5 + 4 b4 + 2 b3 + b2
-__device__ __forceinline__ int sum16_col(int lane) {
-  return ((lane >> 5) & 1) * 8 + ((lane >> 4) & 1) * 4 + ((lane >> 3) & 1) * 2 + ((lane >> 2) & 1);
+// v of lane C of each 16 lanes, in all 16
+template <int C>
+__device__ __forceinline__ double bcast16(double v) {
+  return __builtin_amdgcn_mov_dpp(v, 0x150 + C, 0xF, 0xF, true);  // row_newbcast, one 64-bit move
 }
 
 // v_permlane32_swap on both halves of a and b, then the sum: lanes 0-31 get
@@ -2122,227 +2214,460 @@ __device__ __forceinline__ double swap16_add(double a, double b) {
   return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
 }
 
-// Sum p[0..15] over the wavefront; lane l returns the sum of column
-// sum16_col(l).  Each exchange pairs lanes that hold the same column set and
-// differ in one lane bit (5, 4, 3, 2): the lane keeps the half of its set
-// that the bit selects and adds the partner's copy of that half.  The last
-// two steps sum the quad.  Fixed order: the same sums on every run.
-__device__ __forceinline__ double wave_sum16(const double (&p)[PNB]) {
-  const int lane = threadIdx.x & 63;
-  const bool h3 = lane & 8, h2 = lane & 4;
-  double q8[8], q4[4], q2[2];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) q8[i] = swap32_add(p[i], p[i + 8]);   // bit 5: columns i / i + 8
-#pragma unroll
-  for (int i = 0; i < 4; ++i) q4[i] = swap16_add(q8[i], q8[i + 4]);  // bit 4: + 0 / + 4
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {  // row_mirror: lane 15 - m of the 16-lane row (bit 3 differs)
-    const double keep = h3 ? q4[i + 2] : q4[i], send = h3 ? q4[i] : q4[i + 2];
-    q2[i] = keep + dpp_d<0x140>(send);
-  }
-  // row_half_mirror: lane 7 - m of the 8-lane half (bit 2 differs, bit 3 kept)
-  double q = (h2 ? q2[1] : q2[0]) + dpp_d<0x141>(h2 ? q2[0] : q2[1]);
-  q += dpp_d<0xB1>(q);  // quad_perm [1,0,3,2]
-  q += dpp_d<0x4E>(q);  // quad_perm [2,3,0,1]
-  return q;
+// sum over l < J of T[li][l] y_l (y_l in lane l), by wavefront
+template <int L, int J>
+__device__ __forceinline__ double panel_ty(const double (&Trow)[PNB], double y) {
+  if constexpr (L < J) return __builtin_fma(Trow[L], bcast16<L>(y), panel_ty<L + 1, J>(Trow, y));
+  else return 0.0;
 }
 
-// The 16 column sums of p over the workgroup (8 wavefronts); lane l returns
-// the sum of column l & 15.  red: 8 x PNB doubles of LDS.  Every wavefront
-// adds the 8 partials in the same order, so all threads see the same sums.
-__device__ __forceinline__ double panel_sums16(const double (&p)[PNB], lds_f64* red) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const double q = wave_sum16(p);
-  if ((lane & 3) == 0) red[wv * PNB + sum16_col(lane)] = q;
-  __syncthreads();
-  double t = 0.0;
+// The sums S of column J1 (this lane's column against it, rows below J1) and
+// row J1's entry R of this lane's column, for the step that reflects column J1.
+template <int J1, int NP, int NR>
+__device__ __forceinline__ void panel_sums(const double (&x)[NR], int row0, lds_f64* red, double& S, double& R) {
+  const int lane = threadIdx.x & 63, li = lane & 15, wv = threadIdx.x >> 6, r0 = opaque(row0);
+  lds_f64 *part = red + (J1 & 1) * 8 * PNB, *rowb = red + 2 * 8 * PNB + (J1 & 1) * PNB;
+  const double a0 = bcast16<J1>(x[0]);
+  double p0 = (r0 > J1 ? a0 : 0.0) * x[0], p1 = 0.0;
 #pragma unroll
-  for (int w = 0; w < 8; ++w) t += red[w * PNB + (lane & 15)];
-  return t;
+  for (int q = 1; q < NP; ++q) {
+    if (q & 1) p1 = __builtin_fma(bcast16<J1>(x[q]), x[q], p1);
+    else p0 = __builtin_fma(bcast16<J1>(x[q]), x[q], p0);
+  }
+  double p = p0 + p1;
+  p = swap32_add(p, p);
+  p = swap16_add(p, p);
+  if (lane < PNB) part[wv * PNB + li] = p;
+  if (r0 == J1) rowb[li] = x[0];
+  __syncthreads();
+  double t[8];
+#pragma unroll
+  for (int w = 0; w < 8; ++w) t[w] = part[w * PNB + li];
+  R = rowb[li];
+  S = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+}
+
+template <int J, int NP, int NR>
+__device__ __forceinline__ void panel_step(double (&x)[NR], int row0, double S, double R, double& ms,
+                                           double (&Trow)[PNB], double* tau, int nb, lds_f64* red) {
+  const int tid = threadIdx.x, lane = tid & 63, li = opaque(lane & 15), wv = tid >> 6, r0 = opaque(row0);
+  // reflector J from alpha = a[J][J] and sg = the norm^2 below it (zero columns
+  // past nb give tau 0): with the norm n, beta = -sign(alpha) n, tau = (n +
+  // |alpha|) / n, v = a / (alpha - beta).  1 / n and 1 / (n + |alpha|) by Newton
+  // steps from the hardware's estimates (last-bit accurate; a third of the
+  // instructions of a square root and two divisions, which every wavefront runs).
+  const double alpha = bcast16<J>(R), sg = bcast16<J>(S);
+  const double n2 = __builtin_fma(alpha, alpha, sg), aa = fabs(alpha);
+  const double y0 = __builtin_amdgcn_rsq(n2), e0 = __builtin_fma(-n2 * y0, y0, 1.0);
+  const double rn = __builtin_fma(y0 * e0, __builtin_fma(0.375, e0, 0.5), y0);
+  double n = n2 * rn;
+  n = __builtin_fma(__builtin_fma(-n, n, n2), 0.5 * rn, n);
+  const double s = aa + n;
+  double y = __builtin_amdgcn_rcp(s);
+  y = __builtin_fma(__builtin_fma(-s, y, 1.0), y, y);
+  y = __builtin_fma(__builtin_fma(-s, y, 1.0), y, y);
+  const bool on = sg != 0.0;
+  const double beta = on ? -copysign(n, alpha) : alpha;
+  const double tj = on ? s * rn : 0.0;
+  const double scale = on ? copysign(y, alpha) : 0.0;
+  // z_c = v_J . a_c = a[J][c] + scale S[c]: for c < J the y_c of T (a_c is
+  // reflector c there), for c > J, times tau_J, what reflector J takes from
+  // column c
+  const double z = __builtin_fma(scale, S, R);
+  if (wv == 7) {  // T[:, J] = -tau_J T[:, 0:J] y, a row per lane
+    const double acc = panel_ty<0, J>(Trow, z);
+    Trow[J] = li == J ? tj : (li < J ? -tj * acc : 0.0);
+  }
+  if (tid == 0 && J < nb) tau[J] = tj;
+  const double zu = li > J ? -tj * z : 0.0, zs = zu * scale;
+  ms = li == J ? scale : ms;
+  {
+    const double a0 = bcast16<J>(x[0]);
+    x[0] = r0 > J ? __builtin_fma(zs, a0, x[0]) : (r0 == J ? (li == J ? beta : x[0] + zu) : x[0]);
+  }
+#pragma unroll
+  for (int q = 1; q < NP; ++q) x[q] = __builtin_fma(zs, bcast16<J>(x[q]), x[q]);
+  if constexpr (J + 1 < PNB) {
+    double S1, R1;
+    panel_sums<J + 1, NP>(x, row0, red, S1, R1);
+    panel_step<J + 1, NP>(x, row0, S1 * ms, R1 * ms, ms, Trow, tau, nb, red);
+  }
 }
 
 // Factor the panel P = W[p0:, p0:p0+nb] (global, ld; mr = rows - p0 rows,
-// nb <= mr): R on and above its diagonal, the reflectors below (unit diagonal
-// implied), tau[0..nb), and the panel's T (PNB x PNB, zero rows and columns
-// past nb) into Tl (LDS) and Tg.  L: LDS, the panel staged through its first
-// mr * PLD doubles (coalesced global reads and writes); red: 2 x 8 x PNB sums
-// and 2 x PNB row doubles of LDS, disjoint from the staging area and Tl.
-template <int RPT>
+// nb <= mr <= 32 NR): R on and above its diagonal, the reflectors below (unit
+// diagonal implied), tau[0..nb), and the panel's T (PNB x PNB, zero rows and
+// columns past nb) into Tl (LDS) and Tg.  red: 2 x 8 x PNB sums and 2 x PNB row
+// doubles of LDS, disjoint from Tl.
+template <int NR>
 __device__ __noinline__ void reg_panel(double* W, int rows_in, int ld_in, int p0_in, int nb_in, double* tau,
-                                       double* Tg, lds_f64* Tl, lds_f64* L, lds_f64* red) {
-  const int tid = threadIdx.x;
+                                       double* Tg, lds_f64* Tl, lds_f64* red) {
+  const int lane = threadIdx.x & 63, li = lane & 15, wv = threadIdx.x >> 6, r0 = 4 * wv + (lane >> 4);
   const int rows = uni(rows_in), ld = uni(ld_in), p0 = uni(p0_in), nb = uni(nb_in);
-  const int mr = rows - p0, ne = mr * PNB;
+  const int mr = rows - p0;
   double* P = W + (int64_t)p0 * ld + p0;
-  lds_f64* rowb = red + 2 * 8 * PNB;
-  // global -> LDS (8 loads in flight per thread) -> registers
-  for (int e0 = 0; e0 < ne; e0 += 8 * 512) {
-    double t[8];
+  double x[NR], Trow[PNB], ms = 1.0, S, R;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int e = e0 + u * 512 + tid, r = e >> 4, c = e & 15;
-      t[u] = (e < ne && c < nb) ? P[(int64_t)r * ld + c] : 0.0;
-    }
+  for (int q = 0; q < NR; ++q) x[q] = P[(int64_t)min(32 * q + r0, mr - 1) * ld + min(li, nb - 1)];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int e = e0 + u * 512 + tid;
-      if (e < ne) L[(e >> 4) * PLD + (e & 15)] = t[u];
-    }
-  }
-  __syncthreads();
-  double x[RPT][PNB];
+  for (int q = 0; q < NR; ++q) x[q] = (32 * q + r0 < mr && li < nb) ? x[q] : 0.0;
 #pragma unroll
-  for (int k = 0; k < RPT; ++k) {
-    const int r = tid + 512 * k;
-#pragma unroll
-    for (int c = 0; c < PNB; ++c) x[k][c] = r < mr ? L[r * PLD + c] : 0.0;
-  }
-  // column layout: lane l holds, for column l & 15, the sum S (over the
-  // rows below the current row j) and row j's entry R
-  double S, R, Trow[PNB];
-  const int cl = threadIdx.x & 15;
-  {
-    double p[PNB];
-#pragma unroll
-    for (int c = 0; c < PNB; ++c) p[c] = 0.0;
-#pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-      const double a = (tid + 512 * k > 0) ? x[k][0] : 0.0;
-#pragma unroll
-      for (int c = 0; c < PNB; ++c) p[c] = __builtin_fma(a, x[k][c], p[c]);
-    }
-    if (tid == 0) {
-#pragma unroll
-      for (int c = 0; c < PNB; ++c) rowb[c] = x[0][c];
-    }
-    S = panel_sums16(p, red);
-    R = rowb[cl];
-  }
-  const int ti = tid & 15;  // the row of T this thread keeps (written by threads 0..15)
-#pragma unroll
-  for (int j = 0; j < PNB; ++j) {
-    // reflector j from alpha = a[j][j] and S[j] = the norm^2 below it (zero
-    // columns past nb give tau 0)
-    const double alpha = readlane_d(R, j), sg = readlane_d(S, j);
-    double tj = 0.0, beta = alpha, scale = 0.0;
-    if (sg != 0.0) {
-      beta = -copysign(sqrt(alpha * alpha + sg), alpha);
-      tj = (beta - alpha) / beta;
-      scale = 1.0 / (alpha - beta);
-    }
-    // z_c = v_j . a_c = a[j][c] + scale * S[c]: for c < j the y_c of T (a_c
-    // holds reflector c there), for c > j, times tau_j, what reflector j
-    // takes from column c
-    double zl = __builtin_fma(scale, S, R);
-    zl = cl > j ? tj * zl : (cl < j ? zl : 0.0);
-    double z[PNB];
-#pragma unroll
-    for (int c = 0; c < PNB; ++c) z[c] = readlane_d(zl, c);
-    // T[:, j] = -tau_j T[:, 0:j] y
-    {
-      double acc = 0.0;
-#pragma unroll
-      for (int l = 0; l < PNB; ++l)
-        if (l < j) acc = __builtin_fma(Trow[l], z[l], acc);
-      Trow[j] = ti == j ? tj : (ti < j ? -tj * acc : 0.0);
-    }
-    if (tid == 0 && j < nb) tau[j] = tj;
-    double p[PNB];
-#pragma unroll
-    for (int c = 0; c < PNB; ++c) p[c] = 0.0;
-#pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-      const int r = tid + 512 * k;
-      const double v = r > j ? scale * x[k][j] : (r == j ? 1.0 : 0.0);
-#pragma unroll
-      for (int c = 0; c < PNB; ++c)  // constant trip counts: every loop unrolls, the arrays stay in registers
-        if (c > j) x[k][c] = __builtin_fma(-z[c], v, x[k][c]);
-      x[k][j] = r > j ? v : (r == j ? beta : x[k][j]);
-      if (j + 1 < PNB) {
-        const double a = r > j + 1 ? x[k][j + 1] : 0.0;
-#pragma unroll
-        for (int c = 0; c < PNB; ++c) p[c] = __builtin_fma(a, x[k][c], p[c]);
-      }
-    }
-    if (j + 1 < PNB) {
-      lds_f64* rb = rowb + ((j + 1) & 1) * PNB;
-      if (tid == j + 1) {
-#pragma unroll
-        for (int c = 0; c < PNB; ++c) rb[c] = x[0][c];
-      }
-      S = panel_sums16(p, red + ((j + 1) & 1) * 8 * PNB);
-      R = rb[cl];
-    }
-  }
-  if (tid < PNB) {
+  for (int c = 0; c < PNB; ++c) Trow[c] = 0.0;
+  panel_sums<0, NR>(x, r0, red, S, R);
+  panel_step<0, NR>(x, r0, S, R, ms, Trow, tau, nb, red);
+  if (threadIdx.x >= 448 && lane < PNB) {  // wavefront 7 keeps T
 #pragma unroll
     for (int c = 0; c < PNB; ++c) {
-      Tl[tid * PNB + c] = Trow[c];
-      Tg[tid * PNB + c] = Trow[c];
+      Tl[li * PNB + c] = Trow[c];
+      Tg[li * PNB + c] = Trow[c];
     }
   }
-  // registers -> LDS -> global
 #pragma unroll
-  for (int k = 0; k < RPT; ++k) {
-    const int r = tid + 512 * k;
-    if (r < mr) {
-#pragma unroll
-      for (int c = 0; c < PNB; ++c) L[r * PLD + c] = x[k][c];
-    }
-  }
-  __syncthreads();
-  for (int e = tid; e < ne; e += 512) {
-    const int r = e >> 4, c = e & 15;
-    if (c < nb) P[(int64_t)r * ld + c] = L[r * PLD + c];
+  for (int q = 0; q < NR; ++q) {
+    const int r = 32 * q + r0;
+    if (r < mr && li < nb) P[(int64_t)r * ld + li] = r > li ? x[q] * ms : x[q];
   }
   __syncthreads();
 }
 
-// QR of W (global rows x cols, ld) whose panels fit LDS (rows * PLD <= 16384):
-// each panel is factored in registers (reg_panel), its reflectors and T
-// written back (T of every panel to Tg, for q_form_tall), and the trailing
-// columns updated by tall_wy with the reflectors read from W.  L: the tall
-// layout (TALL_LDS doubles); the panel is staged through its first part,
-// which tall_wy reuses once the panel is written back.
+// ---------------------------------------------------------------------------
+// Blocked QR and Q formation on this workgroup alone, by column groups in
+// registers (left-looking): a group of NT 16-column tiles is loaded once, in the
+// layout of the panels (lane (lk, li) of wavefront w: column li, rows 32 q + 4 w +
+// lk), every earlier panel is applied to it there, its own panels are factored
+// there, and it is stored once.  That layout is also the MFMA's: one register
+// over the lanes is 4 rows x 16 columns, operand B (and, of V, V^T's operand A);
+// four registers are a 16 x 16 block, a D tile.  Applying panel (V, T):
+//   W = V^T M: a product per register, the wavefronts' partials added through LDS
+//   U = op(T) W: 16 x 16 x 16, by every wavefront for itself
+//   M -= V U: V's registers turned round in LDS (block_to_a), a block at a time
+// so V is read once per group, the next panel's while this one is applied, and M
+// never: a 570 x 285 QR moves 7 MB instead of the 15 MB of updating all columns
+// right of each panel, which at 256 workgroups streaming their matrices from HBM
+// was its bound (1.07 ms; now 1.03, alone on the chip 0.94; 0.25 ms is its 77
+// Mflop at one CU's 0.31 Tflop/s: half of the rest is the panels).  LDS at L: 4096 partials | 512 W | 8 x 272 turning | 288 sums | T.
+// ---------------------------------------------------------------------------
+constexpr int QC_W = 4096, QC_S = QC_W + 512, QC_RED = QC_S + 8 * 16 * PLD, QC_T = QC_RED + 2 * 8 * PNB + 2 * PNB;
+static_assert(QC_T + PNB * PNB <= TALL_LDS, "column-group QR: LDS");
+
+// Block k (four registers) of the panel whose first column and row are `top`:
+// row r of the matrix is row r - top of the panel.
+template <int NR>
+__device__ __forceinline__ void qc_load_v(const glb_f64* W, int rows, int ld, int top, int cmax, int k, double (&v)[NR]) {
+  const int lane = threadIdx.x & 63, li = lane & 15, r0 = opaque(4 * (threadIdx.x >> 6) + (lane >> 4));
+  const int c = min(top + li, cmax);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[4 * k + e] = W[(int64_t)min(32 * (4 * k + e) + r0, rows - 1) * ld + c];
+}
+
+// M (NT tiles of NR registers) <- (I - V op(T) V^T) M; ta = op(T) as operand A.
+// v: V as loaded (its unit diagonal, the zeros above and past the last row and
+// past column kk put in here), blocks [k0, k1); next(k) may load the next panel's
+// block k into v as soon as this one's is done with.
+template <int NR, int NT, typename F>
+__device__ __forceinline__ void qc_apply(double (&v)[NR], const double (&ta)[4], double (&m)[NT][NR], int rows, int top,
+                                         int kk, int k0, int k1, lds_f64* L, F next) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  lds_f64* S = L + QC_S + wv * (16 * PLD);
+  f64x4 w[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) w[t] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < NR / 4; ++k) {
+    if (k >= k0 && k < k1) {
+      const int li = opaque(lane & 15), r0 = 4 * wv + (lane >> 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = 32 * (4 * k + e) + r0, d = r - top - li;
+        v[4 * k + e] = (r < rows && d > 0 && top + li < kk) ? v[4 * k + e] : (d == 0 ? 1.0 : 0.0);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) w[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[4 * k + e], m[t][4 * k + e], w[t], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) L[(t * 8 + wv) * 256 + e * 64 + lane] = w[t][e];
+  __syncthreads();
+  if (tid < NT * 256) {
+    const lds_f64* p = L + (tid >> 8) * 2048 + (tid & 255);
+    double x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = p[i * 256];
+    L[QC_W + tid] = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+  }
+  __syncthreads();
+  f64x4 u[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) u[t] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      u[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ta[q], L[QC_W + t * 256 + q * 64 + lane], u[t], 0, 0, 0);
+#pragma unroll
+  for (int t = 0; t < NT; ++t) u[t] = -u[t];
+#pragma unroll
+  for (int k = 0; k < NR / 4; ++k) {
+    if (k >= k0 && k < k1) {
+      const double vb[4] = {v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
+      double a[4];
+      block_to_a(S, vb, a);
+      next(k);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          f64x4 d = {m[t][4 * k], m[t][4 * k + 1], m[t][4 * k + 2], m[t][4 * k + 3]};
+          d = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], u[t][q], d, 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) m[t][4 * k + e] = d[e];
+        }
+    }
+  }
+}
+
+// x[q] <- x[q + n] (zeros in): the finished rows leave the registers
+template <int NR>
+__device__ __forceinline__ void qc_shift(double (&x)[NR], int n) {
+#pragma unroll
+  for (int b = 1; b < NR; b *= 2)
+    if (n & b) {
+#pragma unroll
+      for (int q = 0; q < NR; ++q) x[q] = q + b < NR ? x[q + b < NR ? q + b : 0] : 0.0;
+    }
+}
+
+// One panel in registers: x's rows from `off` (0 or 16) of its first register
+// on; see panel_step.  Stores tau, T (Tl and Tg); leaves R and the unscaled
+// reflectors in x and their scale in ms.
+template <int NP, int NR>
+__device__ __forceinline__ void qc_panel(double (&x)[NR], int off, double& ms, double* tau, int nb, double* Tg,
+                                         lds_f64* L) {
+  const int lane = threadIdx.x & 63, li = lane & 15, r0 = 4 * (threadIdx.x >> 6) + (lane >> 4) - off;
+  double Trow[PNB], S, R;
+#pragma unroll
+  for (int c = 0; c < PNB; ++c) Trow[c] = 0.0;
+  panel_sums<0, NP>(x, r0, L + QC_RED, S, R);
+  panel_step<0, NP>(x, r0, S, R, ms, Trow, tau, nb, L + QC_RED);
+  if (threadIdx.x >= 448 && lane < PNB) {  // wavefront 7 keeps T
+#pragma unroll
+    for (int c = 0; c < PNB; ++c) {
+      L[QC_T + li * PNB + c] = Trow[c];
+      Tg[li * PNB + c] = Trow[c];
+    }
+  }
+}
+
+// QR of W (global, rows <= 32 NR, cols, ld) as qr_panel: R on and above the
+// diagonal, reflectors below, tau, T of every panel in Tg.
+template <int NR, int NT>
+__device__ __noinline__ void qr_cols(double* W_in, int rows_in, int cols_in, int ld_in, double* tau, double* Tg,
+                                     lds_f64* L) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4, row0 = 4 * (threadIdx.x >> 6) + lk;
+  const int rows = uni(rows_in), cols = uni(cols_in), ld = uni(ld_in);
+  const int kk = rows < cols ? rows : cols;
+  const int k1 = (rows + 127) >> 7;  // register blocks that hold rows
+  glb_f64* W = (glb_f64*)W_in;
+  const glb_f64* Tgg = (const glb_f64*)Tg;
+  QTT_PT_INIT;
+  for (int c0 = 0; c0 < cols; c0 += 16 * NT) {
+    double m[NT][NR], v[NR], ta[4];
+    const int np = min(c0, kk + 15) >> 4;  // earlier panels
+    const int r0 = opaque(row0);
+    if (np > 0) {
+#pragma unroll
+      for (int k = 0; k < NR / 4; ++k)
+        if (k < k1) qc_load_v(W, rows, ld, 0, ld - 1, k, v);
+    }
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      if (32 * q < rows) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const double x = W[(int64_t)min(32 * q + r0, rows - 1) * ld + min(c0 + 16 * t + li, cols - 1)];
+          m[t][q] = (32 * q + r0 < rows && c0 + 16 * t + li < cols) ? x : 0.0;
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) m[t][q] = 0.0;
+      }
+    }
+#pragma clang loop unroll(disable)
+    for (int i = 0; i < np; ++i) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) ta[q] = Tgg[i * PNB * PNB + (4 * q + lk) * PNB + li];  // T^T
+      const int top = 16 * i, nk0 = (top + 16) >> 7;
+      qc_apply(v, ta, m, rows, top, cols, top >> 7, k1, L, [&](int k) {
+        if (i + 1 < np && k >= nk0) qc_load_v(W, rows, ld, top + 16, ld - 1, k, v);
+      });
+    }
+    QTT_PT(8);
+    auto store = [&](const double (&x)[NR], int t, int qoff, int qend, bool scaled, int off, double ms) {
+      const int c = c0 + 16 * t + li, rr = opaque(row0);
+#pragma unroll
+      for (int q = 0; q < NR; ++q) {
+        const int r = 32 * (q + qoff) + rr;
+        if (q < qend && r < rows && c < cols)
+          W[(int64_t)r * ld + c] = scaled && (q > 0 || rr - off > li) ? x[q] * ms : x[q];
+      }
+    };
+    if (c0 >= kk) {  // right of the last panel: only updated
+#pragma unroll
+      for (int t = 0; t < NT; ++t) store(m[t], t, 0, NR, false, 0, 1.0);
+    } else {
+      const int q0 = c0 >> 5, nrem = ((rows + 31) >> 5) - q0;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        store(m[t], t, 0, q0, false, 0, 1.0);  // finished rows
+        qc_shift(m[t], q0);
+      }
+#pragma clang loop unroll(disable)
+      for (int t = 0; t < NT; ++t) {  // the tile at hand is m[0]
+        const int p0 = c0 + 16 * t, off = p0 & 31;
+        double ms = 1.0;
+        QTT_PT(9);
+        if (p0 < kk) {
+          double* Tp = Tg + (p0 / PNB) * PNB * PNB;
+          const int nb = min(PNB, kk - p0);
+          if (nrem <= 5) {
+            qc_panel<5>(m[0], off, ms, tau + p0, nb, Tp, L);
+          } else if constexpr (NR > 10) {
+            if (nrem <= 10) qc_panel<10>(m[0], off, ms, tau + p0, nb, Tp, L);
+            else qc_panel<NR>(m[0], off, ms, tau + p0, nb, Tp, L);
+          } else {
+            qc_panel<NR>(m[0], off, ms, tau + p0, nb, Tp, L);
+          }
+        }
+        QTT_PT(1);
+        store(m[0], t, q0, NR, p0 < kk, off, ms);
+        QTT_PT(9);
+        if constexpr (NT > 1) {
+          if (t + 1 < NT) {
+            double y[1][NR];
+#pragma unroll
+            for (int q = 0; q < NR; ++q) {
+              v[q] = m[0][q] * ms;
+              y[0][q] = m[NT - 1][q];
+            }
+            __syncthreads();  // T in LDS
+            if (p0 < kk) {
+#pragma unroll
+              for (int q = 0; q < 4; ++q) ta[q] = L[QC_T + (4 * q + lk) * PNB + li];
+              qc_apply(v, ta, y, 32 * NR, off, cols, 0, (nrem + 3) >> 2, L, [](int) {});
+            }
+#pragma unroll
+            for (int q = 0; q < NR; ++q) m[0][q] = y[0][q];
+            QTT_PT(10);
+          }
+        }
+      }
+    }
+    __syncthreads();
+    QTT_PT(9);
+    if (threadIdx.x == 0 && blockIdx.x == 0) QTT_PANEL_COUNT;
+  }
+}
+
+// x <- Q or U of qr_cols' reflectors (W, rows <= 32 NR), row-major in Mq (rows
+// x ncol): as q_form_tall's first part.
+template <int NR, int NT>
+__device__ __noinline__ void q_cols(const double* W_in, int rows_in, int k_in, int ld_in, const double* Tg_in,
+                                    double* Mq_in, const double* Jb_in, int n_in, const int* perm, int m_in,
+                                    lds_f64* L) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4, row0 = 4 * (threadIdx.x >> 6) + lk;
+  const int rows = uni(rows_in), kk = uni(k_in), ld = uni(ld_in), n = uni(n_in);
+  const bool isu = Jb_in != nullptr;
+  const int ncol = isu ? uni(m_in) : kk, k1 = (rows + 127) >> 7, npan = (kk + PNB - 1) / PNB;
+  const glb_f64 *W = (const glb_f64*)W_in, *Tg = (const glb_f64*)Tg_in, *Jb = (const glb_f64*)Jb_in;
+  glb_f64* Mq = (glb_f64*)Mq_in;
+  for (int c0 = 0; c0 < ncol; c0 += 16 * NT) {
+    double m[NT][NR], v[NR], ta[4];
+    const int r0 = opaque(row0);
+    // Q: a panel right of the group's columns finds zeros only
+    const int last = isu ? npan - 1 : min(npan - 1, (c0 + 16 * NT - 1) >> 4);
+#pragma unroll
+    for (int k = 0; k < NR / 4; ++k)
+      if (k >= (16 * last) >> 7 && k < k1) qc_load_v(W, rows, ld, 16 * last, kk - 1, k, v);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int c = c0 + 16 * t + li, pc = (isu && c < ncol) ? (perm ? perm[c] : c) : 0;
+#pragma unroll
+      for (int q = 0; q < NR; ++q) {
+        const int r = 32 * q + r0;
+        if (isu) {
+          m[t][q] = 0.0;
+          if (32 * q < n) {
+            const double x = Jb[(int64_t)pc * n + min(r, n - 1)];
+            m[t][q] = (r < n && c < ncol) ? x : 0.0;
+          }
+        } else {
+          m[t][q] = (r == c && c < ncol) ? 1.0 : 0.0;
+        }
+      }
+    }
+#pragma clang loop unroll(disable)
+    for (int i = last; i >= 0; --i) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) ta[q] = Tg[i * PNB * PNB + li * PNB + 4 * q + lk];
+      const int top = 16 * i;
+      if (i < last && ((top + 16) >> 7) != (top >> 7)) {  // the block that this panel reaches first
+#pragma unroll
+        for (int k = 0; k < NR / 4; ++k)
+          if (k == top >> 7 && k < k1) qc_load_v(W, rows, ld, top, kk - 1, k, v);
+      }
+      qc_apply(v, ta, m, rows, top, kk, top >> 7, k1, L, [&](int k) {
+        if (i > 0) qc_load_v(W, rows, ld, top - 16, kk - 1, k, v);
+      });
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int c = c0 + 16 * t + li, rr = opaque(row0);
+#pragma unroll
+      for (int q = 0; q < NR; ++q) {
+        const int r = 32 * q + rr;
+        if (r < rows && c < ncol) Mq[(int64_t)r * ncol + c] = m[t][q];
+      }
+    }
+  }
+  __syncthreads();
+}
+
+// QR of W (global rows x cols, ld) of at most 963 rows (rows * PLD <= 16384): on
+// this workgroup alone by column groups (qr_cols), or, large and with helper
+// workgroups, each panel in registers (reg_panel) and the trailing columns
+// updated by all (tall_wy) with the reflectors read from W.  R, the reflectors
+// and tau as LAPACK leaves them, T of every panel in Tg for q_form_tall.  L: the
+// tall layout (TALL_LDS doubles).
 __device__ __noinline__ void qr_panel(double* W, int rows_in, int cols_in, int ld_in, double* tau, double* Tg,
                                       lds_f64* L, CoopJob* job, int nwg_in, int* iflag) {
   const int nwg = uni(nwg_in);
   const int rows = uni(rows_in), cols = uni(cols_in), ld = uni(ld_in);
   const int k = rows < cols ? rows : cols;
+  QTT_PT_INIT;
+  if (!(job != nullptr && nwg > 1) || (int64_t)rows * cols <= QC_SHARE) {
+    if (rows <= 256) qr_cols<8, 2>(W, rows, cols, ld, tau, Tg, L);
+    else if (rows <= 640) qr_cols<20, 2>(W, rows, cols, ld, tau, Tg, L);
+    else qr_cols<32, 1>(W, rows, cols, ld, tau, Tg, L);
+    QTT_PT(4);
+    return;
+  }
   lds_f64* red = L + 8 * TALL_REGION;          // 2 x 8 x PNB sums, 2 x PNB rows
   lds_f64* Tl = L + 8 * TALL_REGION + 16 * 128;
-  // on this workgroup alone, panels go in pairs: the second panel's columns
-  // are updated by the first, and the rest by both in one pass (tall_wy2)
-  const bool pairs = !(job != nullptr && nwg > 1);
-  lds_f64* T1 = red + 512;   // the first panel's T while the second is factored
-  lds_f64* Gp = red + 768;   // V2^T V1
-  QTT_PT_INIT;
-  auto panel = [&](int p0, int nb) {
-    if (rows - p0 <= 512)
-      reg_panel<1>(W, rows, ld, p0, nb, tau + p0, Tg + (p0 / PNB) * PNB * PNB, Tl, L, red);
-    else
-      reg_panel<2>(W, rows, ld, p0, nb, tau + p0, Tg + (p0 / PNB) * PNB * PNB, Tl, L, red);
-  };
-  for (int p0 = 0; p0 < k;) {
+  for (int p0 = 0; p0 < k; p0 += PNB) {
     const int nb = k - p0 < PNB ? k - p0 : PNB, mr = rows - p0;
-    panel(p0, nb);
+    double* Tp = Tg + (p0 / PNB) * PNB * PNB;
+    if (mr <= 160) reg_panel<5>(W, rows, ld, p0, nb, tau + p0, Tp, Tl, red);
+    else if (mr <= 320) reg_panel<10>(W, rows, ld, p0, nb, tau + p0, Tp, Tl, red);
+    else if (mr <= 576) reg_panel<18>(W, rows, ld, p0, nb, tau + p0, Tp, Tl, red);
+    else reg_panel<32>(W, rows, ld, p0, nb, tau + p0, Tp, Tl, red);
     QTT_PT(1);
-    const int p1 = p0 + nb;
-    double* M = W + (int64_t)p0 * ld;
-    const double* V1 = W + (int64_t)p0 * ld + p0;
-    if (pairs && p1 < k && p1 + PNB < cols) {
-      const int nb2 = k - p1 < PNB ? k - p1 : PNB;
-      tall_wy(M, ld, mr, p1, p1 + nb2, V1, ld, nb, Tl, true, L, nullptr, 1, iflag);
-      __syncthreads();
-      for (int e = threadIdx.x; e < PNB * PNB; e += blockDim.x) T1[e] = Tl[e];
-      __syncthreads();
-      panel(p1, nb2);
-      tall_wy2(M, ld, mr, p1 + nb2, cols, V1, W + (int64_t)p1 * ld + p1, ld, nb, nb2, T1, Tl, Gp, L, true, false);
-      p0 = p1 + nb2;
-    } else {
-      if (p1 < cols) tall_wy(M, ld, mr, p1, cols, V1, ld, nb, Tl, true, L, job, nwg, iflag);
-      p0 = p1;
-    }
+    if (p0 + nb < cols)
+      tall_wy(W + (int64_t)p0 * ld, ld, mr, p0 + nb, cols, W + (int64_t)p0 * ld + p0, ld, nb, Tl, true, L, job, nwg,
+              iflag);
     __syncthreads();
     QTT_PT(4);
     if (threadIdx.x == 0) QTT_PANEL_COUNT;
@@ -2539,52 +2864,136 @@ __device__ __noinline__ void mode_product_mfma32(const double* Rrows, const int*
 // Mode product with R in global memory (the global-workspace path) as FP64
 // MFMA tiles, v_mfma_f64_16x16x4f64: Y[(aa*m + i)*Bu + bb] = sum_c
 // R[perm(i)][c] U[(aa*nu + c)*Bu + bb] over the output columns j = aa*Bu + bb
-// in [j0, j1).  A unit is 32 output rows (two 16-row tiles sharing each B
-// operand) by 16 columns; A = R rows (lane: row li, column lk of the k-step),
-// B = U (lane: k-row lk, column li), D element e = row lk + 4e, column li.
-__device__ __noinline__ void mode_product_mfma(const double* Rrows, const int* perm, bool use_perm, int m_in,
-                                               int b_in, const double* Uc, double* gY, int Au_in, int nu_in,
-                                               int Bu_in, int j0_in, int j1_in) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
-  const int li = lane & 15, lk = lane >> 4;
-  const int m = uni(m_in), b = uni(b_in), nu = uni(nu_in), Bu = uni(Bu_in), j0 = uni(j0_in), j1 = uni(j1_in);
-  (void)Au_in;
-  const int nit = (m + 31) >> 5, njt = (j1 - j0 + 15) >> 4;
-  for (int u = wv; u < nit * njt; u += nwv) {
-    const int it = u / njt, jt = u - it * njt;
-    const int i0 = it * 32, jc = j0 + jt * 16 + li;
-    const bool jon = jc < j1;
-    const int aa = jon ? jc / Bu : 0, bb = jon ? jc - aa * Bu : 0;
-    const double* up = Uc + (int64_t)aa * nu * Bu + bb;
-    const int ra = i0 + li, rb = i0 + 16 + li;
-    const bool aon = ra < m, bon = rb < m;
-    const double* rpa = Rrows + (int64_t)(aon ? (use_perm ? perm[ra] : ra) : 0) * b;
-    const double* rpb = Rrows + (int64_t)(bon ? (use_perm ? perm[rb] : rb) : 0) * b;
-    f64x4 da = {0.0, 0.0, 0.0, 0.0}, db = {0.0, 0.0, 0.0, 0.0};
-    // without a permutation the rows are a QR's R (upper triangular, its zeros
-    // stored): the k-steps left of the tile's first row add nothing
-    for (int c0 = use_perm ? 0 : i0; c0 < nu; c0 += 32) {  // 8 k-steps: all 24 loads in flight before the MFMAs
-      double bv[8], av[8], aw[8];
+// in [j0, j1).  A unit is 32 output rows by NT 16-column tiles of one wavefront:
+// A = R rows (lane: row li, column lk of the k-step), loaded with the columns
+// across the lanes and turned round in LDS (block_to_a: two 128-byte lines per
+// 16 lanes; in operand order each load touched 16 lines, which bounded the
+// product), B = U (lane: k-row lk, column li), D element e = row lk + 4e, column
+// li; 16 k at a time, the next 16 in flight.  u <- R u of a 285 x 285 R and 570
+// columns: 0.69 -> 0.34 ms (0.16 ms at one CU's 0.31 Tflop/s); S: 544 doubles of
+// LDS per wavefront.
+template <int NT>
+__device__ __forceinline__ void mode_product_unit(const glb_f64* R, const int* perm, bool use_perm, int m, int b,
+                                                  const glb_f64* U, glb_f64* Y, int nu, int Bu, int j1, int i0,
+                                                  int jt0, lds_f64* S) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  int ro[8];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int c = c0 + 4 * q + lk;
-        const bool con = c < nu;
-        bv[q] = (jon && con) ? up[(int64_t)c * Bu] : 0.0;
-        av[q] = (aon && con) ? rpa[c] : 0.0;
-        aw[q] = (bon && con) ? rpb[c] : 0.0;
-      }
+  for (int e = 0; e < 8; ++e) {
+    const int i = min(i0 + 4 * e + lk, m - 1);
+    ro[e] = (use_perm ? perm[i] : i) * b;
+  }
+  const glb_f64* up[NT];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        da = __builtin_amdgcn_mfma_f64_16x16x4f64(av[q], bv[q], da, 0, 0, 0);
-        db = __builtin_amdgcn_mfma_f64_16x16x4f64(aw[q], bv[q], db, 0, 0, 0);
-      }
+  for (int t = 0; t < NT; ++t) {
+    const int jc = min(jt0 + 16 * t + li, j1 - 1), aa = jc / Bu;
+    up[t] = U + (int64_t)aa * nu * Bu + (jc - aa * Bu);
+  }
+  double av[8], bv[NT][4];
+  auto load = [&](int c0) {
+    const int ca = c0 + li, cc = min(ca, nu - 1);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) av[e] = R[ro[e] + cc];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int64_t o = (int64_t)min(c0 + 4 * q + lk, nu - 1) * Bu;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) bv[t][q] = up[t][o];
     }
-    if (jon) {
+  };
+  f64x4 d0[NT], d1[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) d0[t] = d1[t] = f64x4{0.0, 0.0, 0.0, 0.0};
+  // without a permutation the rows are a QR's R (upper triangular, its zeros
+  // stored): the k-steps left of the tile's first row add nothing
+  const int cs = use_perm ? 0 : i0;
+  load(cs);
+  for (int c0 = cs; c0 < nu; c0 += 16) {
+    const bool in = c0 + li < nu;
+    double x0[4], x1[4], a0[4], a1[4], bw[NT][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x0[e] = in ? av[e] : 0.0;
+      x1[e] = in ? av[4 + e] : 0.0;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) bw[t][e] = bv[t][e];
+    }
+    load(c0 + 16);  // past the last step: clamped, not used
+    block_to_a(S, x0, a0);
+    block_to_a(S + 16 * PLD, x1, a1);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        d0[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[q], bw[t][q], d0[t], 0, 0, 0);
+        d1[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[q], bw[t][q], d1[t], 0, 0, 0);
+      }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int jc = jt0 + 16 * t + li, aa = min(jc, j1 - 1) / Bu, bb = jc - aa * Bu;
+    if (jc < j1) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int i = i0 + lk + 4 * e;
-        if (i < m) gY[((int64_t)aa * m + i) * Bu + bb] = da[e];
-        if (i + 16 < m) gY[((int64_t)aa * m + i + 16) * Bu + bb] = db[e];
+        if (i < m) Y[((int64_t)aa * m + i) * Bu + bb] = d0[t][e];
+        if (i + 16 < m) Y[((int64_t)aa * m + i + 16) * Bu + bb] = d1[t][e];
+      }
+    }
+  }
+}
+
+__device__ __noinline__ void mode_product_mfma(const double* Rrows, const int* perm, bool use_perm, int m_in,
+                                               int b_in, const double* Uc, double* gY, int nu_in, int Bu_in,
+                                               int j0_in, int j1_in, lds_f64* lw) {
+  const int wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
+  const int m = uni(m_in), b = uni(b_in), nu = uni(nu_in), Bu = uni(Bu_in), j0 = uni(j0_in), j1 = uni(j1_in);
+  const glb_f64 *R = (const glb_f64*)Rrows, *U = (const glb_f64*)Uc;
+  glb_f64* Y = (glb_f64*)gY;
+  lds_f64* S = lw + wv * (2 * 16 * PLD);
+  const int nit = (m + 31) >> 5, nt = (j1 - j0 + 15) >> 4;
+  // tiles per unit: as many as leave the wavefronts' last round full (a unit of
+  // NT tiles costs about NT + 1/4: its R block is loaded and turned round once)
+  auto cost = [&](int w) { return (nit * ((nt + w - 1) / w) + nwv - 1) / nwv * (4 * w + 1); };
+  const int c4 = cost(4), c2 = cost(2), c1 = cost(1);
+  __syncthreads();  // S is the caller's LDS
+  if (c4 <= c2 && c4 <= c1) {
+    const int nj = (nt + 3) >> 2;
+    for (int u = wv; u < nit * nj; u += nwv)
+      mode_product_unit<4>(R, perm, use_perm, m, b, U, Y, nu, Bu, j1, (u / nj) * 32, j0 + (u - (u / nj) * nj) * 64, S);
+  } else if (c2 <= c1) {
+    const int nj = (nt + 1) >> 1;
+    for (int u = wv; u < nit * nj; u += nwv)
+      mode_product_unit<2>(R, perm, use_perm, m, b, U, Y, nu, Bu, j1, (u / nj) * 32, j0 + (u - (u / nj) * nj) * 32, S);
+  } else {
+    for (int u = wv; u < nit * nt; u += nwv)
+      mode_product_unit<1>(R, perm, use_perm, m, b, U, Y, nu, Bu, j1, (u / nt) * 32, j0 + (u - (u / nt) * nt) * 16, S);
+  }
+}
+
+// Rb (k x b) <- the upper triangle of W (ld b), zeros below: a row per
+// wavefront, two rows' loads in flight.
+__device__ __noinline__ void copy_upper(double* Rb_in, const double* W_in, int k, int b) {
+  glb_f64* Rb = (glb_f64*)Rb_in;
+  const glb_f64* W = (const glb_f64*)W_in;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
+  for (int i = 2 * wv; i < k; i += 2 * nwv) {
+    const int i1 = min(i + 1, k - 1);
+    for (int c0 = lane; c0 < b; c0 += 256) {
+      double t[2][4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int c = min(c0 + 64 * u, b - 1);
+        t[0][u] = W[(int64_t)i * b + c];
+        t[1][u] = W[(int64_t)i1 * b + c];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int c = c0 + 64 * u;
+        if (c < b) {
+          Rb[(int64_t)i * b + c] = c >= i ? t[0][u] : 0.0;
+          if (i + 1 < k) Rb[(int64_t)(i + 1) * b + c] = c >= i + 1 ? t[1][u] : 0.0;
+        }
       }
     }
   }
@@ -2844,8 +3253,8 @@ __device__ void coop_work(CoopJob* job, int wg, int nwg, lds_f64* lw) {
         mode_product_body<QTT_F32_SPLIT>(job->R, job->perm, job->use_perm != 0, job->m, job->rb, job->U, job->Y,
                                          job->Au, job->nu, job->Bu, j0, j1);
       else
-        mode_product_mfma(job->R, job->perm, job->use_perm != 0, job->m, job->rb, job->U, job->Y, job->Au, job->nu,
-                          job->Bu, j0, j1);
+        mode_product_mfma(job->R, job->perm, job->use_perm != 0, job->m, job->rb, job->U, job->Y, job->nu, job->Bu, j0,
+                          j1, lw);
     }
   } else if (type == 3) {
     const long long tot = job->ytot;
@@ -3048,7 +3457,7 @@ __device__ __noinline__ void coop_wy_rows(CoopJob* job, int wg, int nwg) {
 // workgroup 0 quits.  A job of workgroups 0 .. nact-1 is not followed by the
 // next before they have all counted it, so a helper that takes part always
 // sees its job; one that does not may see a later job and skips to it.
-__device__ void coop_helper(CoopJob* job, int wg, int nwg, lds_i32* sflag, lds_f64* lw) {
+__device__ __noinline__ void coop_helper(CoopJob* job, int wg, int nwg, lds_i32* sflag, lds_f64* lw) {
   const int tid = threadIdx.x;
   for (int expected = 1;;) {
     if (tid == 0) {
@@ -3396,10 +3805,7 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
       double* Mq = Tg + (((int64_t)k + PNB) * PNB);
       if (pmode == 3) qr_tall(W, rows, b, b, tau, Tg, pnl, job, nwg, iflag);  // panels in global memory
       else qr_panel(W, rows, b, b, tau, Tg, pnl, job, nwg, iflag);            // panels in LDS
-      for (int e = tid; e < k * b; e += bs) {
-        const int i = e / b, c = e - i * b;
-        Rb[e] = c >= i ? W[(int64_t)i * b + c] : 0.0;
-      }
+      copy_upper(Rb, W, k, b);
       __syncthreads();
       QTT_PHASE(-1, 2);  // factored
       if (lazyT) {
@@ -3458,10 +3864,7 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
       } else if (pmode) {  // blocked QR; the reflectors stay in W for U below
         if (pmode == 3) qr_tall(W, rows, b, b, tau, vbuf, pnl, job, nwg, iflag);
         else qr_panel(W, rows, b, b, tau, vbuf, pnl, job, nwg, iflag);
-        for (int e = tid; e < b * b; e += bs) {
-          const int i = e / b, c = e - i * b;
-          Rb[e] = c >= i ? W[(int64_t)i * b + c] : 0.0;
-        }
+        copy_upper(Rb, W, b, b);
       } else {
         geqr2<G>(W, rows, b, b, tau);
         for (int e = tid; e < b * b; e += bs) {
@@ -3552,11 +3955,11 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
       return cv;
     };
     // Wide or square matrices on the global workspace: the QR-preconditioned
-    // rounds, from 12 rows (below, the two QRs cost what the rounds do) where R2 and J fit LDS;
+    // rounds, from 8 rows (below, the two QRs cost what the rounds do) where R2 and J fit LDS;
     // with helper workgroups again from 192 (3D comb operate: 256 x 384 moves 25.3
     // -> 12.7 ms; at 128 x 128 the two QRs cost what the saved sweeps do); alone,
     // where the rounds run in global memory, whenever the lanes hold a row.
-    const bool precond = !REG && gws && pnl != nullptr && !tall && n >= 12 &&
+    const bool precond = !REG && gws && pnl != nullptr && !tall && n >= 8 &&
                          (n <= 96 || (job && nwg > 1 ? n >= 192 && b <= 512 : n <= 512));
     // A tall move that can drop nothing (cutoff <= 0: at most exactly zero singular
     // values would go; maxdim >= n) and whose R has no zero on its diagonal
@@ -3698,7 +4101,7 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
       else if (prec == QTT_F32_SPLIT)
         mode_product<QTT_F32_SPLIT>(Rrows, perm, use_perm, m, b, Uc, gY, (int)Au, (int)nu, (int)Bu);
       else
-        mode_product_mfma(Rrows, perm, use_perm, m, b, Uc, gY, (int)Au, (int)nu, (int)Bu, 0, (int)(Au * Bu));
+        mode_product_mfma(Rrows, perm, use_perm, m, b, Uc, gY, (int)nu, (int)Bu, 0, (int)(Au * Bu), pnl_any);
     } else {
       if (prec == QTT_F32) mode_product<QTT_F32>(Rrows, perm, use_perm, m, b, Uc, gY, (int)Au, (int)nu, (int)Bu);
       else if (prec == QTT_F32_SPLIT)
@@ -3706,10 +4109,51 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
       else mode_product<QTT_F64>(Rrows, perm, use_perm, m, b, Uc, gY, (int)Au, (int)nu, (int)Bu);
     }
     __syncthreads();
-    for (int e = tid; e < ytot; e += bs) Ud[e] = gY[e];
+    if (gws) copy_doubles(Ud, gY, ytot);
+    else
+      for (int e = tid; e < ytot; e += bs) Ud[e] = gY[e];
   }
   QTT_PHASE(-1, 4);  // u written
   return m;
+}
+
+template <typename T>
+__device__ __forceinline__ T* uni_ptr(T* p) {
+  const unsigned long long v = (unsigned long long)p;
+  return (T*)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+              (unsigned)__builtin_amdgcn_readfirstlane((int)v));
+}
+
+// A move on the global workspace, as a function of its own: the blocked QR and
+// the products it calls use every register, and inlined with them the moves in
+// LDS kept what they hold across their steps in scratch memory (418 spilled
+// registers against 35; a 1D operate's sweep 577 -> 725 us).
+template <int G>
+__device__ __noinline__ int run_move_global(const SweepArgs* a_in, lds_f64* lds, lds_f64* pnl, int pnl_cap, int pmode,
+                                            int rows, int b, int tr, int Bx, int Au, int nu, int Bu, int x, int u,
+                                            double* lazyT, const double* uT, lds_f64* pnl_any) {
+  const SweepArgs& a = *uni_ptr(a_in);
+  x = uni(x);
+  u = uni(u);
+  return run_move<G, false>(a.gscr, true, a.job, a.nwg, nullptr, false, pnl, uni(pnl_cap), uni(pmode), uni(rows), uni(b),
+                            uni(tr), 0, uni(Bx), uni(Au), uni(nu), uni(Bu), a.data + a.off[x], a.data + a.off[u],
+                            a.data + a.off[u], a.gY, a.cutoff, a.maxdim, a.max_sweeps, a.prec, a.status,
+                            (int*)(lds_i32*)(lds + 16), (double*)lds, (double*)(lds + 24), a.gscr, pnl_any, uni_ptr(lazyT),
+                            uni_ptr(uT));
+}
+
+// A move in LDS of more than 256 rows or columns that the blocked path does not take.
+__device__ __noinline__ int run_move_plain(const SweepArgs* a_in, lds_f64* lds, lds_f64* wsl, int rows, int b, int tr,
+                                           int Bx, int Au, int nu, int Bu, int x, int u, double* lazyT,
+                                           const double* uT, lds_f64* pnl_any) {
+  const SweepArgs& a = *uni_ptr(a_in);
+  x = uni(x);
+  u = uni(u);
+  return run_move<64, false>((double*)wsl, false, nullptr, 1, nullptr, false, nullptr, 0, 0, uni(rows), uni(b), uni(tr), 0,
+                             uni(Bx), uni(Au), uni(nu), uni(Bu), a.data + a.off[x], a.data + a.off[u],
+                             a.data + a.off[u], a.gY, a.cutoff, a.maxdim, a.max_sweeps, a.prec, a.status,
+                             (int*)(lds_i32*)(lds + 16), (double*)lds, (double*)(lds + 24), a.gscr, pnl_any, uni_ptr(lazyT),
+                             uni_ptr(uT));
 }
 
 __global__ void __launch_bounds__(512) truncate_kernel(const SweepArgs* __restrict__ all) {
@@ -3804,7 +4248,17 @@ __global__ void __launch_bounds__(512) truncate_kernel(const SweepArgs* __restri
     lds_f64* pnl = nullptr;
     int pnl_cap = 0;  // doubles of LDS at pnl
     int pmode = 0;
-    if (need > a.ws_lds && TALL_LDS + 64 <= a.ws_lds) pmode = (int64_t)rows * PLD <= 8 * TALL_REGION ? 1 : 3;
+    // The blocked path also takes matrices that would fit LDS where it is the
+    // faster one (float64 products only): more than 256 rows or columns (the LDS
+    // kernels then give a wavefront per column or row pair: a 32 x 285 QR move 950 ->
+    // 270 us, a 32 x 285 SVD move 1300 -> 480), QR moves from 48 x 48 (64 x 80 114 ->
+    // 109 us, 160 x 80 180 -> 122: Q is kept as reflectors and u is an MFMA product),
+    // and wide SVD moves from 24 rows (24 x 80: 212 and 304 -> 234 and 239 us with 7
+    // and 10 sweeps; 20 x 80: 160 -> 208).
+    const bool blocked = TALL_LDS + 64 <= a.ws_lds &&
+                         (need > a.ws_lds || (a.prec == QTT_F64 && (!small || (tr ? rows <= b && rows >= 24 && b >= 48
+                                                                                  : rows >= 48 && b >= 48))));
+    if (blocked) pmode = (int64_t)rows * PLD <= 8 * TALL_REGION ? 1 : 3;
     if (pmode) {
       pnl = pnl_any;
       pnl_cap = QTT_LDS_DOUBLES - poff;
@@ -3824,20 +4278,20 @@ __global__ void __launch_bounds__(512) truncate_kernel(const SweepArgs* __restri
     const double* Uc = a.data + a.off[u];
     double* Ud = a.data + a.off[u];
     int m;
-    if (need <= a.ws_lds) {
+    if (need <= a.ws_lds && !blocked) {
       if (small)
         m = run_move<8, true>(wsl, false, nullptr, 1, jpad, jwave, nullptr, 0, 0, rows, b, tr, rpl, (int)Bx, Au, nu, Bu, Xc, Uc, Ud, a.gY, a.cutoff, a.maxdim, a.max_sweeps, a.prec, a.status,
                         iflag, red, dbc, a.gscr, pnl_any, lazyT, uT);
       else
-        m = run_move<64, false>(wsl, false, nullptr, 1, nullptr, false, nullptr, 0, 0, rows, b, tr, 0, (int)Bx, Au, nu, Bu, Xc, Uc, Ud, a.gY, a.cutoff, a.maxdim, a.max_sweeps, a.prec, a.status,
-                         iflag, red, dbc, a.gscr, pnl_any, lazyT, uT);
+        m = run_move_plain(&a, (lds_f64*)lds, (lds_f64*)wsl, rows, b, tr, (int)Bx, (int)Au, (int)nu, (int)Bu, x, u, lazyT, uT,
+                           pnl_any);
     } else {
       if (small)
-        m = run_move<8, false>(a.gscr, true, a.job, a.nwg, nullptr, false, pnl, pnl_cap, pmode, rows, b, tr, 0, (int)Bx, Au, nu, Bu, Xc, Uc, Ud, a.gY, a.cutoff, a.maxdim, a.max_sweeps, a.prec, a.status,
-                        iflag, red, dbc, a.gscr, pnl_any, lazyT, uT);
+        m = run_move_global<8>(&a, (lds_f64*)lds, pnl, pnl_cap, pmode, rows, b, tr, (int)Bx, (int)Au, (int)nu, (int)Bu, x,
+                               u, lazyT, uT, pnl_any);
       else
-        m = run_move<64, false>(a.gscr, true, a.job, a.nwg, nullptr, false, pnl, pnl_cap, pmode, rows, b, tr, 0, (int)Bx, Au, nu, Bu, Xc, Uc, Ud, a.gY, a.cutoff, a.maxdim, a.max_sweeps, a.prec, a.status,
-                         iflag, red, dbc, a.gscr, pnl_any, lazyT, uT);
+        m = run_move_global<64>(&a, (lds_f64*)lds, pnl, pnl_cap, pmode, rows, b, tr, (int)Bx, (int)Au, (int)nu, (int)Bu, x,
+                               u, lazyT, uT, pnl_any);
     }
     QTT_PHASE(st, 5);
     if (tid == 0) {

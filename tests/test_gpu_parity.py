@@ -483,6 +483,26 @@ def test_truncate_preconditioned_batch_moves(q, po, eng, rng, maxdim):
         assert _compare_networks(q, po, g, ref, fi, rng) < 1e-11
 
 
+@pytest.mark.parametrize("link", [16, 17, 27, 43, 54, 97, 107, 160, 161])
+def test_truncate_column_groups(q, po, eng, rng, link):
+    # kernel-operator products of bond b = 3 link: the QR moves are 2b x b matrices,
+    # 96 (the smallest blocked), 102, 162, 258, 324, 582, 642, 960 and 966 rows, on
+    # both sides of the register classes of the column groups (160, 256, 320, 640
+    # rows; panels of 960 rows at most, above that panels in global memory), with
+    # last columns that fill no tile; then wide SVD moves of 24, 48 and 80 rows and
+    # MFMA mode products of every shape between.
+    s = q.continuous_siteinds(q.named_grid((8, 1)))
+    op = q.fredholm_operator(s)
+    fs = [q.random_itn(s, link_space=c, rng=rng, std=1.0 / math.sqrt(c)) for c in (link, link - 5)]
+    for maxdim in (12, 40):
+        gs, _ = q.operate_batch([op] * 2, fs, maxdim=maxdim)
+        for fi, g in zip(fs, gs):
+            t = fi.topo
+            ref, _ = po.truncate(t.parent, t.sdim, po.contract(t.parent, t.sdim, op.cores, fi.cores), 0.0, maxdim)
+            assert list(g.bonds()) == [c.shape[0] for c in ref]
+            assert _compare_networks(q, po, g, ref, fi, rng) < 1e-11
+
+
 # ------------------------------------------------------------------ comb tree (config-3 shape, reduced)
 def test_comb_operate_and_integrate(q, po, eng, rng):
     from itensornumericalanalysis_jl_amd import workloads
@@ -661,6 +681,24 @@ def test_evaluate_batch(q, po, eng, rng):
         yb = y.cpu().numpy()
         assert rel_l2(yb, oracle_eval(po, f, x)) < TOL
         assert np.array_equal(yb, q.evaluate(f, x))  # same arithmetic as the single-network launch
+
+
+@pytest.mark.parametrize("bond,npts", [(1, 1), (7, 15), (8, 16384), (8, 16385), (9, 7), (16, 12288), (17, 3),
+                                       (32, 12288), (32, 12289), (31, 2)])
+def test_evaluate_few_points(q, po, eng, rng, bond, npts):
+    # one lane per vector entry (few points: up to 16384 for bonds up to 8, 12288
+    # above) on both sides of that rule and of the lane groups of 8, 16 and 32, with
+    # groups that the points do not fill: the oracle's values, and bit for bit those
+    # of the batched kernels (the same order of sums)
+    import torch
+    s = q.continuous_siteinds(q.named_grid((13, 1)))
+    f = q.random_itn(s, link_space=bond, rng=rng, std=1.0 / math.sqrt(bond))
+    xs = rng.uniform(0, 1, (npts, 1))
+    y = q.evaluate(f, xs)
+    yb = q.evaluate_batch([f], [torch.tensor(xs, device="cuda")])[0].cpu().numpy()
+    assert rel_l2(y, oracle_eval(po, f, xs)) < TOL
+    if npts <= (16384 if bond <= 8 else 12288):
+        assert np.array_equal(y, yb)
 
 
 # ------------------------------------------------------------------ gradient
