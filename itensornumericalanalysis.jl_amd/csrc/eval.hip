@@ -402,9 +402,12 @@ __global__ void pack_split_kernel(const double* __restrict__ pack, int64_t n, fl
 // points); here a site is CHI multiply-adds per lane, the vector through LDS,
 // and the rows of the next sites, known from the digits alone, are on their
 // way meanwhile.  The sums run in the order of chain1_site, so the values are
-// bit for bit those of the other kernels.  The cores are read where they lie
-// (no packed copy).  What bounds it with more points: each lane reads its own
-// core row, 64 accesses per load.
+// bit for bit those of the other kernels.  Lanes past the bond keep a zero, also
+// next to entries that overflowed (0 inf would be NaN, and spread): an infinite
+// value stays infinite.  (The lane-per-point kernels form one padded entry at odd
+// bonds and give NaN there.)  The cores are read where they lie (no packed copy).
+// What bounds it with more points: each lane reads its own core row, 64 accesses
+// per load.
 // ---------------------------------------------------------------------------
 template <int CHI>
 __global__ void __launch_bounds__(64)
@@ -424,7 +427,8 @@ eval_chain_few_kernel(const double* __restrict__ data, const int64_t* __restrict
   for (int c = 0; c < QTT_MAX_COORD; ++c)
     if (c < nc) kw[c] = digit_word(active ? xs[p * nc + c] : 0.0, t.ndigits[c], bad);
   double a[D][CHI];
-  auto fetch = [&](int i, double (&x)[CHI]) {  // the row of site nv-1-i for this lane's entry and digit
+  bool has[D];  // this lane holds an entry of the site's vector
+  auto fetch = [&](int i, double (&x)[CHI], bool& on) {  // the row of site nv-1-i for this lane's entry and digit
     const int k = max(nv - 1 - i, 0);
     const int chil = bond[k], chir = k == nv - 1 ? 1 : bond[k + 1];
     const int c = t.vcoord[k];
@@ -433,7 +437,7 @@ eval_chain_few_kernel(const double* __restrict__ data, const int64_t* __restrict
       const uint64_t w = c == 0 ? kw[0] : c == 1 ? kw[1] : c == 2 ? kw[2] : kw[3];
       d = (int)((w >> (t.ndigits[c] - t.vdigit[k])) & 1u);
     }
-    const bool on = l < chil;
+    on = l < chil;
     const double* T = data + off[k] + ((int64_t)(on ? l : 0) * t.sdim[k] + d) * chir;
     if (chir & 1) {
 #pragma unroll
@@ -451,7 +455,7 @@ eval_chain_few_kernel(const double* __restrict__ data, const int64_t* __restrict
   double* v = vec[lane / CHI];
   v[l] = l == 0 ? 1.0 : 0.0;
 #pragma unroll
-  for (int i = 0; i < D; ++i) fetch(i, a[i]);
+  for (int i = 0; i < D; ++i) fetch(i, a[i], has[i]);
   for (int i0 = 0; i0 < nv; i0 += D) {
 #pragma unroll
     for (int j = 0; j < D; ++j) {
@@ -465,8 +469,8 @@ eval_chain_few_kernel(const double* __restrict__ data, const int64_t* __restrict
           s = __builtin_fma(a[j][e + 1], q.y, s);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        v[l] = s;
-        fetch(i0 + j + D, a[j]);
+        v[l] = has[j] ? s : 0.0;
+        fetch(i0 + j + D, a[j], has[j]);
       }
     }
   }
