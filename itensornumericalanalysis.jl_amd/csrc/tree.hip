@@ -68,6 +68,8 @@ struct TreeJob {
   int64_t dstride;   // doubles of one digit slice of P
   int R, n, npad, nt, ngrp;  // rows; output bond, padded; 16-column tiles per workgroup, groups of them
   int m, kbl, nk;    // input legs (the last one padded to kbl blocks of 16), k blocks in all
+  int big;           // trees: the last leg's place among the vertex's own legs (it was exchanged with the
+                     // last of them); -1: a chain (see tree_value)
   int rpw;           // rows per workgroup
   int ldu, ldw;      // LDS row strides of a tile's vectors (last leg, first of two legs); ldu 0: not staged
   int kc, kper;      // chunks of k blocks (one workgroup each) and blocks per chunk
@@ -193,6 +195,39 @@ __device__ __forceinline__ void tree_tile_of(const TreeJob& J, const double* P, 
   else tree_tile<NT, ML, const double*, const f64x2*>(J, P, u, w, lrow, k0, k1, acc);
 }
 
+// One entry of a tree's vertex: row orow, output index n (slice P), k blocks
+// [k0, k1).  A core entry of zero adds nothing whatever the legs hold, and
+// neither does one whose legs, from the last, reach a zero: a sum of functions
+// has zero blocks, and where one term overflows (inf) the other's entries must
+// not become 0 inf = NaN.  A matrix product cannot leave products out, nor the
+// padding of a leg beside an infinite factor, so an entry that comes out as NaN
+// is formed again here.  (A chain's products are all formed, on every route.)
+__device__ __forceinline__ double tree_value(const TreeJob& J, const double* __restrict__ P, int orow, int n, int k0,
+                                             int k1) {
+  double s = 0.0;
+  for (int kb = k0; kb < k1; ++kb) {
+    const int q = kb / J.kbl;
+    const double* Pb = P + ((int64_t)kb * (J.npad >> 4) + (n >> 4)) * 256 + 2 * (n & 15);
+    for (int kk = 0; kk < 16; ++kk) {
+      double w = Pb[((kk >> 1) & 1) * 128 + (kk >> 2) * 32 + (kk & 1)];
+      for (int o = J.m - 1; o >= 0 && w != 0.0; --o) {
+        const int j = o == J.m - 1 ? J.big : o == J.big ? J.m - 1 : o;
+        int i = (kb - q * J.kbl) * 16 + kk;
+        if (j < J.m - 1) {
+          i = q;
+          for (int x = J.m - 2; x > j; --x) i /= J.leg[x].dim;
+          i %= J.leg[j].dim;
+        }
+        const TreeLeg& L = J.leg[j];
+        const int row = L.idx ? L.idx[orow] : (orow >> L.shift) & L.mask;
+        w *= L.u[(int64_t)row * L.stride + i];
+      }
+      s += w;
+    }
+  }
+  return s;
+}
+
 template <int NT>
 __device__ __forceinline__ void tree_rows(const TreeJob& J, const int* rows, int n0, int n1, int ng, int kc, int k0,
                                           int k1, lds_f64* lds) {
@@ -255,13 +290,26 @@ __device__ __forceinline__ void tree_rows(const TreeJob& J, const int* rows, int
     else if (J.m == 1) tree_tile_of<NT, 1>(J, P, u, w, lu, lw, r, k0, k1, acc);
     else if (J.m == 2) tree_tile_of<NT, 2>(J, P, u, w, lu, lw, r, k0, k1, acc);
     else tree_tile_of<NT, 3>(J, P, u, w, lu, lw, r, k0, k1, acc);
+    bool nan = false;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int orow = rows[t * 16 + lk + 4 * e];
       if (orow >= 0) {
 #pragma unroll
-        for (int c = 0; c < NT; ++c)  // (the padding stays zero also for infinite values)
-          out[(int64_t)orow * J.npad + 16 * c + li] = c0 + 16 * c + li < J.n ? acc[c][e] : 0.0;
+        for (int c = 0; c < NT; ++c) {  // (the padding stays zero also for infinite values)
+          const double x = c0 + 16 * c + li < J.n ? acc[c][e] : 0.0;
+          out[(int64_t)orow * J.npad + 16 * c + li] = x;
+          nan |= x != x;
+        }
+      }
+    }
+    if (nan && J.big >= 0) {
+#pragma clang loop unroll(disable)
+      for (int x = 0; x < 4 * NT; ++x) {
+        const int orow = rows[t * 16 + lk + 4 * (x & 3)], c = 16 * (x >> 2) + li;
+        if (orow < 0 || c0 + c >= J.n) continue;
+        double* o = out + (int64_t)orow * J.npad + c;
+        if (*o != *o) *o = tree_value(J, J.P + (t < t0 ? 0 : J.dstride), orow, c0 + c, k0, k1);
       }
     }
   }
@@ -362,10 +410,11 @@ tree_index_kernel(TreeIndexArgs a, const double* __restrict__ xs, int64_t npts, 
 }
 
 // f = <u_a, u_b> over the centre edge, 16 lanes per point (b null: u_a's only
-// entry).  A point with a negative or NaN coordinate gives NaN and the flag.
+// entry).  A point with a negative or NaN coordinate gives NaN and the flag.  On
+// a tree a zero entry adds nothing (see tree_value).
 __global__ void __launch_bounds__(256)
-tree_dot_kernel(TreeLeg a, TreeLeg b, const double* __restrict__ xs, int64_t npts, int nc, double* __restrict__ out,
-                int* __restrict__ flag) {
+tree_dot_kernel(TreeLeg a, TreeLeg b, bool tree, const double* __restrict__ xs, int64_t npts, int nc,
+                double* __restrict__ out, int* __restrict__ flag) {
   const int64_t p = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 4;
   const int li = threadIdx.x & 15;
   if (p >= npts) return;  // whole 16-lane groups
@@ -385,6 +434,13 @@ tree_dot_kernel(TreeLeg a, TreeLeg b, const double* __restrict__ xs, int64_t npt
     s += s1;
 #pragma unroll
     for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (tree && s != s) {  // (the 16 lanes hold the same sum)
+      s = 0.0;
+      for (e = li; e < a.dim; e += 16)
+        if (ua[e] != 0.0 && ub[e] != 0.0) s = __builtin_fma(ua[e], ub[e], s);
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    }
   } else {
     s = ua[0];
   }
@@ -460,6 +516,7 @@ struct VPlan {
   int level = 0;             // longest path of input vertices below
   int n = 1, npad = 16, nt = 1, ngrp = 1;
   int kbl = 1, nk = 1, slices = 1;
+  int big = 0;               // the last input's place before it was exchanged with the last
   int64_t pack = 0;          // offset in the packed copy
   int64_t packT = 0;         // offset in the transposed copy (gradient)
   bool table = false;
@@ -610,6 +667,7 @@ int tree_pack(qtt_ctx* ctx, qtt_net* net) {
       for (size_t i = 0; i < p.in.size(); i++)
         if (edge_dim(net, v, p.in[i]) > edge_dim(net, v, p.in[big])) big = i;
       std::swap(p.in[big], p.in.back());
+      p.big = (int)big;
     }
     for (size_t i = 0; i < p.in.size(); i++) {
       const int w = p.in[i];
@@ -862,6 +920,7 @@ struct Call {
     J.m = (int)p.in.size();
     J.kbl = p.kbl;
     J.nk = p.nk;
+    J.big = t.chain ? -1 : p.big;
     const int c = t.vcoord[v];
     J.out = p.table ? S.d_tab + p.buf : pbuf + p.buf * nrows;
     if (c >= 0) {
@@ -958,7 +1017,8 @@ int launch_eval_tree(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts,
     TreeLeg b;
     std::memset(&b, 0, sizeof(b));
     if (centre >= 0) b = c.point_leg(t.parent[centre], np);
-    tree_dot_kernel<<<(unsigned)((np + 15) / 16), 256, 0, ctx->stream>>>(a, b, x0, np, nc, out + p0, ctx->flags());
+    tree_dot_kernel<<<(unsigned)((np + 15) / 16), 256, 0, ctx->stream>>>(a, b, !t.chain, x0, np, nc, out + p0,
+                                                                   ctx->flags());
     if ((rc = qtt_hip_check(ctx, hipGetLastError(), "tree_dot_kernel"))) return rc;
   }
   // queued only: work on another stream that takes the scratch (or this
@@ -1604,6 +1664,7 @@ int launch_grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double
     J.nt = pw.nt;
     J.ngrp = pw.ngrp;
     J.m = 1;
+    J.big = -1;
     J.kc = 1;
     J.kper = J.nk;
     J.out = out;

@@ -60,3 +60,43 @@ def test_few_points_infinite(q, po, eng, rng, bond, npts):
     xs = rng.uniform(0, 1, (npts, 1))
     xs[:4, 0] = [0.0, 0.25, 0.5, 1.0]
     _same_with_infinities(q.evaluate(f, xs), oracle_eval(po, f, xs))
+
+
+def _tree(q, kind):
+    if kind == "comb":
+        return _comb(q, 3, 5)
+    # one vertex without a digit and four branches: three input legs wherever the tree is cut
+    verts = [(0, 0)] + [(i, j) for i in range(1, 5) for j in range(1, 4)]
+    edges = [((0, 0), (i, 1)) for i in range(1, 5)] + [((i, j), (i, j + 1)) for i in range(1, 5) for j in range(1, 3)]
+    return q.continuous_siteinds(q.NamedGraph(verts, edges), [[(i, j) for j in range(1, 4)] for i in range(1, 5)])
+
+
+@pytest.mark.parametrize("kind", ["comb", "star"])
+@pytest.mark.parametrize("bond,npts", [(3, 1), (5, 40), (16, 300), (20, 3000)])
+def test_tree_infinite(q, po, eng, rng, kind, bond, npts):
+    # bonds that are padded in the matrix products, points as rows and as table
+    # entries; branches that overflow by themselves, beside others that do not
+    if kind == "star":
+        bond = min(bond, 6)
+    f = _overflowing(q, _tree(q, kind), bond, rng, 1e110 if kind == "star" else 1e80)
+    xs = rng.uniform(0, 1, (max(npts, 2), f.dimension()))
+    xs[0], xs[1] = 0.0, 1.0
+    _same_with_infinities(q.evaluate(f, xs), oracle_eval(po, f, xs))
+
+
+@pytest.mark.parametrize("kind", ["comb", "star"])
+@pytest.mark.parametrize("npts", [2, 3000])
+def test_tree_zero_blocks_beside_infinite(q, po, eng, rng, kind, npts):
+    # a sum of two functions has zero blocks: where one of them overflows the sum is
+    # infinite, and with that one's block of the root zero it is the other's value
+    s = _tree(q, kind)
+    f1, f2 = _overflowing(q, s, 3, rng, 1e110 if kind == "star" else 1e80), _overflowing(q, s, 2, rng, 1.0)
+    f = q.builders.add_host(f1, f2)
+    xs = rng.uniform(0, 1, (npts, f.dimension()))
+    xs[0], xs[1] = 0.0, 1.0
+    y1, y2 = oracle_eval(po, f1, xs), oracle_eval(po, f2, xs)
+    _same_with_infinities(q.evaluate(f, xs), y1 + y2)
+    cores = [c.copy() for c in f.cores]
+    cores[0][(slice(None), slice(None)) + (slice(0, 3),) * len(f.topo.children[0])] = 0.0
+    f.set_cores(cores)
+    assert np.max(np.abs(q.evaluate(f, xs) / y2 - 1.0)) < TOL
