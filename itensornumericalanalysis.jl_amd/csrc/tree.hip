@@ -1183,6 +1183,7 @@ struct RunArgs {
   const double* u;
   int stride;
   int n, width;     // sorted positions; doubles per row (16, 32, 48 or 64)
+  int dim;          // entries of u's rows (a row's padding stays zero beside an infinite weight)
   double *S, *head, *tail;
   unsigned char* seen;
 };
@@ -1194,7 +1195,7 @@ template <int G>
 __device__ __forceinline__ void run_group(const RunArgs& a, int grp, int e) {
   const int q0 = grp * RUN, q1 = min(a.n, q0 + RUN);
   if (q0 >= a.n) return;
-  const bool eon = e < a.width;
+  const bool eon = e < a.width, uon = e < a.dim;
   const int before = q0 ? a.rec[q0 - 1].key : -1, after = q1 < a.n ? a.rec[q1].key : -1;
   int cur = a.rec[q0].key;
   bool first = true;  // still in the group's first run
@@ -1218,7 +1219,7 @@ __device__ __forceinline__ void run_group(const RunArgs& a, int grp, int e) {
       const int qq = min(q + i, q1 - 1);
       const SortRec rec = a.rec[qq];
       row[i] = rec.key;
-      x[i] = eon ? rec.w * a.u[(int64_t)rec.r * a.stride + e] : 0.0;
+      x[i] = uon ? rec.w * a.u[(int64_t)rec.r * a.stride + e] : 0.0;
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -1266,7 +1267,7 @@ __global__ void __launch_bounds__(256) run_join_kernel(RunJobs js) {
   if (e < a.width) a.S[(int64_t)row * a.width + e] += s;
 }
 
-// S[p][e] = w[p] u(p)[e] for point rows at the centre
+// S[p][e] = w[p] u(p)[e] for point rows at the centre (zero in the padding)
 __global__ void __launch_bounds__(256)
 point_scale_kernel(const double* __restrict__ w, TreeLeg u, int64_t n, double* __restrict__ S) {
   const int64_t total = n * u.stride;
@@ -1274,7 +1275,7 @@ point_scale_kernel(const double* __restrict__ w, TreeLeg u, int64_t n, double* _
     const int64_t p = i / u.stride;
     const int e = (int)(i - p * u.stride);
     const int r = u.idx ? u.idx[p] : (int)p;
-    S[i] = w[p] * u.u[(int64_t)r * u.stride + e];
+    S[i] = e < u.dim ? w[p] * u.u[(int64_t)r * u.stride + e] : 0.0;
   }
 }
 
@@ -1800,6 +1801,7 @@ int launch_grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double
         a.stride = into[f].stride;
         a.n = (int)np;
         a.width = wd;
+        a.dim = into[f].dim;
         a.S = St + S.vp[c.frontier[f]].buf;
         a.head = head[f];
         a.tail = tail[f];

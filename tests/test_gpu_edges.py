@@ -100,3 +100,22 @@ def test_tree_zero_blocks_beside_infinite(q, po, eng, rng, kind, npts):
     cores[0][(slice(None), slice(None)) + (slice(0, 3),) * len(f.topo.children[0])] = 0.0
     f.set_cores(cores)
     assert np.max(np.abs(q.evaluate(f, xs) / y2 - 1.0)) < TOL
+
+
+@pytest.mark.parametrize("bond,npts", [(1, 3), (5, 4), (5, 3000), (16, 300), (20, 9), (33, 2000)])
+def test_gradient_infinite_weight(q, po, eng, rng, bond, npts):
+    # one sample with an infinite weight: the entries that its digits select are
+    # infinite, all others are the gradient of the other samples
+    L = 11
+    f = _overflowing(q, _chain(q, L, bond), bond, rng, 1.0)
+    f.set_cores([np.abs(c) for c in f.cores])
+    xs, yb = rng.uniform(0, 1, (npts, 1)), rng.uniform(0.5, 1.5, npts)
+    t = f.topo
+    j = npts // 2
+    rest = np.arange(npts) != j
+    ref = po.eval_grad(t.parent, t.sdim, f.cores, t.vcoord, t.vdigit, t.Lc, xs[rest], yb[rest])
+    yb[j] = np.inf
+    for v, (g, r) in enumerate(zip(q.eval_grad(f, xs, yb), ref)):
+        d = int(xs[j, 0] * 2.0 ** t.vdigit[v]) & 1
+        assert np.all(g[:, d] == np.inf)
+        assert rel_l2(g[:, 1 - d], r[:, 1 - d]) < TOL
