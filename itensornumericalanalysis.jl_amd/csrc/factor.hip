@@ -3996,11 +3996,21 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
     if (!conv) {
       if (tid == 0) status[1] = 1;
     }
-    for (int i = tid; i < n; i += bs) {  // by decreasing norm (any order when all are kept)
+    // by decreasing norm (any order when all are kept).  perm indexes rows from
+    // here on, so the ranks are an order in any case: a row whose norm is NaN
+    // (an entry of the network was) comes first, so that it is kept and shows.
+    auto key = [&](int i) {
+      const double s = sig[i];
+      return s == s ? s : HUGE_VAL;
+    };
+    for (int i = tid; i < n; i += bs) {
       int r = 0;
-      const double si = sig[i];
+      const double si = key(i);
       if (!keep_all)
-        for (int j = 0; j < n; ++j) r += (sig[j] > si || (sig[j] == si && j < i)) ? 1 : 0;
+        for (int j = 0; j < n; ++j) {
+          const double sj = key(j);
+          r += (sj > si || (sj == si && j < i)) ? 1 : 0;
+        }
       perm[keep_all ? i : r] = i;
     }
     __syncthreads();

@@ -119,3 +119,30 @@ def test_gradient_infinite_weight(q, po, eng, rng, bond, npts):
         d = int(xs[j, 0] * 2.0 ** t.vdigit[v]) & 1
         assert np.all(g[:, d] == np.inf)
         assert rel_l2(g[:, 1 - d], r[:, 1 - d]) < TOL
+
+
+# ------------------------------------------------------------------ NaN
+@pytest.mark.parametrize("bond,cutoff,maxdim", [(6, 1e-10, 1 << 30), (24, 1e-10, 20), (40, 0.0, 16), (80, 1e-8, 64),
+                                                (110, 0.0, 60)])
+@pytest.mark.parametrize("where", ["first", "middle", "last"])
+def test_truncate_nan(q, eng, rng, bond, cutoff, maxdim, where):
+    # a network with a NaN entry: rows whose norm is NaN still have a place in the
+    # order of the singular values (moves in LDS, on the global workspace, with
+    # helper workgroups); the calls after it are what they were
+    s = _chain(q, 13, bond)
+    good = q.random_itn(s, link_space=bond, rng=rng)
+    op = q.second_derivative_operator(s)
+    def values():
+        g = q.truncate(good, cutoff=cutoff, maxdim=maxdim)
+        return q.evaluate(g, np.linspace(0, 1, 50)[:, None]), g.bonds()
+    before = values()
+    cores = [c.copy() for c in good.cores]
+    v = {"first": 0, "middle": 6, "last": 12}[where]
+    cores[v].reshape(-1)[cores[v].size // 2] = np.nan
+    bad = q.ITensorNetworkFunction(s, cores)
+    for g in (q.truncate(bad, cutoff=cutoff, maxdim=maxdim), q.operate(op, bad, cutoff=cutoff, maxdim=maxdim)):
+        b = g.bonds()
+        assert np.all(b >= 1) and np.all(b <= min(maxdim, 64))
+        assert np.isnan(q.integrate(g))
+    after = values()
+    assert np.array_equal(before[0], after[0]) and np.array_equal(before[1], after[1])
