@@ -1720,6 +1720,13 @@ __device__ __forceinline__ void wy_p3_unit2(double* M, int ldm, int mr, int col0
   }
 }
 
+// LDS of a global-workspace move outside the blocked path: the tiles of the
+// gather (64 x 65) or the turned blocks of the mode product (8 wavefronts x 2).
+// The bonds of a network with some 16,000 vertices leave less: those moves
+// then take the forms that need none.
+constexpr int MOVE_LDS = 8 * 2 * 16 * PLD;
+static_assert(MOVE_LDS >= 64 * 65, "gather_tiles");
+
 constexpr int64_t WY_COOP_MIN = int64_t(1) << 15;  // entries of a row-chunk (two-job) shared update
 constexpr int64_t WY_COLS_MIN = int64_t(1) << 13;  // entries of a column-tile (one-job) shared update
 
@@ -3756,7 +3763,7 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
   int* perm = (int*)(sig + k);                  // k ints (2k doubles reserved)
   double* vbuf = sig + 3 * (int64_t)k;          // 2 rows
   // gather the matrix: M[a*Bx + bb][i] = X[(a*b + i)*Bx + bb] (sizes < 2^31, checked on the host)
-  if (!inplace && gws && bx > 1) {
+  if (!inplace && gws && bx > 1 && pnl_any != nullptr) {
     // tiled transposes, with the helper workgroups when the matrix is large
     if (job != nullptr && nwg > 1 && (int64_t)rows * b >= (int64_t(1) << 15)) {
       if (tid == 0) {
@@ -4091,9 +4098,10 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
       zp = nullptr;
     }
     q_form_tall(Uc, (int)(Au * Bu), (int)nu, (int)nu, uT, gY, Ud, (int)Bu, zs, b, zp, m, pnl_any, job, nwg, iflag);
-  } else if (!REG && gws && job && nwg > 1 && Au * Bu * nu * (int64_t)m >= (int64_t(1) << 22)) {
+  } else if (!REG && gws && job && nwg > 1 && pnl_any != nullptr && Au * Bu * nu * (int64_t)m >= (int64_t(1) << 22)) {
     // a large product in global memory: columns spread over the helper workgroups
-    if (!mode_product_coop(Rrows, perm, use_perm, m, b, Uc, gY, Ud, (int)Au, (int)nu, (int)Bu, job, nwg, iflag, pnl,
+    // (also of moves outside the blocked path: pnl is null there)
+    if (!mode_product_coop(Rrows, perm, use_perm, m, b, Uc, gY, Ud, (int)Au, (int)nu, (int)Bu, job, nwg, iflag, pnl_any,
                            prec)) {
       if (tid == 0) status[1] = 1;
     }
@@ -4111,8 +4119,10 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
         mode_product_mfma32(Rrows, perm, use_perm, m, b, Uc, gY, (int)nu, (int)Bu, 0, (int)(Au * Bu));
       else if (prec == QTT_F32_SPLIT)
         mode_product<QTT_F32_SPLIT>(Rrows, perm, use_perm, m, b, Uc, gY, (int)Au, (int)nu, (int)Bu);
-      else
+      else if (pnl_any != nullptr)
         mode_product_mfma(Rrows, perm, use_perm, m, b, Uc, gY, (int)nu, (int)Bu, 0, (int)(Au * Bu), pnl_any);
+      else
+        mode_product<QTT_F64>(Rrows, perm, use_perm, m, b, Uc, gY, (int)Au, (int)nu, (int)Bu);
     } else {
       if (prec == QTT_F32) mode_product<QTT_F32>(Rrows, perm, use_perm, m, b, Uc, gY, (int)Au, (int)nu, (int)Bu);
       else if (prec == QTT_F32_SPLIT)
@@ -4189,7 +4199,8 @@ __global__ void __launch_bounds__(512) truncate_kernel(const SweepArgs* __restri
   double* wsl = lds + 64 + nvi;
   // LDS of the blocked QR's panels and WY updates (TALL_LDS doubles), 16-byte aligned
   const int poff = (64 + nvi + 1) & ~1;
-  lds_f64* pnl_any = (lds_f64*)(lds + poff);
+  // (null where the bonds leave less than MOVE_LDS)
+  lds_f64* pnl_any = poff + MOVE_LDS <= QTT_LDS_DOUBLES ? (lds_f64*)(lds + poff) : nullptr;
   for (int v = tid; v < t.nv; v += bs) {
     bond[v] = a.bond_g[v];
     kq[v] = -1;

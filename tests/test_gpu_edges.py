@@ -146,3 +146,30 @@ def test_truncate_nan(q, eng, rng, bond, cutoff, maxdim, where):
         assert np.isnan(q.integrate(g))
     after = values()
     assert np.array_equal(before[0], after[0]) and np.array_equal(before[1], after[1])
+
+
+# ------------------------------------------------------------------ very many vertices
+@pytest.mark.parametrize("extra,bond,maxdim", [(1300, 128, 128), (17000, 48, 20), (19500, 24, 10)])
+def test_truncate_very_many_vertices(q, po, eng, rng, extra, bond, maxdim):
+    # the vertices' bonds take the LDS that moves beyond it use otherwise: no room
+    # for the blocked path (with a product that helper workgroups share), then none
+    # for the tiles of a gather either
+    nd = 16
+    g = q.named_grid((extra + nd, 1))
+    f0 = [(extra + i, 1) for i in range(1, nd + 1)]
+    s = q.continuous_siteinds(g, [f0])
+    cap = [1] * (extra + 1) + [min(bond, 2 ** min(j, nd - j)) for j in range(1, nd)] + [1]
+    cores = [np.ones((1, 1, 1)) for _ in range(extra)]
+    for j in range(nd):
+        a, b = cap[extra + j], cap[extra + j + 1]
+        shape = (a, 2, b) if j + 1 < nd else (a, 2)
+        cores.append(rng.standard_normal(shape) * (0.8 ** np.arange(a)).reshape((-1,) + (1,) * (len(shape) - 1)))
+    f = q.ITensorNetworkFunction(s, cores)
+    t = f.topo
+    for cutoff in (0.0, 1e-10):
+        got = q.truncate(f, cutoff=cutoff, maxdim=maxdim)
+        ref, err = po.truncate(t.parent, t.sdim, f.cores, cutoff, maxdim)
+        assert np.array_equal(got.bonds(), [c.shape[0] for c in ref])
+        xs = rng.uniform(0, 1, (200, 1))
+        yr = po.evaluate(t.parent, t.sdim, ref, t.vcoord, t.vdigit, t.Lc, xs)[0]
+        assert rel_l2(q.evaluate(got, xs), yr) < 1e-10
