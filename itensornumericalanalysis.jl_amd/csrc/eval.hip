@@ -61,6 +61,10 @@ __global__ void pack_chain_kernel(const double* __restrict__ data, const int64_t
   }
 }
 
+// RAW: the cores as they lie (pack and poff are then the network's data and
+// offsets), for calls that may not make the packed copy; the same sums in the
+// same order.
+template <bool RAW>
 __global__ void __launch_bounds__(256)
 eval_chain_f64_kernel(const double* __restrict__ pack, const int64_t* __restrict__ poff,
                       const int* __restrict__ bond, TopoView t, const double* __restrict__ xs,
@@ -90,18 +94,30 @@ eval_chain_f64_kernel(const double* __restrict__ pack, const int64_t* __restrict
     }
     const uint64_t dmask = 0 - (uint64_t)d;
     const double* __restrict__ P = pack + poff[k];
-    const int lpad = (chil + 3) & ~3;
+    const int lpad = (chil + 3) & ~3, sd = t.sdim[k];
     for (int l0 = 0; l0 < chil; l0 += 4) {
       double a0[4] = {0.0, 0.0, 0.0, 0.0}, a1[4] = {0.0, 0.0, 0.0, 0.0};
-      const double* __restrict__ q = P + 2 * l0;
-      for (int r = 0; r < chir; ++r) {
-        const double vr = v[(size_t)r * bs];
+      if constexpr (RAW) {
+        for (int r = 0; r < chir; ++r) {
+          const double vr = v[(size_t)r * bs];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          a0[i] = __builtin_fma(q[2 * i], vr, a0[i]);
-          a1[i] = __builtin_fma(q[2 * i + 1], vr, a1[i]);
+          for (int i = 0; i < 4; ++i) {
+            const double* __restrict__ T = P + (int64_t)min(l0 + i, chil - 1) * sd * chir + r;
+            a0[i] = __builtin_fma(T[0], vr, a0[i]);
+            a1[i] = __builtin_fma(T[sd > 1 ? chir : 0], vr, a1[i]);
+          }
         }
-        q += 2 * lpad;
+      } else {
+        const double* __restrict__ q = P + 2 * l0;
+        for (int r = 0; r < chir; ++r) {
+          const double vr = v[(size_t)r * bs];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            a0[i] = __builtin_fma(q[2 * i], vr, a0[i]);
+            a1[i] = __builtin_fma(q[2 * i + 1], vr, a1[i]);
+          }
+          q += 2 * lpad;
+        }
       }
       double sel[4];
 #pragma unroll
@@ -1122,7 +1138,11 @@ int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, doub
   // of 40 sites of bond 15: 1530 us in float-float, 135 us in float64).
   if (precision != QTT_F64 && !(t.chain && t.ncoord <= QTT_MAX_COORD))
     return qtt_fail(ctx, QTT_EINVAL, "evaluate: float32 paths are implemented for chains only");
-  // a stream that is being captured takes only kernels that need no scratch
+  // A stream that is being captured takes only kernels that need no scratch, and
+  // nothing is made for the network there: an allocation or a copy from the host
+  // breaks the capture, and a packed copy or a table that is only recorded would
+  // pass for made until the first replay.  Without the packed copy the kernels that
+  // read the cores run, without the tables those that need none.
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   (void)hipStreamIsCapturing(ctx->stream, &cap);
   const bool capturing = cap != hipStreamCaptureStatusNone;
@@ -1134,8 +1154,11 @@ int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, doub
     // cannot take, stay refused.)
     if (maxb > 32 && maxb <= 160 && !ctx->force_lds_eval && !capturing)
       return launch_eval_tree(ctx, net, xs, npts, out);
-    if (maxb <= 32 && npts <= few_points(maxb) && !ctx->force_lds_eval && !ctx->eval_ppl &&
-        ctx->eval_tbits < 0 && !ctx->eval_tuned.count(eval_tune_key(maxb, npts))) {
+    const bool raw = capturing && !net->pack_valid;
+    if (maxb <= 32 && !ctx->force_lds_eval &&
+        (raw || (npts <= few_points(maxb) && !ctx->eval_ppl && ctx->eval_tbits < 0 &&
+                 !ctx->eval_tuned.count(eval_tune_key(maxb, npts))))) {
+      if (npts > (int64_t(1) << 31)) return qtt_fail(ctx, QTT_EINVAL, "evaluate: too many points");
 #define QTT_FEW_LAUNCH(C)                                                                                     \
   eval_chain_few_kernel<C><<<dim3((unsigned)((npts + 64 / C - 1) / (64 / C))), 64, 0, ctx->stream>>>(         \
       net->d_data, net->d_off, net->d_bond, tv, xs, npts, out, ctx->flags())
@@ -1145,7 +1168,7 @@ int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, doub
 #undef QTT_FEW_LAUNCH
       return qtt_hip_check(ctx, hipGetLastError(), "eval_chain_few_kernel");
     }
-    int rc = ensure_pack(ctx, net);
+    int rc = raw ? QTT_OK : ensure_pack(ctx, net);
     if (rc) return rc;
     if (maxb <= 32 && !ctx->force_lds_eval) {
       // tuned shape if qtt_tune_eval measured one for this bond class and point
@@ -1161,6 +1184,7 @@ int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, doub
       }
       if (ctx->eval_ppl) ppl = ctx->eval_ppl;
       if (ctx->eval_tbits >= 0) tb = ctx->eval_tbits;
+      if (capturing && !(net->env_valid && net->env_tb == tb)) tb = 0;
       return launch_eval_env(ctx, net, xs, npts, out, maxb, ppl, wg, tb);
     }
     // LDS: two vectors of maxb entries per lane
@@ -1173,12 +1197,17 @@ int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, doub
     if (nb > INT32_MAX) return qtt_fail(ctx, QTT_EINVAL, "evaluate: too many points");
     const size_t lds = per_lane * bs;
     if (lds > 64 * 1024) {
-      rc = qtt_hip_check(ctx, hipFuncSetAttribute((const void*)eval_chain_f64_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+      const void* fn = raw ? (const void*)eval_chain_f64_kernel<true> : (const void*)eval_chain_f64_kernel<false>;
+      rc = qtt_hip_check(ctx, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
                          "evaluate LDS attribute");
       if (rc) return rc;
     }
-    eval_chain_f64_kernel<<<dim3((unsigned)nb), bs, lds, ctx->stream>>>(
-        net->d_pack, net->d_pack_off, net->d_bond, tv, xs, npts, out, ctx->flags(), (int)maxb);
+    if (raw)
+      eval_chain_f64_kernel<true><<<dim3((unsigned)nb), bs, lds, ctx->stream>>>(
+          net->d_data, net->d_off, net->d_bond, tv, xs, npts, out, ctx->flags(), (int)maxb);
+    else
+      eval_chain_f64_kernel<false><<<dim3((unsigned)nb), bs, lds, ctx->stream>>>(
+          net->d_pack, net->d_pack_off, net->d_bond, tv, xs, npts, out, ctx->flags(), (int)maxb);
     return qtt_hip_check(ctx, hipGetLastError(), "eval_chain kernel");
   }
   if (capturing) return qtt_fail(ctx, QTT_EHIP, "evaluate: a tree cannot be evaluated on a captured stream");
@@ -1592,12 +1621,12 @@ int launch_eval_noalloc(qtt_ctx* ctx, const qtt_net* net, const double* xs, int6
   if (nb > INT32_MAX) return qtt_fail(ctx, QTT_EINVAL, "evaluate: too many points");
   const size_t lds = per_lane * bs;
   if (lds > 64 * 1024) {
-    rc = qtt_hip_check(ctx, hipFuncSetAttribute((const void*)eval_chain_f64_kernel,
+    rc = qtt_hip_check(ctx, hipFuncSetAttribute((const void*)eval_chain_f64_kernel<false>,
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
                        "evaluate LDS attribute");
     if (rc) return rc;
   }
-  eval_chain_f64_kernel<<<dim3((unsigned)nb), bs, lds, ctx->stream>>>(pack, poff, net->d_bond, tv, xs, npts, out,
-                                                                      ctx->flags(), (int)maxb);
+  eval_chain_f64_kernel<false><<<dim3((unsigned)nb), bs, lds, ctx->stream>>>(pack, poff, net->d_bond, tv, xs, npts,
+                                                                             out, ctx->flags(), (int)maxb);
   return qtt_hip_check(ctx, hipGetLastError(), "eval_chain_f64_kernel");
 }

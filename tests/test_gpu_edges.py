@@ -173,3 +173,61 @@ def test_truncate_very_many_vertices(q, po, eng, rng, extra, bond, maxdim):
         xs = rng.uniform(0, 1, (200, 1))
         yr = po.evaluate(t.parent, t.sdim, ref, t.vcoord, t.vdigit, t.Lc, xs)[0]
         assert rel_l2(q.evaluate(got, xs), yr) < 1e-10
+
+
+# ------------------------------------------------------------------ captured streams
+@pytest.mark.parametrize("bond,npts,warm", [(5, 20000, 0), (5, 20000, 3), (16, 20000, 3), (16, 20000, 20000),
+                                            (16, 40000, 3), (16, 40000, 40000), (31, 13000, 1), (32, 5, 0),
+                                            (33, 700, 0), (33, 700, 700), (96, 300, 5), (160, 65, 65)])
+def test_evaluate_captured(q, po, eng, rng, bond, npts, warm):
+    # a captured evaluate, the network fresh or used with `warm` points before: the
+    # capture makes nothing for the network, replays give the values of eager calls,
+    # and so do the eager calls before the first replay
+    import torch
+    L = 30 if bond <= 32 else 12
+    s = _chain(q, L, bond)
+    f = q.random_itn(s, link_space=bond, rng=rng, std=1.0 / math.sqrt(bond))
+    xs = rng.uniform(0, 1, (npts, 1))
+    xd = torch.tensor(xs, device="cuda")
+    out = torch.zeros(npts, dtype=torch.float64, device="cuda")
+    if warm:
+        q.evaluate(f, xd[:warm].contiguous())
+    else:
+        q.api.device_network(f)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        q.evaluate(f, xd, out=out)
+    y = q.evaluate(f, xd)
+    eng.sync()
+    assert rel_l2(y.cpu().numpy(), oracle_eval(po, f, xs)) < TOL
+    for r in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(out.cpu().numpy(), y.cpu().numpy()) < TOL
+        assert torch.equal(q.evaluate(f, xd), y)
+        xd.copy_(torch.flip(xd, (0,)))  # other points in the same buffer
+        y = q.evaluate(f, xd)
+        eng.sync()
+
+
+def test_evaluate_tree_captured_refused(q, po, eng, rng):
+    # a tree needs its plan made: refused on a captured stream, without harm to the
+    # calls after it
+    import torch
+    f = q.random_itn(_comb(q, 3, 4), link_space=5, rng=rng)
+    xs = rng.uniform(0, 1, (50, 3))
+    xd = torch.tensor(xs, device="cuda")
+    q.evaluate(f, xd)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    other = torch.zeros(8, device="cuda")
+    with torch.cuda.graph(graph):
+        other += 1.0
+        with pytest.raises(q.api._capi.EngineError):
+            q.evaluate(f, xd)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert float(other.sum()) == 8.0
+    assert rel_l2(q.evaluate(f, xd).cpu().numpy(), oracle_eval(po, f, xs)) < TOL
