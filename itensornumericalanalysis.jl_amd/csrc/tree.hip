@@ -14,8 +14,9 @@
 // vectors, one per digit string, however many points there are: below a limit
 // its rows are the digit strings (a table), and points that share digits share
 // the work.  The tables depend only on the cores, so they are kept with the
-// network, like its packed chain copy, until the cores change.  Above the limit
-// the rows are the points.  A table's row index has the vertex's own digit as
+// network, like its packed chain copy, until the cores change; they lie by
+// number of digits, so a call that wants fewer finds its own among more, and one
+// that wants more builds what is missing.  Above the limit the rows are the points.  A table's row index has the vertex's own digit as
 // its top bit, then its input tables' indices.
 //
 // The product.  Rows of one digit use one slice of the core, so a workgroup
@@ -40,6 +41,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <new>
 
 namespace {
 
@@ -303,7 +305,7 @@ __device__ __forceinline__ void tree_rows(const TreeJob& J, const int* rows, int
         }
       }
     }
-    if (nan && J.big >= 0) {
+    if (__builtin_expect(J.big >= 0 && nan, 0)) {
 #pragma clang loop unroll(disable)
       for (int x = 0; x < 4 * NT; ++x) {
         const int orow = rows[t * 16 + lk + 4 * (x & 3)], c = 16 * (x >> 2) + li;
@@ -519,7 +521,9 @@ struct VPlan {
   int big = 0;               // the last input's place before it was exchanged with the last
   int64_t pack = 0;          // offset in the packed copy
   int64_t packT = 0;         // offset in the transposed copy (gradient)
-  bool table = false;
+  bool fits = false;         // its rows can be digit strings (they and its inputs' are few enough)
+  int64_t tab = 0;           // then: offset in the table buffer
+  bool table = false;        // this call's choice
   int64_t buf = 0;           // offset in the table buffer / point buffers (per row for points)
 };
 
@@ -584,8 +588,13 @@ struct TreeState {
   int64_t packT_cap = 0;
   double* d_tab = nullptr;   // vectors of every table vertex
   int64_t tab_cap = 0;
-  int tab_digits = -1;       // largest table's digits in the buffer (-1: none built)
+  int tab_digits = 0;        // tables of fewer digits than this are built
+  // what was queued last to make any of the above: ev follows it on ev_stream
+  hipEvent_t ev = nullptr;
+  hipStream_t ev_stream = nullptr;
+  bool making = false;       // something was queued since
   ~TreeState() {
+    if (ev) (void)hipEventDestroy(ev);
     if (d_pack) (void)hipFree(d_pack);
     if (d_packT) (void)hipFree(d_packT);
     if (d_tab) (void)hipFree(d_tab);
@@ -597,8 +606,38 @@ void tree_state_stale(TreeState* s) {
   if (s) {
     s->packed = false;
     s->packedT = false;
-    s->tab_digits = -1;
+    s->tab_digits = 0;
   }
+}
+
+// A network's packed cores and tables may be used from any stream (and through
+// another context) right after the call that queued them: a call on another
+// stream waits on the device for what was made last.  Nothing built is written
+// again while it is valid, so uses need no such mark.
+static int tree_enter(qtt_ctx* ctx, qtt_net* net) {
+  if (!net->tree && !(net->tree = new (std::nothrow) TreeState)) return qtt_fail(ctx, QTT_ENOMEM, "host allocation");
+  TreeState& S = *net->tree;
+  if (!S.ev_stream || S.ev_stream == ctx->stream) return QTT_OK;
+  if (hipEventQuery(S.ev) == hipSuccess) {
+    S.ev_stream = nullptr;
+    return QTT_OK;
+  }
+  (void)hipGetLastError();  // not ready
+  return qtt_hip_check(ctx, hipStreamWaitEvent(ctx->stream, S.ev, 0), "tree event");
+}
+
+// after a call's work is queued, also when it failed on the way
+static int tree_leave(qtt_ctx* ctx, qtt_net* net) {
+  TreeState& S = *net->tree;
+  if (!S.making) return QTT_OK;
+  int rc = QTT_OK;
+  if (!S.ev) rc = qtt_hip_check(ctx, hipEventCreateWithFlags(&S.ev, hipEventDisableTiming), "tree event");
+  if (!rc) rc = qtt_hip_check(ctx, hipEventRecord(S.ev, ctx->stream), "tree event");
+  if (!rc) {
+    S.ev_stream = ctx->stream;
+    S.making = false;
+  }
+  return rc;
 }
 
 namespace {
@@ -623,11 +662,10 @@ int64_t site_stride(const qtt_net* net, int v) {
 
 // Orientation, shapes and the packed copy (once per network state).
 int tree_pack(qtt_ctx* ctx, qtt_net* net) {
-  if (!net->tree) net->tree = new TreeState;
   TreeState& S = *net->tree;
   if (S.packed) return QTT_OK;
   const HostTopo& t = net->t;
-  S.tab_digits = -1;
+  S.tab_digits = 0;
   S.centre = choose_centre(net);
   S.vp.assign(t.nv, VPlan());
   S.order.clear();
@@ -682,7 +720,18 @@ int tree_pack(qtt_ctx* ctx, qtt_net* net) {
     p.slices = t.vcoord[v] >= 0 ? 2 : 1;
     p.pack = tot;
     tot += (int64_t)p.slices * p.nk * p.npad * 16;
+    p.fits = p.nd <= TREE_BITS && (int64_t(p.npad) << p.nd) <= (int64_t(1) << 21);
+    for (int w : p.in) p.fits = p.fits && S.vp[w].fits;
   }
+  int64_t tabs = 0;
+  for (int nd = 0; nd <= TREE_BITS; nd++)
+    for (int v : S.order) {
+      VPlan& p = S.vp[v];
+      if (!p.fits || p.nd != nd) continue;
+      p.tab = tabs;
+      tabs += int64_t(p.npad) << nd;
+    }
+  S.making = true;
   if (S.pack_cap < tot) {
     if (S.d_pack) (void)hipFree(S.d_pack);
     S.d_pack = nullptr;
@@ -845,7 +894,8 @@ struct Call {
 
   // Tables: a vertex with nd digits behind it is a table when 2^nd <= npts / 2
   // (its rows then cost at most half of a row per point, also on a call that
-  // builds them), nd <= 16 and the table holds at most 2^21 doubles.  copies:
+  // builds them), nd <= 16 and the table holds at most 2^21 doubles (the choice
+  // does not depend on what is built already, so neither do the values).  copies:
   // buffers per point vertex (the chunk of points keeps them near 512 MiB).
   int plan(int copies) {
     const HostTopo& t = net->t;
@@ -855,12 +905,11 @@ struct Call {
     front_of.assign(t.nv, -1);
     for (int v : S.order) {
       VPlan& p = S.vp[v];
-      p.table = p.nd <= limit && (int64_t(p.npad) << p.nd) <= (int64_t(1) << 21);
-      for (int w : p.in) p.table = p.table && S.vp[w].table;
+      p.table = p.fits && p.nd <= limit;
       if (p.table) {
-        p.buf = tabs;
-        tabs += int64_t(p.npad) << p.nd;
-        digits = std::max(digits, p.nd + 1);  // of the largest table: names the set of tables
+        p.buf = p.tab;
+        tabs += int64_t(p.npad) << p.nd;  // (the tables of at most this many digits lie in front)
+        digits = std::max(digits, p.nd + 1);
       } else {
         any_point = true;
         p.buf = per;
@@ -880,7 +929,7 @@ struct Call {
       if (S.d_tab) (void)hipFree(S.d_tab);
       S.d_tab = nullptr;
       S.tab_cap = 0;
-      S.tab_digits = -1;
+      S.tab_digits = 0;
       const int rc = qtt_hip_check(ctx, hipMalloc(&S.d_tab, tabs * sizeof(double)), "hipMalloc tree tables");
       if (rc) return rc;
       S.tab_cap = tabs;
@@ -949,12 +998,13 @@ struct Call {
     if (p.table) return {S.d_tab + p.buf, idx + front_of[v] * chunk, p.npad, p.n, 0, 0};
     return {pbuf + p.buf * nrows, nullptr, p.npad, p.n, 0, -1};
   }
-  int forward(bool table, int64_t nrows, const double* x0) {
+  // the vertices whose rows are points, or tables of at least `from` digits
+  int forward(bool table, int from, int64_t nrows, const double* x0) {
     Level lv(ctx, part, kpart);
     for (int l = 0; l <= most_level; l++) {
       for (int v : S.order) {
         const VPlan& p = S.vp[v];
-        if (p.level != l || p.table != table) continue;
+        if (p.level != l || p.table != table || p.nd < from) continue;
         TreeJob J = make_job(v, nrows, x0);
         const int r = lv.add(p, J);
         if (r) return r;
@@ -964,9 +1014,10 @@ struct Call {
     }
     return QTT_OK;
   }
-  int tables() {  // once per network state and set of tables
-    if (S.tab_digits == digits || digits == 0) return QTT_OK;
-    const int rc = forward(true, 0, nullptr);
+  int tables() {  // once per network state
+    if (S.tab_digits >= digits) return QTT_OK;
+    S.making = true;
+    const int rc = forward(true, S.tab_digits, 0, nullptr);
     if (!rc) S.tab_digits = digits;
     return rc;
   }
@@ -997,7 +1048,7 @@ struct Call {
 
 }  // namespace
 
-int launch_eval_tree(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, double* out) {
+static int eval_tree(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, double* out) {
   const HostTopo& t = net->t;
   int rc = tree_pack(ctx, net);
   if (rc) return rc;
@@ -1012,7 +1063,7 @@ int launch_eval_tree(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts,
     const int64_t np = std::min(c.chunk, npts - p0);
     const double* x0 = xs + p0 * nc;
     if ((rc = c.index(np, x0))) return rc;
-    if (c.any_point && (rc = c.forward(false, np, x0))) return rc;
+    if (c.any_point && (rc = c.forward(false, 0, np, x0))) return rc;
     const TreeLeg a = c.point_leg(centre < 0 ? 0 : centre, np);
     TreeLeg b;
     std::memset(&b, 0, sizeof(b));
@@ -1021,9 +1072,17 @@ int launch_eval_tree(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts,
                                                                    ctx->flags());
     if ((rc = qtt_hip_check(ctx, hipGetLastError(), "tree_dot_kernel"))) return rc;
   }
-  // queued only: work on another stream that takes the scratch (or this
-  // network's tables, through this function) waits for it
-  return qtt_scratch_queued(ctx);
+  return QTT_OK;
+}
+
+int launch_eval_tree(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, double* out) {
+  int rc = tree_enter(ctx, net);
+  if (rc) return rc;
+  rc = eval_tree(ctx, net, xs, npts, out);
+  // queued only: work on another stream that takes the scratch, or what was made
+  // for the network, waits for it
+  const int rl = tree_leave(ctx, net), rq = qtt_scratch_queued(ctx);
+  return rc ? rc : rl ? rl : rq;
 }
 
 // ---------------------------------------------------------------------------
@@ -1441,6 +1500,7 @@ __global__ void __launch_bounds__(256) tree_core_sum_kernel(CoreSums js) {
 int tree_pack_transposed(qtt_ctx* ctx, qtt_net* net) {
   TreeState& S = *net->tree;
   if (S.packedT) return QTT_OK;
+  S.making = true;
   int64_t tot = 0;
   for (int v : S.order) {
     VPlan& p = S.vp[v];
@@ -1496,7 +1556,7 @@ int tree_pack_transposed(qtt_ctx* ctx, qtt_net* net) {
 
 }  // namespace
 
-int launch_grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double* ybar, int64_t npts, double* grad) {
+static int grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double* ybar, int64_t npts, double* grad) {
   const HostTopo& t = net->t;
   if (npts == 0) {
     grad_zero_kernel<<<256, 256, 0, ctx->stream>>>(grad, qtt_net_size(net), nullptr, 0);
@@ -1716,7 +1776,7 @@ int launch_grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double
     grad_weight_kernel<<<nb, 256, 0, ctx->stream>>>(x0, ybar + p0, np, nc, wts, ctx->flags());
     if ((rc = qtt_hip_check(ctx, hipGetLastError(), "grad_weight_kernel"))) return rc;
     if ((rc = c.index(np, x0))) return rc;
-    if (c.any_point && (rc = c.forward(false, np, x0))) return rc;
+    if (c.any_point && (rc = c.forward(false, 0, np, x0))) return rc;
     // the values that reach each table, by point
     std::vector<TreeLeg> into(nf);
     std::vector<const double*> wof(nf, nullptr);
@@ -1841,4 +1901,15 @@ int launch_grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double
   }
   if ((rc = cores_of(true, 0, nullptr, false))) return rc;
   return qtt_hip_check(ctx, hipStreamSynchronize(ctx->stream), "grad sync");
+}
+
+int launch_grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double* ybar, int64_t npts, double* grad) {
+  int rc = tree_enter(ctx, net);
+  if (rc) return rc;
+  rc = grad_chain(ctx, net, xs, ybar, npts, grad);
+  const int rl = tree_leave(ctx, net);
+  if (!rc) return rl;
+  const int rq = qtt_scratch_queued(ctx);  // it may have failed with work queued
+  (void)rq;
+  return rc;
 }

@@ -231,3 +231,93 @@ def test_evaluate_tree_captured_refused(q, po, eng, rng):
     torch.cuda.synchronize()
     assert float(other.sum()) == 8.0
     assert rel_l2(q.evaluate(f, xd).cpu().numpy(), oracle_eval(po, f, xs)) < TOL
+
+
+# ------------------------------------------------------------------ calls of changing size, streams, contexts
+@pytest.mark.parametrize("kind", ["wide", "comb"])
+def test_tables_serve_other_sizes(q, po, eng, rng, kind):
+    # point counts up and down on one network, evaluate and gradient: the same bits as
+    # a fresh network's first call of that size
+    s = _chain(q, 18, 40) if kind == "wide" else _comb(q, 3, 9)
+    f = q.random_itn(s, link_space=40 if kind == "wide" else 9, rng=rng, std=0.3)
+    xs = rng.uniform(0, 1, (70000, f.dimension()))
+    yb = rng.standard_normal(70000)
+    def fresh():
+        return q.ITensorNetworkFunction(s, f.cores)
+    for n in (300, 70000, 1, 9, 70000, 2000, 300):
+        assert np.array_equal(q.evaluate(f, xs[:n]), q.evaluate(fresh(), xs[:n]))
+        if kind == "wide" and n in (300, 2000):
+            g = q.eval_grad(f, xs[:n], yb[:n])
+            assert all(np.array_equal(a, b) for a, b in zip(g, q.eval_grad(fresh(), xs[:n], yb[:n])))
+    assert rel_l2(q.evaluate(f, xs[:500]), oracle_eval(po, f, xs[:500])) < TOL
+    # and after the cores changed
+    h = q.truncate(f, cutoff=0.0, maxdim=6)
+    for n in (2000, 10, 2000):
+        assert rel_l2(q.evaluate(h, xs[:n]), oracle_eval(po, h, xs[:n])) < TOL
+
+
+@pytest.mark.parametrize("kind", ["wide", "comb"])
+def test_tree_evaluate_on_streams(q, po, eng, rng, kind):
+    # one network used on two streams and through a second context, nothing waited for
+    # in between: what the first call makes is there for the second, and the scratch
+    # that both use is taken in turn
+    import ctypes
+    import torch
+    s = _chain(q, 20, 40) if kind == "wide" else _comb(q, 3, 10)
+    bond = 150 if kind == "wide" else 40
+    n = 30000
+    xs = rng.uniform(0, 1, (n, 1 if kind == "wide" else 3))
+    xd = torch.tensor(xs, device="cuda")
+    other = q.api._capi.Context(0)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    for rep in range(3):
+        f = q.random_itn(s, link_space=bond, rng=rng, std=1.0 / math.sqrt(bond))
+        g = q.random_itn(s, link_space=bond, rng=rng, std=1.0 / math.sqrt(bond))
+        dn = q.api.device_network(f)
+        q.api.device_network(g)
+        out = [torch.zeros(n, dtype=torch.float64, device="cuda") for _ in range(4)]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
+            q.evaluate(f, xd, out=out[0])
+        with torch.cuda.stream(b):
+            q.evaluate(f, xd, out=out[1])
+            q.evaluate(g, xd, out=out[2])
+        other.check(q.api._capi.lib().qtt_eval(other.handle, dn.handle, ctypes.c_void_p(xd.data_ptr()), n,
+                                               ctypes.c_void_p(out[3].data_ptr()), 0))
+        other.sync()
+        torch.cuda.synchronize()
+        yf, yg = oracle_eval(po, f, xs[:300]), oracle_eval(po, g, xs[:300])
+        assert rel_l2(out[0][:300].cpu().numpy(), yf) < TOL
+        assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[3])
+        assert rel_l2(out[2][:300].cpu().numpy(), yg) < TOL
+    other.close()
+
+
+# ------------------------------------------------------------------ more points than one pass takes
+@pytest.mark.parametrize("nc", [1, 3])
+def test_evaluate_in_passes(q, po, eng, rng, nc):
+    # more point rows than the scratch holds at once: 40 sites of bond 160 are some
+    # 2200 doubles per point beyond the tables, so a pass takes 30 thousand points; the
+    # backbone of a comb of bond 64 is 192, 350 thousand points
+    s = _chain(q, 40, 160) if nc == 1 else _comb(q, 3, 14)
+    f = q.random_itn(s, link_space=160 if nc == 1 else 64, rng=rng, std=0.1)
+    n = 45007 if nc == 1 else 400003
+    xs = rng.uniform(0, 1, (n, nc))
+    y = q.evaluate(f, xs)
+    sel = np.concatenate([np.arange(0, n, n // 200), [n - 1]])
+    assert rel_l2(y[sel], oracle_eval(po, f, np.ascontiguousarray(xs[sel]))) < TOL
+
+
+@pytest.mark.parametrize("bond,L,n", [(53, 50, 30011), (20, 60, 60001)])
+def test_gradient_in_passes(q, po, eng, rng, bond, L, n):
+    # several passes of points add into the cores' gradient: against the sum of the
+    # gradients of pieces that one pass takes
+    f = q.random_itn(_chain(q, L, bond), link_space=bond, rng=rng, std=1.0 / math.sqrt(bond))
+    xs, yb = rng.uniform(0, 1, (n, 1)), rng.standard_normal(n)
+    g = q.eval_grad(f, xs, yb)
+    parts = [q.eval_grad(f, xs[i:i + 5000], yb[i:i + 5000]) for i in range(0, n, 5000)]
+    for v, a in enumerate(g):
+        assert rel_l2(a, sum(p[v] for p in parts)) < TOL
+    t = f.topo
+    ref = po.eval_grad(t.parent, t.sdim, f.cores, t.vcoord, t.vdigit, t.Lc, xs[:300], yb[:300])
+    assert all(rel_l2(a, b) < TOL for a, b in zip(q.eval_grad(f, xs[:300], yb[:300]), ref))
