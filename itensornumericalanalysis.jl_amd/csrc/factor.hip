@@ -935,8 +935,18 @@ __device__ inline int rr_player(int pos, int t, int nn) {
 // Jacobi runs again with the rule off (cutoff 0, rotations continued in J),
 // which rotates only the unconverged pairs of the block.  A cutoff outside
 // (0, 1) rotates every pair.
+//   The rule ends after JACOBI_NOISE_SWEEPS sweeps: rows just above the level
+// converge only linearly against rows below it that are not orthogonal to each
+// other, as slowly as their norms are close.  (Matrices with most singular values
+// within a factor of 3 of the level: of 12 x 24 ones 1 in 20 was not done in 60
+// sweeps, of 110 x 140 ones all; with the rule ended after 12 sweeps they take 13
+// to 21.  Most matrices that converge under the rule take 5 to 12.)
+constexpr int JACOBI_NOISE_SWEEPS = 12;
 __device__ inline double noise_level(double fro2, double cut, int n) {
   return (cut > 0.0 && cut < 1.0) ? cut * fro2 / (double)n : 0.0;
+}
+__device__ __forceinline__ double noise_at(double noise, int sweep) {
+  return sweep < JACOBI_NOISE_SWEEPS ? noise : 0.0;
 }
 
 // true if the noise block of the rows with norms sig[0..n) cannot change the
@@ -997,8 +1007,9 @@ __device__ bool jacobi_rows(double* X, int n, int b, double* J, int* flag, doubl
   for (int64_t e = tid; e < (int64_t)n * b; e += bs) fro += X[e] * X[e];
   const double fsum = block_sum(fro, red);
   const double small = fsum * DBL_EPSILON * DBL_EPSILON;
-  const double noise = noise_level(fsum, cut, n);
+  const double level = noise_level(fsum, cut, n);
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
+    const double noise = noise_at(level, sweep);
     if (tid == 0) *flag = 0;
     __syncthreads();
     for (int t = 0; t < nn - 1; ++t) {
@@ -1184,10 +1195,11 @@ __device__ __noinline__ bool jacobi_rows_reg(F* X, int ldx_in, int n_in, int b_i
   }
   const double fsum = block_sum(fro, red);
   const double small = fsum * DBL_EPSILON * DBL_EPSILON;
-  const double noise = noise_level(fsum, cut, n);
+  const double level = noise_level(fsum, cut, n);
   const double stop2 = jacobi_stop2(tol);
   QTT_JT_INIT;
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
+    const double noise = noise_at(level, sweep);
     if (tid == 0) *flag = 0;
     __syncthreads();
     QTT_JC(6);
@@ -1297,13 +1309,14 @@ __device__ __noinline__ bool jacobi_wave(lds_f64* X, int ldx_in, int n_in, int b
   }
   const double fsum = block_sum(fro, red);
   const double small = fsum * DBL_EPSILON * DBL_EPSILON;
-  const double noise = noise_level(fsum, cut, n);
+  const double level = noise_level(fsum, cut, n);
   const double stop2 = jacobi_stop2(tol);
   if (tid < 64) {
     const int pi = tid / G;
     const bool player = pi < nn / 2;
     int sweeps = max_sweeps, conv = 0;
     for (int sweep = 0; sweep < max_sweeps; ++sweep) {
+    const double noise = noise_at(level, sweep);
       int rot = 0;
       for (int t = 0; t < nn - 1; ++t) {
         int p = rr_player(pi, t, nn), q = rr_player(nn - 1 - pi, t, nn);
@@ -3518,7 +3531,7 @@ __device__ bool jacobi_coop(double* X, int n, int b, double* J, CoopJob* job, in
   for (int e2 = tid; e2 < n * b; e2 += bs) fro += X[e2] * X[e2];
   const double fsum = block_sum(fro, red);
   const double small = fsum * DBL_EPSILON * DBL_EPSILON;
-  const double noise = noise_level(fsum, cut, n);
+  const double level = noise_level(fsum, cut, n);
   const int len = b > n ? b : n;
   const int e = len <= 128 ? 2 : len <= 256 ? 4 : len <= 384 ? 6 : 8;
   lds_i32* sflag = (lds_i32*)iflag;
@@ -3547,6 +3560,7 @@ __device__ bool jacobi_coop(double* X, int n, int b, double* J, CoopJob* job, in
   if (blocked)
     for (int b2 = tid; b2 < nblk; b2 += bs) job->ver[b2] = 0;  // published by the first post
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
+    const double noise = noise_at(level, sweep);
     if (tid == 0) __hip_atomic_store(&job->rot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int t = 0; t < (blocked ? 1 : rounds); ++t) {
       if (tid == 0) {

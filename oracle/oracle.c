@@ -560,7 +560,10 @@ int or_qr(int r, int c, const double* M, double* Q, double* R) {
  * mutually orthogonal.  svd_factor then checks whether the noise block can
  * change what the truncation keeps (see noise_block_exact) and, if it can,
  * calls this again with cut = 0 and init_j = 0 to finish the SVD.  Any other
- * cut rotates every pair.  init_j = 0 continues from the rotations in J. */
+ * cut rotates every pair.  init_j = 0 continues from the rotations in J.
+ * The rule ends after NOISE_SWEEPS sweeps: rows just above the level converge
+ * only linearly against rows below it that are not orthogonal to each other. */
+#define NOISE_SWEEPS 12
 static int jacobi_rows(int n, int c, double* X, double* J, double cut, int init_j) {
   if (init_j)
     for (int i = 0; i < n; i++)
@@ -574,8 +577,9 @@ static int jacobi_rows(int n, int c, double* X, double* J, double cut, int init_
   double fro = 0.0;
   for (long e = 0; e < (long)n * c; e++) fro += X[e] * X[e];
   const double small = fro * DBL_EPSILON * DBL_EPSILON;
-  const double noise = (cut > 0.0 && cut < 1.0) ? cut * fro / (double)n : 0.0;
+  const double level = (cut > 0.0 && cut < 1.0) ? cut * fro / (double)n : 0.0;
   for (int sweep = 0; sweep < 100; sweep++) {
+    const double noise = sweep < NOISE_SWEEPS ? level : 0.0;
     int rot = 0;
     for (int p = 0; p < n - 1; p++)
       for (int q = p + 1; q < n; q++) {

@@ -321,3 +321,46 @@ def test_gradient_in_passes(q, po, eng, rng, bond, L, n):
     t = f.topo
     ref = po.eval_grad(t.parent, t.sdim, f.cores, t.vcoord, t.vdigit, t.Lc, xs[:300], yb[:300])
     assert all(rel_l2(a, b) < TOL for a, b in zip(q.eval_grad(f, xs[:300], yb[:300]), ref))
+
+
+# ------------------------------------------------------------------ singular values around the cutoff's level
+def _level_matrix(n, b, cut, seed):
+    """n x b with singular values 1, two between, and the others within a factor of
+    some 3 of the level below which rows are not rotated against each other."""
+    rng = np.random.default_rng(seed)
+    k = min(n, b)
+    lev = np.sqrt(cut / k)
+    S = np.concatenate([[1.0], 0.1 ** rng.uniform(0.3, 3, 2), lev * np.exp(rng.uniform(np.log(0.2), np.log(3), k - 3))])
+    U = np.linalg.qr(rng.standard_normal((n, k)))[0]
+    V = np.linalg.qr(rng.standard_normal((b, k)))[0]
+    return (U * S) @ V.T, S
+
+
+# (moves of one wavefront, in LDS, preconditioned, tall, on the global workspace,
+# with helper workgroups; seeds that do not converge while the rule holds)
+@pytest.mark.parametrize("n,b,seed", [(12, 24, 25), (12, 24, 31), (20, 40, 2), (20, 40, 19), (32, 64, 4), (32, 64, 17),
+                                      (34, 30, 18), (64, 96, 0), (64, 96, 9), (110, 140, 0), (150, 260, 0),
+                                      (200, 260, 1)])
+def test_truncate_values_at_noise_level(q, po, eng, n, b, seed):
+    import ctypes
+    from types import SimpleNamespace
+    cut = 1e-8
+    M, S = _level_matrix(n, b, cut, seed)
+    topo = SimpleNamespace(nv=2, parent=np.array([-1, 0]), sdim=np.array([b, n]), vcoord=np.array([-1, -1]),
+                           vdigit=np.array([0, 0]), Lc=np.zeros(0), ncoord=0,
+                           core_shape=lambda v, bond: (1, b, int(bond[1])) if v == 0 else (int(bond[1]), n))
+    cores = [np.eye(b).reshape(1, b, b), np.ascontiguousarray(M.T)]
+    capi = q.api._capi
+    net = capi.DeviceNetwork.upload(eng, topo, cores)
+    err = ctypes.c_double()
+    eng.check(capi.lib().qtt_truncate(eng.handle, net.handle, cut, 1 << 40, ctypes.byref(err)))
+    c0, c1 = net.download()
+    s2 = np.sort(S ** 2)
+    drop = int(np.sum(np.cumsum(s2) <= cut * s2.sum()))
+    assert c1.shape[0] == len(S) - drop
+    lost = s2[:drop].sum()
+    assert abs(err.value - lost / s2.sum()) <= 1e-6 * lost / s2.sum()
+    assert abs(np.sum((c0[0] @ c1 - M.T) ** 2) - lost) <= 1e-6 * lost
+    # the oracle as well
+    ref, e = po.truncate(topo.parent, topo.sdim, cores, cut, 1 << 40)
+    assert ref[1].shape[0] == c1.shape[0] and abs(e - err.value) <= 1e-6 * err.value
