@@ -957,15 +957,35 @@ static EnvPlan env_plan(const qtt_net* net, int tb) {
   return p;
 }
 
-// Digit sites per table when nothing is tuned: 12, from 2^15 points (below,
-// values are bit for bit those of the batch kernels, which take no tables).  Two
-// tables of 2^12 rows stay in an XCD's L2 and are built in one short launch;
-// larger ones save two sites per digit (20 us per site at 10^6 points of bond 16)
-// but their rows come from beyond the L2.  10^6 points, 40 sites of bond 16,
-// repeated / first call: 10 digits 408 / 541 us, 12 digits 337 / 468, 14 digits
-// 403 / 561, 16 digits 296 / 751, 18 digits 171 / 760.  (qtt_tune_eval weighs
-// the repeated calls alone.)
-static int default_table_bits(int64_t npts) { return npts < (int64_t(1) << 15) ? 0 : 12; }
+// Digit sites per table when nothing is tuned: none below 2^15 points (values are
+// bit for bit those of the batch kernels there, which take no tables); from there
+// as many as leave a row reused about 32 times, at least 12, and at most what the
+// L2 of an XCD holds beside the rest (two tables of some 2 MB: 12 digits up to bond
+// 32, 13 up to bond 20, 16 up to bond 8, whose small rows cost little from beyond it
+// too).  From 2^21 points 16 digits, their middle sites saved being worth more than
+// the L2.  A network's first call allocates and builds the tables too.  us per call,
+// 40 sites, 12 / 13 / 14 / 15 / 16 digits, called back to back on the same points
+// (with other points each time 10^6 points of bond 16 take longer, 383 against 337
+// with 12 digits):
+//             10^6 points                      2 10^6 (bonds 4, 16, 32: 2^21)
+//   bond 4    47 / 43 / 41 / 45 / 43           79 / 75 / 71 / 67 / 67
+//   bond 8    108 / 98 / 89 / 86 / 80          195 / 178 / 162 / 152 / 138
+//   bond 12   211 / 186 / 223 / 222 / 167      407 / 365 / 412 / 427 / 306
+//   bond 16   337 / 309 / 401 / 363 / 297      667 / 596 / 782 / 721 / 587
+//   bond 20   692 / 617 / 880 / 847 / 723      1279 / 1137 / 1760 / 1584 / 1325
+//   bond 32   1676 / 2348 / 2355 / 2036 / 1662 3347 / 4986 / 4452 / 3750 / 3057
+// 10^7 points of bond 16: 2967 / 2644 / 3492 / 3133 / 2556.  A new network's first
+// call, 10^6 points of bond 16: 530 / 488 / 548 / - / 463; of bond 20: 980 / 884 /
+// 1109 / - / 930.  (16 digits are the fastest in many places, but every network keeps
+// its tables: 17 MB at bond 16 where 13 digits are 2.  qtt_tune_eval chooses among
+// all sizes for a program that repeats a call.)
+static int default_table_bits(int64_t npts, int64_t maxb) {
+  if (npts < (int64_t(1) << 15)) return 0;
+  int lg = 15;
+  while (lg < 21 && (int64_t(1) << (lg + 1)) <= npts) ++lg;
+  if (lg == 21) return 16;
+  return std::max(12, std::min(lg - 5, maxb <= 8 ? 16 : maxb <= 20 ? 13 : 12));
+}
 
 static EnvTableArgs env_table_args(const qtt_net* net, const EnvPlan& pl, bool left, double* tab) {
   const HostTopo& t = net->t;
@@ -1175,7 +1195,7 @@ int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, doub
       // count; else two points per lane for bonds <= 16 (register room) when
       // there are enough points to fill the GPU at half the workgroup count
       int ppl = maxb <= 16 && npts >= (int64_t(1) << 19) ? 2 : 1, wg = 256;
-      int tb = default_table_bits(npts);
+      int tb = default_table_bits(npts, maxb);
       const auto it = ctx->eval_tuned.find(eval_tune_key(maxb, npts));
       if (it != ctx->eval_tuned.end()) {
         ppl = it->second.ppl;

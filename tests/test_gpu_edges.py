@@ -364,3 +364,17 @@ def test_truncate_values_at_noise_level(q, po, eng, n, b, seed):
     # the oracle as well
     ref, e = po.truncate(topo.parent, topo.sdim, cores, cut, 1 << 40)
     assert ref[1].shape[0] == c1.shape[0] and abs(e - err.value) <= 1e-6 * err.value
+
+
+# ------------------------------------------------------------------ table sizes of large calls
+@pytest.mark.parametrize("bond,n", [(11, (1 << 21) - 1), (11, 1 << 21), (9, (1 << 21) + 333), (8, 1 << 18),
+                                    (3, (1 << 19) - 1), (8, 1 << 20), (7, 1 << 21), (20, 1 << 18), (21, 1 << 18)])
+def test_evaluate_table_sizes(q, po, eng, rng, bond, n):
+    # the default table size changes with the points; larger and smaller calls in turn
+    import torch
+    f = q.random_itn(_chain(q, 17, bond, dims=2), link_space=bond, rng=rng, std=1.0 / math.sqrt(bond))
+    xd = torch.rand(n, 2, dtype=torch.float64, device="cuda")
+    for m in (n, 40000, n):
+        y = q.evaluate(f, xd[:m]).cpu().numpy()
+        sel = np.concatenate([np.arange(0, m, m // 500), [m - 1]])
+        assert rel_l2(y[sel], oracle_eval(po, f, xd.cpu().numpy()[sel])) < TOL
