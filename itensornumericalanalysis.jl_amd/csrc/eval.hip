@@ -1140,11 +1140,27 @@ int tune_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, double
 
 // Points up to which CHI lanes per point (eval_chain_few_kernel) beat one: the
 // lane-per-point kernel takes the same time for 1 to 30,000 points, the other
-// grows with them.  Measured us, few against one lane per point: bond 5, 12
-// sites 9.0 / 13.5 at 1 point, 11.6 / 14.2 at 16,384; bond 8, 28 sites 16 / 38
-// and 35 / 38; bond 16, 40 sites 27 / 189 at 1, 84 / 197 at 8,192, 190 / 190 at
-// 16,384; bond 32, 24 sites 24 / 398, 91 / 405 at 4,096, 401 / 400 at 16,384.
-static int64_t few_points(int64_t maxb) { return maxb <= 8 ? 16384 : 12288; }
+// grows with them.  Measured us, few against one lane per point:
+//   bond  sites   1 point       8,192         12,288        16,384
+//   4     12      7.9 / 6.9     8.9 / 7.5     10 / 7.4      10 / 7.4
+//   4     40      20 / 19       22 / 20       24 / 20       25 / 20
+//   5     6       6.1 / 7.3     6.8 / 7.8     7.3 / 7.8     7.8 / 7.6
+//   5     40      23 / 44       25 / 46       28 / 45       30 / 44
+//   8     6       5.5 / 8.5     7.3 / 9.1     8.4 / 9.1     9.5 / 8.9
+//   8     12      8.4 / 17      12 / 18       14 / 18       17 / 17
+//   8     28      16 / 38       24 / 40       30 / 39       36 / 38
+//   12    40      25 / 110      40 / 114      51 / 114
+//   16    12      10 / 53       27 / 56       36 / 55
+//   16    40      26 / 189      84 / 198      117 / 196     190 / 190
+//   20    24      23 / 166      66 / 172      88 / 171
+//   32    24      24 / 397      185 / 408     253 / 406     401 / 400
+// Up to bond 4 it is never the faster one (half of its lanes hold no entry), but
+// it needs no packed copy: it takes a network's first such call there (8 us where
+// making the copy adds some 40), and the calls after it pack.
+static int64_t few_points(const qtt_net* net, int64_t maxb) {
+  if (maxb <= 4) return net->pack_valid || net->few_seen ? 0 : 12288;
+  return maxb <= 8 && net->t.nv >= 8 ? 16384 : 12288;
+}
 
 int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, double* out,
                 int precision) {
@@ -1176,9 +1192,10 @@ int launch_eval(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, doub
       return launch_eval_tree(ctx, net, xs, npts, out);
     const bool raw = capturing && !net->pack_valid;
     if (maxb <= 32 && !ctx->force_lds_eval &&
-        (raw || (npts <= few_points(maxb) && !ctx->eval_ppl && ctx->eval_tbits < 0 &&
+        (raw || (npts <= few_points(net, maxb) && !ctx->eval_ppl && ctx->eval_tbits < 0 &&
                  !ctx->eval_tuned.count(eval_tune_key(maxb, npts))))) {
       if (npts > (int64_t(1) << 31)) return qtt_fail(ctx, QTT_EINVAL, "evaluate: too many points");
+      if (!capturing) net->few_seen = true;
 #define QTT_FEW_LAUNCH(C)                                                                                     \
   eval_chain_few_kernel<C><<<dim3((unsigned)((npts + 64 / C - 1) / (64 / C))), 64, 0, ctx->stream>>>(         \
       net->d_data, net->d_off, net->d_bond, tv, xs, npts, out, ctx->flags())

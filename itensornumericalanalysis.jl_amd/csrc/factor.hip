@@ -4716,6 +4716,7 @@ int truncate_batch_finish(qtt_ctx* ctx, TruncStaged& st, qtt_net* const* nets, d
   for (int i = 0; i < st.nnet; i++) {
     for (int v = 0; v < nets[i]->t.nv; v++) nets[i]->bond[v] = *bonds++;
     nets[i]->pack_valid = false;
+    nets[i]->few_seen = false;
     nets[i]->pack32_valid = false;
     nets[i]->env_valid = false;
     tree_state_stale(nets[i]->tree);

@@ -110,6 +110,7 @@ struct qtt_net {
   std::vector<int64_t> h_pack_off;  // host sources of the pack offsets / descriptors
   std::vector<int> h_desc;
   bool pack_valid = false;
+  bool few_seen = false;  // evaluated without the packed copy since the cores changed (few_points)
   // float32 copies for the mixed-precision evaluate
   float* d_pack32 = nullptr;
   bool pack32_valid = false;

@@ -378,3 +378,18 @@ def test_evaluate_table_sizes(q, po, eng, rng, bond, n):
         y = q.evaluate(f, xd[:m]).cpu().numpy()
         sel = np.concatenate([np.arange(0, m, m // 500), [m - 1]])
         assert rel_l2(y[sel], oracle_eval(po, f, xd.cpu().numpy()[sel])) < TOL
+
+
+@pytest.mark.parametrize("bond,npts", [(1, 1), (2, 50), (3, 12288), (4, 12289), (4, 7)])
+def test_few_points_small_bonds_repeated(q, po, eng, rng, bond, npts):
+    # up to bond 4 a network's first call of few points reads the cores, the next ones
+    # the packed copy: the same bits, also after the cores changed
+    f = q.random_itn(_chain(q, 12, bond), link_space=bond, rng=rng)
+    xs = rng.uniform(0, 1, (npts, 1))
+    y = q.evaluate(f, xs)
+    assert rel_l2(y, oracle_eval(po, f, xs)) < TOL
+    assert all(np.array_equal(q.evaluate(f, xs), y) for _ in range(3))
+    g = q.truncate(f, cutoff=0.0, maxdim=max(1, bond - 1))
+    z = q.evaluate(g, xs)
+    assert rel_l2(z, oracle_eval(po, g, xs)) < TOL
+    assert np.array_equal(q.evaluate(g, xs), z)
