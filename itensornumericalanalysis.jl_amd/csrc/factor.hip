@@ -939,9 +939,10 @@ __device__ inline int rr_player(int pos, int t, int nn) {
 // converge only linearly against rows below it that are not orthogonal to each
 // other, as slowly as their norms are close.  (Matrices with most singular values
 // within a factor of 3 of the level: of 12 x 24 ones 1 in 20 was not done in 60
-// sweeps, of 110 x 140 ones all; with the rule ended after 12 sweeps they take 13
-// to 21.  Most matrices that converge under the rule take 5 to 12.)
-constexpr int JACOBI_NOISE_SWEEPS = 12;
+// sweeps, of 110 x 140 ones all; with the rule ended after 20 sweeps they take 22
+// to 29.)  Not earlier: a graded matrix that converges under the rule takes up to
+// 15 or so, and rotating its smallest rows against each other, some 8 sweeps more.
+constexpr int JACOBI_NOISE_SWEEPS = 20;
 __device__ inline double noise_level(double fro2, double cut, int n) {
   return (cut > 0.0 && cut < 1.0) ? cut * fro2 / (double)n : 0.0;
 }
