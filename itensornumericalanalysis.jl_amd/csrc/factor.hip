@@ -4286,15 +4286,24 @@ __global__ void __launch_bounds__(512) truncate_kernel(const SweepArgs* __restri
     int pnl_cap = 0;  // doubles of LDS at pnl
     int pmode = 0;
     // The blocked path also takes matrices that would fit LDS where it is the
-    // faster one (float64 products only): more than 256 rows or columns (the LDS
-    // kernels then give a wavefront per column or row pair: a 32 x 285 QR move 950 ->
-    // 270 us, a 32 x 285 SVD move 1300 -> 480), QR moves from 48 x 48 (64 x 80 114 ->
-    // 109 us, 160 x 80 180 -> 122: Q is kept as reflectors and u is an MFMA product),
-    // and wide SVD moves from 24 rows (24 x 80: 212 and 304 -> 234 and 239 us with 7
-    // and 10 sweeps; 20 x 80: 160 -> 208).
-    const bool blocked = TALL_LDS + 64 <= a.ws_lds &&
-                         (need > a.ws_lds || (a.prec == QTT_F64 && (!small || (tr ? rows <= b && rows >= 24 && b >= 48
-                                                                                  : rows >= 48 && b >= 48))));
+    // faster one (float64 products only):
+    //  - more than 256 rows or columns, where the LDS kernels give a wavefront per
+    //    column or row pair.  Tall from 16 columns: a QR move of 300 x 16 121 -> 54
+    //    us, 600 x 16 214 -> 64, but 300 x 4 18 -> 51, 600 x 12 73 -> 63, 1000 x 12
+    //    106 -> 131; SVD moves of 600 x 16 314 -> 217, 300 x 12 117 -> 147, 600 x 8 84
+    //    -> 142 (a vertex with four branches of bond 10: the whole truncation 1.51 ->
+    //    2.16 ms).  Wide from 4 rows (32 x 285 950 -> 270 us, 4 x 300 87 -> 71, 2 x 300
+    //    49 -> 70), SVD moves always (2 x 300 130 -> 108, 32 x 285 1300 -> 480);
+    //  - QR moves from 48 x 48 (64 x 80 114 -> 109 us, 160 x 80 180 -> 122: Q is kept as
+    //    reflectors and u is an MFMA product);
+    //  - wide SVD moves from 24 rows.  By itself a move of 24 x 80 takes 212 and 304
+    //    us with 7 and 10 sweeps in LDS, 234 and 239 here, one of 20 x 80 160 -> 208; the
+    //    truncation of a chain of bond 48 takes 3.71 ms with the line at 24 rows, 3.96
+    //    at 32, 5.80 at 40.
+    const bool faster = !small ? (rows > b ? b >= 16 : tr || rows >= 4)
+                        : tr   ? rows <= b && rows >= 24 && b >= 48
+                               : rows >= 48 && b >= 48;
+    const bool blocked = TALL_LDS + 64 <= a.ws_lds && (need > a.ws_lds || (a.prec == QTT_F64 && faster));
     if (blocked) pmode = (int64_t)rows * PLD <= 8 * TALL_REGION ? 1 : 3;
     if (pmode) {
       pnl = pnl_any;
