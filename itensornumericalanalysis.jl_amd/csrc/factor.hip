@@ -935,19 +935,16 @@ __device__ inline int rr_player(int pos, int t, int nn) {
 // Jacobi runs again with the rule off (cutoff 0, rotations continued in J),
 // which rotates only the unconverged pairs of the block.  A cutoff outside
 // (0, 1) rotates every pair.
-//   The rule ends after JACOBI_NOISE_SWEEPS sweeps: rows just above the level
-// converge only linearly against rows below it that are not orthogonal to each
-// other, as slowly as their norms are close.  (Matrices with most singular values
-// within a factor of 3 of the level: of 12 x 24 ones 1 in 20 was not done in 60
-// sweeps, of 110 x 140 ones all; with the rule ended after 20 sweeps they take 22
-// to 29.)  Not earlier: a graded matrix that converges under the rule takes up to
-// 15 or so, and rotating its smallest rows against each other, some 8 sweeps more.
+//   The rule is given JACOBI_NOISE_SWEEPS sweeps, then it is off as well: rows just
+// above the level converge only linearly against rows below it that are not
+// orthogonal to each other, as slowly as their norms are close.  (Matrices with
+// most singular values within a factor of 3 of the level: of 12 x 24 ones 1 in 20
+// was not done in 60 sweeps, of 110 x 140 ones all; they then take some 8 sweeps
+// more.)  Not fewer: a graded matrix that converges under the rule takes up to 15 or
+// so, and rotating its smallest rows against each other, 8 more.
 constexpr int JACOBI_NOISE_SWEEPS = 20;
 __device__ inline double noise_level(double fro2, double cut, int n) {
   return (cut > 0.0 && cut < 1.0) ? cut * fro2 / (double)n : 0.0;
-}
-__device__ __forceinline__ double noise_at(double noise, int sweep) {
-  return sweep < JACOBI_NOISE_SWEEPS ? noise : 0.0;
 }
 
 // true if the noise block of the rows with norms sig[0..n) cannot change the
@@ -1008,9 +1005,8 @@ __device__ bool jacobi_rows(double* X, int n, int b, double* J, int* flag, doubl
   for (int64_t e = tid; e < (int64_t)n * b; e += bs) fro += X[e] * X[e];
   const double fsum = block_sum(fro, red);
   const double small = fsum * DBL_EPSILON * DBL_EPSILON;
-  const double level = noise_level(fsum, cut, n);
+  const double noise = noise_level(fsum, cut, n);
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
-    const double noise = noise_at(level, sweep);
     if (tid == 0) *flag = 0;
     __syncthreads();
     for (int t = 0; t < nn - 1; ++t) {
@@ -1196,11 +1192,10 @@ __device__ __noinline__ bool jacobi_rows_reg(F* X, int ldx_in, int n_in, int b_i
   }
   const double fsum = block_sum(fro, red);
   const double small = fsum * DBL_EPSILON * DBL_EPSILON;
-  const double level = noise_level(fsum, cut, n);
+  const double noise = noise_level(fsum, cut, n);
   const double stop2 = jacobi_stop2(tol);
   QTT_JT_INIT;
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
-    const double noise = noise_at(level, sweep);
     if (tid == 0) *flag = 0;
     __syncthreads();
     QTT_JC(6);
@@ -1310,14 +1305,13 @@ __device__ __noinline__ bool jacobi_wave(lds_f64* X, int ldx_in, int n_in, int b
   }
   const double fsum = block_sum(fro, red);
   const double small = fsum * DBL_EPSILON * DBL_EPSILON;
-  const double level = noise_level(fsum, cut, n);
+  const double noise = noise_level(fsum, cut, n);
   const double stop2 = jacobi_stop2(tol);
   if (tid < 64) {
     const int pi = tid / G;
     const bool player = pi < nn / 2;
     int sweeps = max_sweeps, conv = 0;
     for (int sweep = 0; sweep < max_sweeps; ++sweep) {
-    const double noise = noise_at(level, sweep);
       int rot = 0;
       for (int t = 0; t < nn - 1; ++t) {
         int p = rr_player(pi, t, nn), q = rr_player(nn - 1 - pi, t, nn);
@@ -3532,7 +3526,7 @@ __device__ bool jacobi_coop(double* X, int n, int b, double* J, CoopJob* job, in
   for (int e2 = tid; e2 < n * b; e2 += bs) fro += X[e2] * X[e2];
   const double fsum = block_sum(fro, red);
   const double small = fsum * DBL_EPSILON * DBL_EPSILON;
-  const double level = noise_level(fsum, cut, n);
+  const double noise = noise_level(fsum, cut, n);
   const int len = b > n ? b : n;
   const int e = len <= 128 ? 2 : len <= 256 ? 4 : len <= 384 ? 6 : 8;
   lds_i32* sflag = (lds_i32*)iflag;
@@ -3561,7 +3555,6 @@ __device__ bool jacobi_coop(double* X, int n, int b, double* J, CoopJob* job, in
   if (blocked)
     for (int b2 = tid; b2 < nblk; b2 += bs) job->ver[b2] = 0;  // published by the first post
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
-    const double noise = noise_at(level, sweep);
     if (tid == 0) __hip_atomic_store(&job->rot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int t = 0; t < (blocked ? 1 : rounds); ++t) {
       if (tid == 0) {
@@ -3905,7 +3898,7 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
     // lanes per row pair sized so a row is at most 4 entries per lane.
     // cut: pairs of rows below its noise level are left alone; init_j: start
     // J from the identity (else continue the rotations already in it)
-    auto jacobi = [&](const double cut, const bool init_j) -> bool {
+    auto jacobi = [&](const double cut, const bool init_j, const int max_sweeps) -> bool {
       bool cv;
       if (REG && G == 8 && jwave) {
         // small matrices: the single-wavefront rounds on a zero-padded copy
@@ -4002,16 +3995,19 @@ __device__ __forceinline__ int run_move(double* ws, const bool gws, CoopJob* job
         for (int e = tid; e < n * n; e += bs) Jb[e] = (e / n == e - (e / n) * n) ? 1.0 : 0.0;
       __syncthreads();
     }
+    const bool rule = cutoff > 0.0 && cutoff < 1.0;
+    const int sweeps = rule ? min(max_sweeps, JACOBI_NOISE_SWEEPS) : max_sweeps;
     bool conv = keep_all ? true
                 : precond ? jacobi_precond(X, n, b, Rb, Jb, tau, vbuf, vbuf + ((int64_t)n + PNB) * PNB, gY, sig, perm,
-                                           pnl, pnl_cap, job, nwg, red, iflag, cutoff, max_sweeps)
-                          : jacobi(cutoff, true);
+                                           pnl, pnl_cap, job, nwg, red, iflag, cutoff, sweeps)
+                          : jacobi(cutoff, true, sweeps);
     row_norms<G>(X, n, b, sig);
     __syncthreads();
-    if (conv && cutoff > 0.0 && cutoff < 1.0 && !noise_block_exact(sig, n, cutoff, iflag + 10)) {
-      // the noise block could change what is kept: finish the SVD among its
-      // rows (pairs with a row above the level are converged and skipped)
-      conv = jacobi(0.0, false);
+    if (rule && (conv ? !noise_block_exact(sig, n, cutoff, iflag + 10) : max_sweeps > sweeps)) {
+      // the noise block could change what is kept, or the rows above it do not
+      // converge beside it: finish the SVD among its rows too (pairs that are
+      // converged are skipped)
+      conv = jacobi(0.0, false, conv ? max_sweeps : max_sweeps - sweeps);
       row_norms<G>(X, n, b, sig);
       __syncthreads();
     }
@@ -4288,7 +4284,7 @@ __global__ void __launch_bounds__(512) truncate_kernel(const SweepArgs* __restri
     // The blocked path also takes matrices that would fit LDS where it is the
     // faster one (float64 products only):
     //  - more than 256 rows or columns, where the LDS kernels give a wavefront per
-    //    column or row pair.  Tall from 16 columns: a QR move of 300 x 16 121 -> 54
+    //    column or row pair, unless `thin` below.  Tall from 16 columns: a QR move of 300 x 16 121 -> 54
     //    us, 600 x 16 214 -> 64, but 300 x 4 18 -> 51, 600 x 12 73 -> 63, 1000 x 12
     //    106 -> 131; SVD moves of 600 x 16 314 -> 217, 300 x 12 117 -> 147, 600 x 8 84
     //    -> 142 (a vertex with four branches of bond 10: the whole truncation 1.51 ->
@@ -4300,10 +4296,9 @@ __global__ void __launch_bounds__(512) truncate_kernel(const SweepArgs* __restri
     //    us with 7 and 10 sweeps in LDS, 234 and 239 here, one of 20 x 80 160 -> 208; the
     //    truncation of a chain of bond 48 takes 3.71 ms with the line at 24 rows, 3.96
     //    at 32, 5.80 at 40.
-    const bool faster = !small ? (rows > b ? b >= 16 : tr || rows >= 4)
-                        : tr   ? rows <= b && rows >= 24 && b >= 48
-                               : rows >= 48 && b >= 48;
-    const bool blocked = TALL_LDS + 64 <= a.ws_lds && (need > a.ws_lds || (a.prec == QTT_F64 && faster));
+    const bool blocked = TALL_LDS + 64 <= a.ws_lds &&
+                         (need > a.ws_lds || (a.prec == QTT_F64 && (!small || (tr ? rows <= b && rows >= 24 && b >= 48
+                                                                                  : rows >= 48 && b >= 48))));
     if (blocked) pmode = (int64_t)rows * PLD <= 8 * TALL_REGION ? 1 : 3;
     if (pmode) {
       pnl = pnl_any;
@@ -4332,7 +4327,14 @@ __global__ void __launch_bounds__(512) truncate_kernel(const SweepArgs* __restri
         m = run_move_plain(&a, (lds_f64*)lds, (lds_f64*)wsl, rows, b, tr, (int)Bx, (int)Au, (int)nu, (int)Bu, x, u, lazyT, uT,
                            pnl_any);
     } else {
-      if (small)
+      // (the few columns or rows that the line above leaves to LDS are told apart
+      // here: in the condition they cost every small move 0.3 us)
+      const bool thin = !small && need <= a.ws_lds && (rows > b ? b < 16 : !tr && rows < 4);
+      if (thin) {
+        lazyT = nullptr;
+        m = run_move_plain(&a, (lds_f64*)lds, (lds_f64*)wsl, rows, b, tr, (int)Bx, (int)Au, (int)nu, (int)Bu, x, u, lazyT, uT,
+                           pnl_any);
+      } else if (small)
         m = run_move_global<8>(&a, (lds_f64*)lds, pnl, pnl_cap, pmode, rows, b, tr, (int)Bx, (int)Au, (int)nu, (int)Bu, x,
                                u, lazyT, uT, pnl_any);
       else

@@ -393,3 +393,31 @@ def test_few_points_small_bonds_repeated(q, po, eng, rng, bond, npts):
     z = q.evaluate(g, xs)
     assert rel_l2(z, oracle_eval(po, g, xs)) < TOL
     assert np.array_equal(q.evaluate(g, xs), z)
+
+
+# ------------------------------------------------------------------ tall and wide moves of few columns or rows
+@pytest.mark.parametrize("s0,b,s1", [(257, 1, 3), (300, 4, 5), (257, 15, 40), (257, 16, 40), (1000, 12, 12), (3, 300, 7),
+                                     (4, 300, 300), (15, 15, 300), (16, 16, 300), (17, 17, 900), (300, 300, 2),
+                                     (260, 260, 3), (700, 20, 600)])
+@pytest.mark.parametrize("maxdim", [1 << 40, 3])
+def test_truncate_thin_moves(q, eng, rng, s0, b, s1, maxdim):
+    # two vertices, so that the moves' matrices are s0 x b (QR) and s1 x min(s0, b)
+    # (SVD): around the lines at 256 rows and at 16 columns or 4 rows
+    import ctypes
+    from types import SimpleNamespace
+    topo = SimpleNamespace(nv=2, parent=np.array([-1, 0]), sdim=np.array([s0, s1]), vcoord=np.array([-1, -1]),
+                           vdigit=np.array([0, 0]), Lc=np.zeros(0), ncoord=0,
+                           core_shape=lambda v, bond: (1, s0, int(bond[1])) if v == 0 else (int(bond[1]), s1))
+    a, c = rng.standard_normal((s0, b)) * 0.8 ** np.arange(b), rng.standard_normal((b, s1))
+    capi = q.api._capi
+    net = capi.DeviceNetwork.upload(eng, topo, [a.reshape(1, s0, b), c])
+    err = ctypes.c_double()
+    eng.check(capi.lib().qtt_truncate(eng.handle, net.handle, 0.0, maxdim, ctypes.byref(err)))
+    c0, c1 = net.download()
+    m = min(s0, b, s1, maxdim)
+    assert c1.shape[0] == m
+    M = a @ c
+    U, S, V = np.linalg.svd(M, full_matrices=False)
+    assert np.linalg.norm(c0[0] @ c1 - (U[:, :m] * S[:m]) @ V[:m]) < 1e-11 * np.linalg.norm(M)
+    lost = np.sum(S[m:] ** 2) / np.sum(S ** 2)
+    assert abs(err.value - lost) <= 1e-11
