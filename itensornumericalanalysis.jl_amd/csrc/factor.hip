@@ -2100,10 +2100,13 @@ __device__ __noinline__ void copy_doubles(double* D_in, const double* Y_in, int6
   }
 }
 
-// Rows up to which a matrix is factored (or its Q formed) in column groups, and
-// the entries above which helper workgroups, where there are any, share it
-// instead: a 256 x 128 QR takes 281 us shared and 175 us on one workgroup; a
-// 768 x 384 one 989 us shared, which is about what one workgroup would need.
+// Rows up to which a matrix is factored (or its Q formed) in column groups; and the
+// entries above which helper workgroups, where there are any, share the work
+// instead.  us of the factorization, alone / shared: 256 x 96 127 / 143, 256 x 128 180 /
+// 193, 128 x 160 152 / 167, 160 x 128 163 / 159, 200 x 160 229 / 220, but 700 x 32 101 / 70,
+// 512 x 64 141 / 116, 300 x 100 233 / 174, 300 x 140 317 / 231, 400 x 200 590 / 371, 768 x 384
+// 2461 / 982: a QR runs alone up to 256 rows.  Forming U alone is the faster up to
+// the limit whatever the rows (moves of 700 x 32 25 us less, 512 x 64 59, 400 x 100 81).
 constexpr int QC_ROWS = 1024;
 constexpr int64_t QC_SHARE = 40960;
 
@@ -2664,7 +2667,7 @@ __device__ __noinline__ void qr_panel(double* W, int rows_in, int cols_in, int l
   const int rows = uni(rows_in), cols = uni(cols_in), ld = uni(ld_in);
   const int k = rows < cols ? rows : cols;
   QTT_PT_INIT;
-  if (!(job != nullptr && nwg > 1) || (int64_t)rows * cols <= QC_SHARE) {
+  if (!(job != nullptr && nwg > 1) || (rows <= 256 && (int64_t)rows * cols <= QC_SHARE)) {
     if (rows <= 256) qr_cols<8, 2>(W, rows, cols, ld, tau, Tg, L);
     else if (rows <= 640) qr_cols<20, 2>(W, rows, cols, ld, tau, Tg, L);
     else qr_cols<32, 1>(W, rows, cols, ld, tau, Tg, L);
