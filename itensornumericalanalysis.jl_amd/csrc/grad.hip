@@ -3,16 +3,18 @@
 // where L_k is the product of the slices left of site k and R_k the product
 // right of it.
 //
-// Float64 chains run in tree.hip (launch_grad_chain).  Here: the float32
-// chain gradient (tiles of 128 points, environments in LDS, per-workgroup
-// partial gradients summed in a fixed order) and the float64 gradient of
-// general trees, bitwise reproducible run to run as well.
+// Float64 chains run in tree.hip (launch_grad_chain), small calls here
+// (grad_chain_reg_kernel, a lane per point).  Here too: the float32 chain gradient
+// (tiles of 128 points, environments in LDS, per-workgroup partial gradients summed
+// in a fixed order) and the float64 gradient of general trees, bitwise
+// reproducible run to run as well.
 #include "qtt_internal.h"
 #include "tree.h"
 
 namespace {
 
 constexpr int GB = 128;  // float32 chain kernel: points per tile = threads per workgroup
+constexpr int GT = 256;  // register kernel: the same
 
 __device__ inline uint64_t digit_word_g(double x, int L, bool& bad) {
   if (!(x >= 0.0)) {
@@ -135,6 +137,284 @@ grad_chain_kernel(const float* __restrict__ pack, const int64_t* __restrict__ po
       __syncthreads();
       for (int r = 0; r < chir; ++r) Lv[(size_t)r * GB + tid] = Nv[(size_t)r * GB + tid];
       __syncthreads();
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// A lane per point (float64 chains of sites with at most two values, bonds up to
+// 16; small calls, see lanes_faster), tiles of 256 points per workgroup:
+//   1. backward pass (last site to first) with the vector in registers; every
+//      R_k is parked in the workgroup's own global buffer (environments are
+//      recomputed per tile, never stored for the whole batch);
+//   2. forward pass rebuilds L_k in registers.  At each site the tile's L_k and
+//      ybar R_k are staged in LDS and reduced over the points: wavefront w
+//      takes site value s = w & 1 and half of the parent-bond rows, walks only
+//      the points whose digit is s (a scalar loop over the ballot of digits)
+//      and keeps a small block of (l, r) sums per lane; the block is added to
+//      the workgroup's own partial gradient (owner-computes, no atomics);
+//   3. a second kernel sums the partials in a fixed order, so the result is
+//      bitwise reproducible run to run.
+// ---------------------------------------------------------------------------
+__device__ inline double bsel(double a, double b, uint64_t mask) {
+  const uint64_t ua = (uint64_t)__double_as_longlong(a), ub = (uint64_t)__double_as_longlong(b);
+  return __longlong_as_double((long long)((ua & ~mask) | (ub & mask)));
+}
+
+__device__ inline uint64_t uniform64(uint64_t x) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
+  return ((uint64_t)hi << 32) | lo;
+}
+
+__device__ inline uint64_t site_digit_mask(const SiteDesc& sd, const uint64_t (&kw)[QTT_MAX_COORD]) {
+  if (sd.coord < 0) return 0;
+  const uint64_t kk = sd.coord == 0 ? kw[0] : sd.coord == 1 ? kw[1] : sd.coord == 2 ? kw[2] : kw[3];
+  return 0 - ((kk >> sd.shift) & 1u);
+}
+
+// v <- T[:, d, :] v over the child bond (packed site P[r][lpad][2]); entries
+// past the parent bond are left at zero.
+template <int CHI>
+__device__ __forceinline__ void step_to_parent(const double* __restrict__ P, const SiteDesc& sd, uint64_t dmask,
+                                               double (&v)[CHI]) {
+  const int lpad = (sd.chil + 3) & ~3;
+  double w[CHI];
+#pragma unroll
+  for (int l0 = 0; l0 < CHI; l0 += 4) {
+    if (l0 < sd.chil) {
+      double a0[4] = {0.0, 0.0, 0.0, 0.0}, a1[4] = {0.0, 0.0, 0.0, 0.0};
+      // rows in pairs, the next pair's scalar loads issued before this pair's
+      // multiply-adds (the packed core has rows up to the bond rounded up to 4,
+      // zero past the bond)
+      const double* __restrict__ Pl = P + l0 * 2;
+      const int rs = lpad * 2;
+      double qa[8], qb[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        qa[e] = Pl[e];
+        qb[e] = Pl[rs + e];
+      }
+#pragma unroll
+      for (int r = 0; r < CHI; r += 2) {
+        if (r != 0 && r >= sd.chir) break;
+        const int rn = r + 2 < sd.chir ? r + 2 : r;
+        double na[8], nb[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          na[e] = Pl[rn * rs + e];
+          nb[e] = Pl[(rn + 1) * rs + e];
+        }
+        const double vu = v[r], vw = v[r + 1];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          a0[i] = __builtin_fma(qa[2 * i], vu, a0[i]);
+          a1[i] = __builtin_fma(qa[2 * i + 1], vu, a1[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          a0[i] = __builtin_fma(qb[2 * i], vw, a0[i]);
+          a1[i] = __builtin_fma(qb[2 * i + 1], vw, a1[i]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          qa[e] = na[e];
+          qb[e] = nb[e];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[l0 + i] = bsel(a0[i], a1[i], dmask);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[l0 + i] = 0.0;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < CHI; ++i) v[i] = w[i];
+}
+
+// L <- L T[:, d, :] over the parent bond; entries past the child bond stay zero.
+template <int CHI>
+__device__ __forceinline__ void step_to_child(const double* __restrict__ P, const SiteDesc& sd, uint64_t dmask,
+                                              double (&L)[CHI]) {
+  const int lpad = (sd.chil + 3) & ~3;
+  double o[CHI];
+#pragma unroll
+  for (int r0 = 0; r0 < CHI; r0 += 4) {
+    if (r0 < sd.chir) {
+      double a0[4] = {0.0, 0.0, 0.0, 0.0}, a1[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int l0 = 0; l0 < CHI; l0 += 4) {
+        if (l0 == 0 || l0 < sd.chil) {  // at least one parent-bond entry: the first block always runs
+          // i outer, rr inner: consecutive multiply-adds go to 8 different
+          // accumulators (r, digit), so none waits on the one before
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+              const double* __restrict__ q = P + ((r0 + rr) * lpad + l0) * 2;
+              a0[rr] = __builtin_fma(q[2 * i], L[l0 + i], a0[rr]);
+              a1[rr] = __builtin_fma(q[2 * i + 1], L[l0 + i], a1[rr]);
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) o[r0 + rr] = bsel(a0[rr], a1[rr], dmask);
+    } else {
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) o[r0 + rr] = 0.0;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < CHI; ++i) L[i] = o[i];
+}
+
+// Reduction block of one lane: BL parent-bond rows x BR child-bond columns.
+template <int CHI>
+struct RedBlock {
+  static constexpr int BR = CHI >= 16 ? 2 : 1;
+  static constexpr int BL = 1;
+  static constexpr int NRB = CHI / BR;  // lanes along the child bond
+};
+
+template <int CHI>
+__global__ void __launch_bounds__(GT)
+grad_chain_reg_kernel(const double* __restrict__ pack, const int64_t* __restrict__ poff,
+                      const SiteDesc* __restrict__ desc, const int* __restrict__ sdim, int nv, int nc,
+                      const int* __restrict__ ndigits, const int64_t* __restrict__ goff,
+                      const int64_t* __restrict__ roff, int64_t rtot, const double* __restrict__ xs,
+                      const double* __restrict__ ybar, int64_t npts, int64_t gsize, double* __restrict__ Rscr,
+                      double* __restrict__ gpart, int* __restrict__ flag) {
+  // The tile's points are staged half at a time (HP = 128 points, two
+  // wavefronts), which halves the LDS footprint so that two workgroups share a
+  // compute unit.
+  constexpr int HP = GT / 2;
+  constexpr int LS = HP + 1;  // odd row stride: the rows read together sit in different banks
+  constexpr int BL = RedBlock<CHI>::BL, BR = RedBlock<CHI>::BR, NRB = RedBlock<CHI>::NRB;
+  extern __shared__ double lds[];
+  double* Ls = lds;                                    // [CHI][LS]  L_k per point of the half
+  double* Rs = lds + CHI * LS;                         // [CHI][LS]  ybar R_k per point of the half
+  uint64_t* bits = (uint64_t*)(lds + 2 * CHI * LS);    // [0, 2): digit ballots, [2, 4): active ballots
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int s_w = wv & 1;
+  const int lb = lane / NRB, rb = lane % NRB;
+  const bool lane_on = lb * BL < CHI / 2;
+  const int lrow0 = lane_on ? (wv >> 1) * (CHI / 2) + lb * BL : 0;
+  const int rcol0 = rb * BR;
+  double* R = Rscr + (size_t)blockIdx.x * rtot * GT;
+  double* G = gpart + (size_t)blockIdx.x * gsize;
+  for (int64_t e = tid; e < gsize; e += GT) G[e] = 0.0;
+  if (tid < CHI) {  // column HP is a zero point, paired with the last point of an odd count
+    Ls[tid * LS + HP] = 0.0;
+    Rs[tid * LS + HP] = 0.0;
+  }
+  const int64_t ntiles = (npts + GT - 1) / GT;
+  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const int64_t p = tile * GT + tid;
+    const bool active = p < npts;
+    bool bad = false;
+    uint64_t kw[QTT_MAX_COORD] = {0, 0, 0, 0};
+#pragma unroll
+    for (int c = 0; c < QTT_MAX_COORD; ++c)
+      if (c < nc) kw[c] = digit_word_g(active ? xs[p * nc + c] : 0.0, ndigits[c], bad);
+    if (bad) flag[0] = 1;
+    const double yb = (active && !bad) ? ybar[p] : 0.0;
+    // ---- backward: R_k over the child bond of site k, parked per tile ----
+    double v[CHI];
+#pragma unroll
+    for (int i = 0; i < CHI; ++i) v[i] = 0.0;
+    v[0] = 1.0;
+    for (int k = nv - 1; k >= 0; --k) {
+      const SiteDesc sd = desc[k];
+      double* Rk = R + roff[k] * GT + tid;
+#pragma unroll
+      for (int r = 0; r < CHI; ++r)
+        if (r < sd.chir) Rk[(int64_t)r * GT] = v[r];
+      if (k == 0) break;
+      step_to_parent<CHI>(pack + poff[k], sd, site_digit_mask(sd, kw), v);
+    }
+    // ---- forward: stage, reduce, advance L ----
+    double L[CHI];
+#pragma unroll
+    for (int i = 0; i < CHI; ++i) L[i] = 0.0;
+    L[0] = 1.0;
+    for (int k = 0; k < nv; ++k) {
+      const SiteDesc sd = desc[k];
+      const uint64_t dmask = site_digit_mask(sd, kw);
+      const double* Rk = R + roff[k] * GT + tid;
+      double rv[CHI];
+#pragma unroll
+      for (int i = 0; i < CHI; ++i) rv[i] = i < sd.chir ? yb * Rk[(int64_t)i * GT] : 0.0;
+      const uint64_t db = __ballot(dmask != 0 && active);
+      const uint64_t ab = __ballot(active);
+      const int sk = sdim[k];
+      double acc[BL][BR];
+#pragma unroll
+      for (int i = 0; i < BL; ++i)
+#pragma unroll
+        for (int q = 0; q < BR; ++q) acc[i][q] = 0.0;
+      for (int h = 0; h < 2; ++h) {
+        if ((wv >> 1) == h) {  // this half's two wavefronts stage their points
+          const int col = tid & (HP - 1);
+#pragma unroll
+          for (int i = 0; i < CHI; ++i) {
+            Ls[i * LS + col] = L[i];
+            Rs[i * LS + col] = rv[i];
+          }
+          if (lane == 0) {
+            bits[wv & 1] = db;
+            bits[2 + (wv & 1)] = ab;
+          }
+        }
+        __syncthreads();
+        if (s_w < sk) {
+          for (int c = 0; c < HP / 64; ++c) {
+            uint64_t m = bits[2 + c];
+            if (sk == 2) m = s_w ? (m & bits[c]) : (m & ~bits[c]);
+            m = uniform64(m);
+            while (m) {
+              const int ja = c * 64 + __builtin_ctzll(m);
+              m &= m - 1;
+              int jb = HP;
+              if (m) {
+                jb = c * 64 + __builtin_ctzll(m);
+                m &= m - 1;
+              }
+              double la[BL], lq[BL], ra[BR], rq[BR];
+#pragma unroll
+              for (int i = 0; i < BL; ++i) {
+                la[i] = Ls[(lrow0 + i) * LS + ja];
+                lq[i] = Ls[(lrow0 + i) * LS + jb];
+              }
+#pragma unroll
+              for (int q = 0; q < BR; ++q) {
+                ra[q] = Rs[(rcol0 + q) * LS + ja];
+                rq[q] = Rs[(rcol0 + q) * LS + jb];
+              }
+#pragma unroll
+              for (int i = 0; i < BL; ++i)
+#pragma unroll
+                for (int q = 0; q < BR; ++q) {
+                  acc[i][q] = __builtin_fma(la[i], ra[q], acc[i][q]);
+                  acc[i][q] = __builtin_fma(lq[i], rq[q], acc[i][q]);
+                }
+            }
+          }
+        }
+        __syncthreads();
+      }
+      if (s_w < sk && lane_on) {
+        double* Gk = G + goff[k];
+#pragma unroll
+        for (int i = 0; i < BL; ++i)
+#pragma unroll
+          for (int q = 0; q < BR; ++q) {
+            const int l = lrow0 + i, r = rcol0 + q;
+            if (l < sd.chil && r < sd.chir) Gk[((int64_t)l * sk + s_w) * sd.chir + r] += acc[i][q];
+          }
+      }
+      if (k + 1 < nv) step_to_child<CHI>(pack + poff[k], sd, dmask, L);
     }
   }
 }
@@ -448,6 +728,48 @@ int launch_apply_grad(qtt_ctx* ctx, const qtt_mpo* op, const qtt_net* net, const
   return qtt_hip_check(ctx, hipStreamSynchronize(ctx->stream), "apply gradient sync");
 }
 
+// Whether a lane per point (grad_chain_reg_kernel) beats the rows of tree.hip.  The
+// rows take some 60 launches, about 6 us per site, however few the points, and where
+// the digits outnumber the tables' (2 x 16 at most) each middle site of each point
+// costs a padded 16-wide row; a lane per point works through every site (both digit
+// slices) and grows with the points and the bond.  Both sides are
+// estimated in us from measurements at 4 to 40 sites, bonds 1 to 16 and 1 to 500,000
+// points, us by lanes / rows:
+//                       1 point     64          2,000       32,000      500,000
+//   4 sites, bond 2     30 / 49     35 / 64     52 / 71     80 / 111    345 / 770
+//   12 sites, bond 4    52 / 97     65 / 144    112 / 120   139 / 115   551 / 189
+//   12 sites, bond 16   159 / 97    179 / 147   235 / 118   308 / 115   1194 / 192
+//   28 sites, bond 4    93 / 170    125 / 230   230 / 282   263 / 315   952 / 284
+//   28 sites, bond 8    148 / 169   180 / 233   285 / 283   363 / 316   1381 / 286
+//   40 sites, bond 2    109 / 289   154 / 341   302 / 422   331 / 517   1181 / 3042
+//   40 sites, bond 16   528 / 287   581 / 340   770 / 407   1064 / 520  3649 / 3055
+// The rows keep what is within 5%.
+static bool lanes_faster(const qtt_net* net, int64_t npts, int64_t maxb) {
+  const HostTopo& t = net->t;
+  if (npts <= 0 || maxb > 16) return false;
+  double sites = 0.0, per_point = 0.4, entries = 0.0;
+  int digits = 0;
+  for (int k = 0; k < t.nv; k++) {
+    if (t.sdim[k] > 2) return false;
+    entries = (double)net->bond[k] * (k == t.nv - 1 ? 1.0 : (double)net->bond[k + 1]);
+    sites += 6.5 + 0.05 * entries;
+    per_point += 0.04 + 0.0004 * entries;
+    digits += t.vcoord[k] >= 0;
+  }
+  const double n = (double)npts;
+  // (a tile of few points walks fewer of them per site)
+  const double few = npts <= 4 ? (maxb <= 8 ? 0.47 : 0.66) : npts <= 64 ? (maxb <= 8 ? 0.58 : 0.8) : 1.0;
+  const double lanes = (21.0 + sites) * few + 1e-3 * n * per_point;
+  int tab = 0;  // digits of a table (tree.hip)
+  while (tab < 16 && (int64_t(4) << tab) <= npts) ++tab;
+  const int mid = std::max(0, digits - 2 * tab);  // sites whose rows are points
+  double rows = 45.0 + (tab ? 6.3 : 4.6) * t.nv;
+  if (tab && mid) rows += npts < 512 ? 15.0 : 60.0 + mid;
+  rows += 1e-3 * n * (digits <= 4 ? 1.4 : digits <= 8 ? 0.4 : 0.15);  // sorting the points
+  rows += 1e-3 * n * mid * (0.3 + 0.37 * std::min(1.0, n / 5e5));
+  return 1.05 * lanes < rows;
+}
+
 int launch_grad(qtt_ctx* ctx, const qtt_net* cnet, const double* xs, const double* ybar,
                 int64_t npts, double* grad, int precision) {
   qtt_net* net = const_cast<qtt_net*>(cnet);
@@ -468,8 +790,8 @@ int launch_grad(qtt_ctx* ctx, const qtt_net* cnet, const double* xs, const doubl
   const size_t fsz = f32 ? sizeof(float) : sizeof(double);
   const size_t lds = (size_t)3 * maxb * GB * fsz + GB * sizeof(int);
   if (lds > 160 * 1024) return qtt_fail(ctx, QTT_EINVAL, "gradient: bond dimension too large");
-  if (!f32) return launch_grad_chain(ctx, net, xs, ybar, npts, grad);
-  int rc = qtt_ensure_pack32(ctx, net);
+  if (!f32 && !lanes_faster(net, npts, maxb)) return launch_grad_chain(ctx, net, xs, ybar, npts, grad);
+  int rc = f32 ? qtt_ensure_pack32(ctx, net) : qtt_ensure_pack(ctx, net);
   if (rc) return rc;
   std::vector<int64_t> goff(nv), roff(nv);
   int64_t gsize = 0, rtot = 0;
@@ -479,25 +801,39 @@ int launch_grad(qtt_ctx* ctx, const qtt_net* cnet, const double* xs, const doubl
     roff[k] = rtot;
     rtot += (k == nv - 1) ? 1 : net->bond[k + 1];
   }
-  const int64_t ntiles = (npts + GB - 1) / GB;
-  int nwg = (int)std::max<int64_t>(1, std::min<int64_t>(ntiles, (int64_t)2 * ctx->cus));
-  size_t bytes = ((size_t)nwg * (rtot * GB + gsize) + 2 * nv + 16) * sizeof(double);
+  const int chi = maxb <= 8 ? 8 : 16, tilep = f32 ? GB : GT;
+  const size_t lds_reg = ((size_t)2 * chi * (GT / 2 + 1) + 4) * sizeof(double);
+  const int64_t ntiles = (npts + tilep - 1) / tilep;
+  const int per_cu = f32 ? 2 : std::max(1, std::min(4, (int)((160 * 1024) / lds_reg)));
+  int nwg = (int)std::max<int64_t>(1, std::min<int64_t>(ntiles, (int64_t)per_cu * ctx->cus));
+  size_t bytes = ((size_t)nwg * (rtot * tilep + gsize) + 2 * nv + 16) * sizeof(double);
   double* scr = qtt_scratch(ctx, bytes);
   if (!scr) return qtt_fail(ctx, QTT_ENOMEM, "gradient scratch");
   double* Rscr = scr;
-  double* gpart = Rscr + (size_t)nwg * rtot * GB;  // each workgroup parks rtot x GB values
+  double* gpart = Rscr + (size_t)nwg * rtot * tilep;  // each workgroup parks rtot x tilep values
   int64_t* d_goff = (int64_t*)(gpart + (size_t)nwg * gsize);
   int64_t* d_roff = d_goff + nv;
   rc = qtt_hip_check(ctx, hipMemcpyAsync(d_goff, goff.data(), nv * sizeof(int64_t), hipMemcpyHostToDevice, ctx->stream), "goff");
   if (!rc) rc = qtt_hip_check(ctx, hipMemcpyAsync(d_roff, roff.data(), nv * sizeof(int64_t), hipMemcpyHostToDevice, ctx->stream), "roff");
   if (rc) return rc;
   const TopoView tv = net->view();
-  if (lds > 64 * 1024) {
+  if (f32 && lds > 64 * 1024) {
     rc = qtt_hip_check(ctx, hipFuncSetAttribute((const void*)grad_chain_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
                        "grad LDS attribute");
     if (rc) return rc;
   }
-  if (npts > 0) {  // the float (hi, lo) pack, hi read; float vectors parked in the scratch
+  if (!f32) {  // (npts > 0)
+    const SiteDesc* dd = (const SiteDesc*)net->d_desc;
+#define QTT_GRAD_LAUNCH(C)                                                                                       \
+  grad_chain_reg_kernel<C><<<nwg, GT, lds_reg, ctx->stream>>>(net->d_pack, net->d_pack_off, dd, tv.sdim, nv,     \
+                                                              tv.ncoord, tv.ndigits, d_goff, d_roff, rtot, xs,   \
+                                                              ybar, npts, gsize, Rscr, gpart, ctx->flags())
+    if (chi == 8) QTT_GRAD_LAUNCH(8);
+    else QTT_GRAD_LAUNCH(16);
+#undef QTT_GRAD_LAUNCH
+    rc = qtt_hip_check(ctx, hipGetLastError(), "grad_chain_reg_kernel");
+    if (rc) return rc;
+  } else if (npts > 0) {  // the float (hi, lo) pack, hi read; float vectors parked in the scratch
     grad_chain_kernel<<<nwg, GB, lds, ctx->stream>>>((const float*)net->d_pack32, net->d_pack_off, net->d_bond, tv, d_goff,
                                                      d_roff, rtot, xs, ybar, npts, gsize, (float*)Rscr, gpart,
                                                      ctx->flags(), (int)maxb);

@@ -421,3 +421,34 @@ def test_truncate_thin_moves(q, eng, rng, s0, b, s1, maxdim):
     assert np.linalg.norm(c0[0] @ c1 - (U[:, :m] * S[:m]) @ V[:m]) < 1e-11 * np.linalg.norm(M)
     lost = np.sum(S[m:] ** 2) / np.sum(S ** 2)
     assert abs(err.value - lost) <= 1e-11
+
+
+# ------------------------------------------------------------------ small gradients and inner products
+@pytest.mark.parametrize("bond", [1, 2, 3, 8, 9, 16])
+@pytest.mark.parametrize("dims,L,npts", [(1, 4, 1), (1, 4, 255), (2, 4, 256), (3, 3, 257), (2, 12, 64), (1, 16, 65),
+                                         (2, 20, 700)])
+def test_gradient_small(q, po, eng, rng, bond, dims, L, npts):
+    # a lane per point (small calls) and rows of digit strings, on both sides of the
+    # line between them, with tiles that the points do not fill
+    f = q.random_itn(_chain(q, L, bond, dims), link_space=bond, rng=rng, std=1.0 / math.sqrt(bond))
+    xs, yb = rng.uniform(0, 1, (npts, dims)), rng.standard_normal(npts)
+    xs[0] = 1.0
+    t = f.topo
+    ref = po.eval_grad(t.parent, t.sdim, f.cores, t.vcoord, t.vdigit, t.Lc, xs, yb)
+    g = q.eval_grad(f, xs, yb)
+    num = math.sqrt(sum(np.sum((a - b) ** 2) for a, b in zip(g, ref)))
+    assert num <= TOL * math.sqrt(sum(np.sum(b ** 2) for b in ref))
+    assert all(np.array_equal(a, b) for a, b in zip(g, q.eval_grad(f, xs, yb)))
+
+
+@pytest.mark.parametrize("kind,ba,bb", [("chain", 1, 1), ("chain", 2, 3), ("chain", 8, 7), ("chain", 11, 9),
+                                        ("chain", 12, 12), ("comb", 2, 2), ("comb", 6, 4), ("comb", 4, 9), ("star", 2, 3),
+                                        ("star", 4, 4), ("single", 1, 1)])
+def test_inner_small(q, po, eng, rng, kind, ba, bb):
+    # one workgroup (small networks) and a launch per height, around the line between them
+    s = _chain(q, 1 if kind == "single" else 13, 2) if kind in ("chain", "single") else _tree(q, kind)
+    f, g = (q.random_itn(s, link_space=b, rng=rng, std=1.0 / b) for b in (ba, bb))
+    t = f.topo
+    ref = po.inner(t.parent, t.sdim, f.cores, g.cores)
+    na, nb = (po.inner(t.parent, t.sdim, h.cores, h.cores) for h in (f, g))
+    assert abs(q.inner(f, g) - ref) <= TOL * math.sqrt(na * nb)
