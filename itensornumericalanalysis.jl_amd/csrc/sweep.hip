@@ -5,7 +5,7 @@
 // The fold over s is fused into the contraction, so each core is read once.
 // inner(a, b) (src/integration.jl:20-32 for the <Sigma|op|f> form) builds
 // E_v[pa][pb] = sum A[pa][s][ca..] B[pb][s][cb..] prod E_c[ca][cb] as matrix
-// products over many workgroups.
+// products over many workgroups, or of small networks by one workgroup.
 #include "qtt_internal.h"
 
 #include <algorithm>
@@ -315,6 +315,68 @@ __global__ void __launch_bounds__(256) integrate_flow_kernel(FlowArgs a) {
       a.sync[2] = 0;
     }
   }
+}
+
+// Inner product of small networks: one workgroup walks all vertices, children first
+// (mode products one child at a time, then a row-by-row dot product); see
+// inner_alone for where the line lies.
+__global__ void __launch_bounds__(512)
+inner_tree_kernel(const double* __restrict__ A, const int64_t* __restrict__ aoff,
+                  const int* __restrict__ abond, const double* __restrict__ B,
+                  const int64_t* __restrict__ boff, const int* __restrict__ bbond, TopoView t,
+                  const int64_t* __restrict__ eoff, double* E, double* Y0, double* Y1, double* out) {
+  const int tid = threadIdx.x, bs = blockDim.x;
+  const int lane = tid & 63, wid = tid >> 6, nw = bs >> 6;
+  for (int v = t.nv - 1; v >= 0; --v) {
+    const int m = t.nch[v];
+    const int* ch = t.chs + t.choff[v];
+    int64_t dims[QTT_MAX_NDIM];
+    const int nd = 2 + m;
+    dims[0] = bbond[v];
+    dims[1] = t.sdim[v];
+    for (int k = 0; k < m; ++k) dims[2 + k] = bbond[ch[k]];
+    const double* cur = B + boff[v];
+    double* bufs[2] = {Y0, Y1};
+    int which = 0;
+    for (int k = 0; k < m; ++k) {
+      const int ax = 2 + k;
+      int64_t Apre = 1, Bpost = 1;
+      for (int i = 0; i < ax; ++i) Apre *= dims[i];
+      for (int i = ax + 1; i < nd; ++i) Bpost *= dims[i];
+      const int64_t nold = dims[ax];
+      const int64_t nnew = abond[ch[k]];
+      const double* Ec = E + eoff[ch[k]];  // [ca][cb]
+      double* nxt = bufs[which];
+      const int64_t total = Apre * nnew * Bpost;
+      for (int64_t e = tid; e < total; e += bs) {
+        const int64_t bb = e % Bpost;
+        const int64_t rest = e / Bpost;
+        const int64_t j = rest % nnew;
+        const int64_t a = rest / nnew;
+        double s = 0.0;
+        for (int64_t i = 0; i < nold; ++i) s += Ec[j * nold + i] * cur[(a * nold + i) * Bpost + bb];
+        nxt[e] = s;
+      }
+      __syncthreads();
+      cur = nxt;
+      which ^= 1;
+      dims[ax] = nnew;
+    }
+    // E_v[pa][pb] = sum_rest A[pa][rest] Y[pb][rest]
+    int64_t rest = 1;
+    for (int i = 1; i < nd; ++i) rest *= dims[i];
+    const double* Av = A + aoff[v];
+    const int na = abond[v], nb = bbond[v];
+    for (int pr = wid; pr < na * nb; pr += nw) {
+      const int pa = pr / nb, pb = pr % nb;
+      double s = 0.0;
+      for (int64_t r = lane; r < rest; r += 64) s += Av[(int64_t)pa * rest + r] * cur[(int64_t)pb * rest + r];
+      s = wave_sum(s);
+      if (lane == 0) E[eoff[v] + pr] = s;
+    }
+    __syncthreads();
+  }
+  if (tid == 0) out[0] = E[eoff[0]];
 }
 
 // ---------------------------------------------------------------------------
@@ -755,7 +817,67 @@ int launch_integrate_batch(qtt_ctx* ctx, int n, const qtt_net* const* nets, doub
   return qtt_hip_check(ctx, hipStreamSynchronize(ctx->stream), "integrate batch sync");
 }
 
+static int inner_one_workgroup(qtt_ctx* ctx, const qtt_net* a, const qtt_net* b, double* out_host) {
+  const HostTopo& t = a->t;
+  std::vector<int64_t> eoff(t.nv);
+  int64_t etot = 0, ymax = 1;
+  for (int v = 0; v < t.nv; v++) {
+    eoff[v] = etot;
+    etot += a->bond[v] * b->bond[v];
+    // largest intermediate: the B core with any subset of child bonds replaced by A's
+    int64_t s = b->bond[v] * t.sdim[v];
+    for (int k = 0; k < t.nch[v]; k++) {
+      int c = t.chs[t.choff[v] + k];
+      s *= std::max(a->bond[c], b->bond[c]);
+    }
+    ymax = std::max(ymax, s);
+  }
+  size_t bytes = (2 + etot + 2 * ymax) * sizeof(double) + t.nv * sizeof(int64_t) + 64;
+  double* scr = qtt_scratch(ctx, bytes);
+  if (!scr) return qtt_fail(ctx, QTT_ENOMEM, "inner scratch");
+  double* d_out = scr;
+  double* E = scr + 2;
+  double* Y0 = E + etot;
+  double* Y1 = Y0 + ymax;
+  int64_t* d_eoff = (int64_t*)(Y1 + ymax);
+  int rc = qtt_hip_check(ctx, hipMemcpyAsync(d_eoff, eoff.data(), t.nv * sizeof(int64_t), hipMemcpyHostToDevice, ctx->stream), "eoff");
+  if (rc) return rc;
+  inner_tree_kernel<<<1, 512, 0, ctx->stream>>>(a->d_data, a->d_off, a->d_bond, b->d_data, b->d_off, b->d_bond,
+                                                a->view(), d_eoff, E, Y0, Y1, d_out);
+  rc = qtt_hip_check(ctx, hipGetLastError(), "inner_tree_kernel");
+  if (rc) return rc;
+  rc = qtt_hip_check(ctx, hipMemcpyAsync(out_host, d_out, sizeof(double), hipMemcpyDeviceToHost, ctx->stream), "inner");
+  if (rc) return rc;
+  return qtt_hip_check(ctx, hipStreamSynchronize(ctx->stream), "inner sync");
+}
+
+// Whether one workgroup (inner_tree_kernel) beats a launch per height: it takes
+// some 1.6 us per vertex and 1 ns per multiply-add of its products, the launches 8 us
+// per height.  us, one workgroup / launches: chains of 12 sites, bond 2 47 / 118, 8
+// 91 / 119, 16 253 / 122; of 40 sites, bond 2 96 / 316, 4 125 / 327, 8 249 / 317, 16
+// 832 / 326; combs of 3 x 6, bond 4 70 / 116, 8 129 / 115; 3 x 16, bond 4 144 / 194.
+static bool inner_alone(const qtt_net* a, const qtt_net* b) {
+  const HostTopo& t = a->t;
+  std::vector<int> height(t.nv, 0);
+  double ns = 0.0;
+  int top = 0;
+  for (int v = t.nv - 1; v >= 0; v--) {
+    double cur = (double)b->bond[v] * t.sdim[v], work = 0.0;
+    for (int k = 0; k < t.nch[v]; k++) cur *= b->bond[t.chs[t.choff[v] + k]];
+    for (int k = 0; k < t.nch[v]; k++) {  // the mode products of b's core, then the dot products
+      const int c = t.chs[t.choff[v] + k];
+      work += cur * a->bond[c];
+      cur = cur / b->bond[c] * a->bond[c];
+    }
+    ns += 1600.0 + work + cur * a->bond[v];
+    if (v) height[t.parent[v]] = std::max(height[t.parent[v]], height[v] + 1);
+    top = std::max(top, height[v]);
+  }
+  return ns < 8000.0 * (top + 1);
+}
+
 int launch_inner(qtt_ctx* ctx, const qtt_net* a, const qtt_net* b, double* out_host) {
+  if (inner_alone(a, b)) return inner_one_workgroup(ctx, a, b, out_host);
   const HostTopo& t = a->t;
   auto pad = [](int64_t x) { return (x + 15) & ~int64_t(15); };
   // heights (vertices of equal height run together), environments, the
