@@ -933,8 +933,8 @@ int launch_inner(qtt_ctx* ctx, const qtt_net* a, const qtt_net* b, double* out_h
     q.npb = (q.nb + 16 * q.gw - 1) / (16 * q.gw);
     const int64_t pairs = q.sq * q.nslab;
     const int64_t blocks = ((q.na + 15) / 16) * (int64_t)q.npb;
-    if (pairs >= (int64_t(1) << 31) || blocks >= (int64_t(1) << 24))
-      return qtt_fail(ctx, QTT_EINVAL, "inner: a core is too large");
+    if (pairs >= (int64_t(1) << 31) || blocks >= (int64_t(1) << 24))  // beyond the launches' 32-bit indices
+      return inner_one_workgroup(ctx, a, b, out_host);
     // a chunk keeps at least 4 pairs (a chain's two digit values stay together)
     const int64_t want = std::max<int64_t>(1, std::min<int64_t>(ctx->cus / blocks, pairs / 4));
     q.per = (int)((pairs + want - 1) / want);
@@ -981,7 +981,7 @@ int launch_inner(qtt_ctx* ctx, const qtt_net* a, const qtt_net* b, double* out_h
           if (i < k) apre *= a->bond[w];
           else if (i > k) bpost *= b->bond[w];
         }
-        if (apre * bpost >= (int64_t(1) << 31)) return qtt_fail(ctx, QTT_EINVAL, "inner: a core is too large");
+        if (apre * bpost >= (int64_t(1) << 31)) return inner_one_workgroup(ctx, a, b, out_host);
         js.unit0[js.n] = units;
         InnerMode& J = js.job[js.n++];
         J.E = E + eoff[c];

@@ -715,7 +715,7 @@ int tree_pack(qtt_ctx* ctx, qtt_net* net) {
       if (i + 1 < p.in.size()) q *= dim;
       else p.kbl = (int)((dim + 15) / 16);
     }
-    if (q * p.kbl >= (int64_t(1) << 27)) return qtt_fail(ctx, QTT_EINVAL, "evaluate: a core is too large");
+    if (q * p.kbl >= (int64_t(1) << 30)) return qtt_fail(ctx, QTT_EINVAL, "evaluate: a core is too large");
     p.nk = (int)(q * p.kbl);
     p.slices = t.vcoord[v] >= 0 ? 2 : 1;
     p.pack = tot;
