@@ -375,8 +375,7 @@ def other_workloads(q, po, ctx, stream, args):
     den = sum(float(np.sum(b ** 2)) for b in ref) ** 0.5
     out["fit_2d"] = {"gradient_ms": gt * 1e3, "points": len(w4.xs),
                       "forward_flops_per_point": flops_fwd,
-                      "gradient_tflops_3x_forward": 3 * flops_fwd * len(w4.xs) / gt / 1e12,
-                      "gradient_note": "flops of one point at a time; points that share digits share their rows, so fewer are executed",
+                      "gradient_points_per_s": len(w4.xs) / gt,
                       "grad_rel_err_vs_oracle_2^14_subset": num / den}
     # 3D comb: 3 x 16 digits, dense random cores of bond 128 (45 MB), d/dx then
     # truncation to maxdim 128, and the full integral (dataflow kernel)

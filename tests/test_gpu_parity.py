@@ -278,6 +278,10 @@ def test_eval_float32_paths(q, po, eng, prec, tol):
     err = rel_l2(y, ref)
     print(f"precision {prec}: rel L2 error vs float64 oracle {err:.3e}")
     assert err < tol
+    # every precision is computed in float64: the same bits, few points and many
+    for n in (1, 5000, 20000):
+        assert np.array_equal(q.evaluate(w.f, w.xs[:n], precision=prec), q.evaluate(w.f, w.xs[:n]))
+    assert err < 1e-12
 
 
 # ------------------------------------------------------------------ integrate / inner
