@@ -940,9 +940,9 @@ __device__ inline int rr_player(int pos, int t, int nn) {
 // orthogonal to each other, as slowly as their norms are close.  (Matrices with
 // most singular values within a factor of 3 of the level: of 12 x 24 ones 1 in 20
 // was not done in 60 sweeps, of 110 x 140 ones all; they then take some 8 sweeps
-// more.)  Not fewer: a graded matrix that converges under the rule takes up to 15 or
-// so, and rotating its smallest rows against each other, 8 more.
-constexpr int JACOBI_NOISE_SWEEPS = 20;
+// more.)  Not fewer: graded matrices that converge under the rule take up to 21 (bond
+// 32 chains and combs at 1e-10), and rotating their smallest rows too, 8 more.
+constexpr int JACOBI_NOISE_SWEEPS = 32;
 __device__ inline double noise_level(double fro2, double cut, int n) {
   return (cut > 0.0 && cut < 1.0) ? cut * fro2 / (double)n : 0.0;
 }

@@ -563,7 +563,7 @@ int or_qr(int r, int c, const double* M, double* Q, double* R) {
  * cut rotates every pair.  init_j = 0 continues from the rotations in J.
  * The rule ends after NOISE_SWEEPS sweeps: rows just above the level converge
  * only linearly against rows below it that are not orthogonal to each other. */
-#define NOISE_SWEEPS 20
+#define NOISE_SWEEPS 32
 static int jacobi_rows(int n, int c, double* X, double* J, double cut, int init_j) {
   if (init_j)
     for (int i = 0; i < n; i++)
