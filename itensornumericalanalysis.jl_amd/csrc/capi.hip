@@ -275,14 +275,17 @@ int qtt_ctx_create(int device, qtt_ctx** out) {
   c->device = device;
   if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&c->own_stream) != hipSuccess ||
       hipMalloc(&c->d_flag, 4 * sizeof(int)) != hipSuccess ||
-      hipMemset(c->d_flag, 0, 4 * sizeof(int)) != hipSuccess) {
+      hipMemset(c->d_flag, 0, 4 * sizeof(int)) != hipSuccess ||
+      hipHostMalloc(&c->h_inf, sizeof(int)) != hipSuccess) {
     (void)hipGetLastError();
+    if (c->d_flag) (void)hipFree(c->d_flag);
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
     delete c;
     return QTT_EHIP;
   }
   if (qtt_noalloc_init(c) != QTT_OK) {  // the device address of the fixed scratch, with the device current
     (void)hipFree(c->d_flag);
+    (void)hipHostFree(c->h_inf);
     (void)hipStreamDestroy(c->own_stream);
     delete c;
     return QTT_EHIP;
@@ -319,6 +322,7 @@ static void ctx_free(qtt_ctx* ctx) {
   if (ctx->d_sync) (void)hipFree(ctx->d_sync);
   if (ctx->scratch_ev) (void)hipEventDestroy(ctx->scratch_ev);
   if (ctx->d_flag) (void)hipFree(ctx->d_flag);
+  if (ctx->h_inf) (void)hipHostFree(ctx->h_inf);
   if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
   delete ctx;
 }

@@ -728,6 +728,13 @@ int launch_apply_grad(qtt_ctx* ctx, const qtt_mpo* op, const qtt_net* net, const
   return qtt_hip_check(ctx, hipStreamSynchronize(ctx->stream), "apply gradient sync");
 }
 
+// the networks of grad_chain_reg_kernel
+static bool lanes_take(const qtt_net* net, int64_t maxb) {
+  for (int k = 0; k < net->t.nv; k++)
+    if (net->t.sdim[k] > 2) return false;
+  return maxb <= 16;
+}
+
 // Whether a lane per point (grad_chain_reg_kernel) beats the rows of tree.hip.  The
 // rows take some 60 launches, about 6 us per site, however few the points, and where
 // the digits outnumber the tables' (2 x 16 at most) each middle site of each point
@@ -746,11 +753,10 @@ int launch_apply_grad(qtt_ctx* ctx, const qtt_mpo* op, const qtt_net* net, const
 // The rows keep what is within 5%.
 static bool lanes_faster(const qtt_net* net, int64_t npts, int64_t maxb) {
   const HostTopo& t = net->t;
-  if (npts <= 0 || maxb > 16) return false;
+  if (npts <= 0 || !lanes_take(net, maxb)) return false;
   double sites = 0.0, per_point = 0.4, entries = 0.0;
   int digits = 0;
   for (int k = 0; k < t.nv; k++) {
-    if (t.sdim[k] > 2) return false;
     entries = (double)net->bond[k] * (k == t.nv - 1 ? 1.0 : (double)net->bond[k + 1]);
     sites += 6.5 + 0.05 * entries;
     per_point += 0.04 + 0.0004 * entries;
@@ -782,15 +788,25 @@ int launch_grad(qtt_ctx* ctx, const qtt_net* cnet, const double* xs, const doubl
   for (int k = 0; k < nv; k++) maxb = std::max(maxb, net->bond[k]);
   if (!t.chain || t.ncoord > QTT_MAX_COORD) {
     if (f32) return qtt_fail(ctx, QTT_EINVAL, "gradient: float32 is implemented for chains");
-    if (t.chain && maxb <= 64) return launch_grad_chain(ctx, net, xs, ybar, npts, grad);
-    return launch_grad_tree(ctx, net, xs, ybar, npts, grad);
+    bool by_tree = !t.chain || maxb > 64;
+    if (!by_tree) {
+      const int rc = launch_grad_chain(ctx, net, xs, ybar, npts, grad, &by_tree);
+      if (rc) return rc;
+    }
+    return by_tree ? launch_grad_tree(ctx, net, xs, ybar, npts, grad) : QTT_OK;
   }
   // three vectors of 128 points in LDS (the float64 path has no such need; it
   // refuses the same bonds as before)
   const size_t fsz = f32 ? sizeof(float) : sizeof(double);
   const size_t lds = (size_t)3 * maxb * GB * fsz + GB * sizeof(int);
   if (lds > 160 * 1024) return qtt_fail(ctx, QTT_EINVAL, "gradient: bond dimension too large");
-  if (!f32 && !lanes_faster(net, npts, maxb)) return launch_grad_chain(ctx, net, xs, ybar, npts, grad);
+  if (!f32 && !lanes_faster(net, npts, maxb)) {
+    bool inf_weight = false;
+    const int rc = launch_grad_chain(ctx, net, xs, ybar, npts, grad, &inf_weight);
+    if (rc || !inf_weight) return rc;
+    // again, by a kernel that multiplies by the weight last
+    if (!lanes_take(net, maxb)) return launch_grad_tree(ctx, net, xs, ybar, npts, grad);
+  }
   int rc = f32 ? qtt_ensure_pack32(ctx, net) : qtt_ensure_pack(ctx, net);
   if (rc) return rc;
   std::vector<int64_t> goff(nv), roff(nv);

@@ -32,6 +32,9 @@ struct qtt_ctx {
   int* d_flag = nullptr;
   int flag_base = 0;  // 0 (asynchronous) or 2 (inside a synchronous entry point)
   int* flags() const { return d_flag + flag_base; }
+  // a word of host memory that a chain gradient's kernels set where a weight is
+  // infinite (read after the call's own wait; no copy)
+  int* h_inf = nullptr;
   // Networks and operators keep their context alive: qtt_ctx_destroy only
   // marks it closed while handles remain, and the last handle destroyed frees it.
   int refs = 0;

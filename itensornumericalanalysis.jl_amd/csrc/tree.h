@@ -8,5 +8,8 @@
 int launch_eval_tree(qtt_ctx* ctx, qtt_net* net, const double* xs, int64_t npts, double* out);
 
 // Gradient of sum_m ybar_m f(x_m) with respect to the cores of a float64 chain
-// with bonds of at most 64 (device pointers; waits for the result).
-int launch_grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double* ybar, int64_t npts, double* grad);
+// with bonds of at most 64 (device pointers; waits for the result).  *inf_weight
+// is set if a weight is infinite: the caller then takes a kernel that multiplies
+// by the weight last (see grad_weight_kernel).
+int launch_grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double* ybar, int64_t npts, double* grad,
+                      bool* inf_weight);

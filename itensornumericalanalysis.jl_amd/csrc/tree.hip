@@ -1110,17 +1110,22 @@ constexpr int SORT_BITS = 8, SORT_BINS = 1 << SORT_BITS;
 constexpr int GRAD_KEYS = 2;       // tables that points meet (one per side of the centre)
 constexpr int RUN = 64;            // sorted positions summed by one group of lanes
 
-// ybar, zero (and the flag) at points with a negative or NaN coordinate
+// ybar, zero (and the flag) at points with a negative or NaN coordinate.  An
+// infinite weight sets *inf, a word of host memory that is read once the call
+// has waited: here a weight meets the row of one side before that row passes
+// the other side's cores, whose sums would turn infinities of both signs into NaN.
 __global__ void __launch_bounds__(256)
 grad_weight_kernel(const double* __restrict__ xs, const double* __restrict__ ybar, int64_t npts, int nc,
-                   double* __restrict__ w, int* __restrict__ flag) {
+                   double* __restrict__ w, int* __restrict__ flag, int* __restrict__ inf) {
   const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (p >= npts) return;
   bool bad = false;
   for (int c = 0; c < nc; ++c)
     if (!(xs[p * nc + c] >= 0.0)) bad = true;
   if (bad) flag[0] = 1;
-  w[p] = bad ? 0.0 : ybar[p];
+  const double y = bad ? 0.0 : ybar[p];
+  if (isinf(y)) *inf = 1;
+  w[p] = y;
 }
 
 __global__ void grad_zero_kernel(double* __restrict__ a, int64_t na, unsigned char* __restrict__ b, int64_t nb) {
@@ -1773,7 +1778,7 @@ static int grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double
     const int64_t np = std::min(chunk, npts - p0);
     const double* x0 = xs + p0 * nc;
     const unsigned nb = (unsigned)((np + 255) / 256);
-    grad_weight_kernel<<<nb, 256, 0, ctx->stream>>>(x0, ybar + p0, np, nc, wts, ctx->flags());
+    grad_weight_kernel<<<nb, 256, 0, ctx->stream>>>(x0, ybar + p0, np, nc, wts, ctx->flags(), ctx->h_inf);
     if ((rc = qtt_hip_check(ctx, hipGetLastError(), "grad_weight_kernel"))) return rc;
     if ((rc = c.index(np, x0))) return rc;
     if (c.any_point && (rc = c.forward(false, 0, np, x0))) return rc;
@@ -1903,12 +1908,17 @@ static int grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double
   return qtt_hip_check(ctx, hipStreamSynchronize(ctx->stream), "grad sync");
 }
 
-int launch_grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double* ybar, int64_t npts, double* grad) {
+int launch_grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double* ybar, int64_t npts, double* grad,
+                      bool* inf_weight) {
   int rc = tree_enter(ctx, net);
   if (rc) return rc;
+  *ctx->h_inf = 0;  // (a call that failed half-way may set it late: the other kernel runs, the results are right)
   rc = grad_chain(ctx, net, xs, ybar, npts, grad);
   const int rl = tree_leave(ctx, net);
-  if (!rc) return rl;
+  if (!rc) {
+    *inf_weight = *(volatile int*)ctx->h_inf != 0;
+    return rl;
+  }
   const int rq = qtt_scratch_queued(ctx);  // it may have failed with work queued
   (void)rq;
   return rc;

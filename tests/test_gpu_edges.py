@@ -121,6 +121,29 @@ def test_gradient_infinite_weight(q, po, eng, rng, bond, npts):
         assert rel_l2(g[:, 1 - d], r[:, 1 - d]) < TOL
 
 
+@pytest.mark.parametrize("bond", [3, 5, 16, 17, 40, 53])
+@pytest.mark.parametrize("npts", [1, 7, 300, 5000])
+def test_gradient_infinite_weight_signs(q, po, eng, rng, bond, npts):
+    # cores of both signs: a weight is the last factor of its sample's term, so one
+    # infinite weight gives infinities of the term's sign and no NaN
+    f = q.random_itn(_chain(q, 13, 2), link_space=bond, rng=rng)
+    xs, yb = rng.uniform(0, 1, (npts, 1)), rng.uniform(-1.5, 1.5, npts)
+    yb[npts // 2] = -np.inf
+    t = f.topo
+    ref = po.eval_grad(t.parent, t.sdim, f.cores, t.vcoord, t.vdigit, t.Lc, xs, yb)
+    for g, r in zip(q.eval_grad(f, xs, yb), ref):
+        inf = np.isinf(r)
+        assert inf.any() and not np.isnan(r).any()
+        assert np.array_equal(g[inf], r[inf])
+        if not inf.all():
+            assert rel_l2(g[~inf], r[~inf]) < TOL
+    # the calls after it are what they were
+    yb[npts // 2] = 0.5
+    ref = po.eval_grad(t.parent, t.sdim, f.cores, t.vcoord, t.vdigit, t.Lc, xs, yb)
+    for g, r in zip(q.eval_grad(f, xs, yb), ref):
+        assert rel_l2(g, r) < TOL
+
+
 # ------------------------------------------------------------------ NaN
 @pytest.mark.parametrize("bond,cutoff,maxdim", [(6, 1e-10, 1 << 30), (24, 1e-10, 20), (40, 0.0, 16), (80, 1e-8, 64),
                                                 (110, 0.0, 60)])
