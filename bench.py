@@ -209,7 +209,7 @@ def main():
     # environment tables: the tuned size, else the launcher's rule (from 2^15 points)
     lg = min(21, int(args.npts).bit_length() - 1)
     tbits = tuned["table_digits"] if tuned else (
-        0 if lg < 15 else 16 if lg == 21 else max(12, min(lg - 5, 16 if chi <= 8 else 13 if max(bonds) <= 20 else 12)))
+        0 if lg < 15 else 16 if lg == 21 or (lg >= 19 and 8 < max(bonds) <= 16) else max(12, min(lg - 5, 16 if chi <= 8 else 13 if max(bonds) <= 20 else 12)))
     if chi <= 32 and tbits > 0:
         kname = (f"eval_chain_env{'2' if chi <= 16 and ppl == 2 else ''}_kernel<{chi}> "
                  f"(env_table_kernel ran once, at the network's first evaluate)")

@@ -962,11 +962,16 @@ static EnvPlan env_plan(const qtt_net* net, int tb) {
 // as many as leave a row reused about 32 times, at least 12, and at most what the
 // L2 of an XCD holds beside the rest (two tables of some 2 MB: 12 digits up to bond
 // 32, 13 up to bond 20, 16 up to bond 8, whose small rows cost little from beyond it
-// too).  From 2^21 points 16 digits, their middle sites saved being worth more than
-// the L2.  A network's first call allocates and builds the tables too.  us per call,
-// 40 sites, 12 / 13 / 14 / 15 / 16 digits, called back to back on the same points
-// (with other points each time 10^6 points of bond 16 take longer, 383 against 337
-// with 12 digits):
+// too).  Bonds 9 to 16 take 16 digits from 2^19 points and all bonds from 2^21, the
+// middle sites saved being worth more than the L2: faster than 12 to 14 in a
+// network's first call (which allocates and builds the tables) and in later ones;
+// below, building them costs what they save (3 10^5 points of bond 12, first / later:
+// 160 / 77 us with 12, 181 / 59 with 16).  First / later call with other points each
+// time, us, 40 sites, 12 / 13 / 14 / 16 digits:
+//                       bond 9                              bond 16
+//   524,288 points      228/117  222/109  238/110  216/106  391/215  389/194  367/242  333/194
+//   10^6 points         270/177  258/164  308/197  261/143  471/336  463/305  516/397  437/293
+// Called back to back on the same points, 12 / 13 / 14 / 15 / 16 digits:
 //             10^6 points                      2 10^6 (bonds 4, 16, 32: 2^21)
 //   bond 4    47 / 43 / 41 / 45 / 43           79 / 75 / 71 / 67 / 67
 //   bond 8    108 / 98 / 89 / 86 / 80          195 / 178 / 162 / 152 / 138
@@ -975,15 +980,14 @@ static EnvPlan env_plan(const qtt_net* net, int tb) {
 //   bond 20   692 / 617 / 880 / 847 / 723      1279 / 1137 / 1760 / 1584 / 1325
 //   bond 32   1676 / 2348 / 2355 / 2036 / 1662 3347 / 4986 / 4452 / 3750 / 3057
 // 10^7 points of bond 16: 2967 / 2644 / 3492 / 3133 / 2556.  A new network's first
-// call, 10^6 points of bond 16: 530 / 488 / 548 / - / 463; of bond 20: 980 / 884 /
-// 1109 / - / 930.  (16 digits are the fastest in many places, but every network keeps
-// its tables: 17 MB at bond 16 where 13 digits are 2.  qtt_tune_eval chooses among
-// all sizes for a program that repeats a call.)
+// call, 10^6 points of bond 20: 980 / 884 / 1109 / - / 930.  (A network keeps its
+// tables, 17 MB at 16 digits and bond 16.  qtt_tune_eval chooses among all sizes for
+// a program that repeats a call.)
 static int default_table_bits(int64_t npts, int64_t maxb) {
   if (npts < (int64_t(1) << 15)) return 0;
   int lg = 15;
   while (lg < 21 && (int64_t(1) << (lg + 1)) <= npts) ++lg;
-  if (lg == 21) return 16;
+  if (lg == 21 || (lg >= 19 && maxb > 8 && maxb <= 16)) return 16;
   return std::max(12, std::min(lg - 5, maxb <= 8 ? 16 : maxb <= 20 ? 13 : 12));
 }
 
