@@ -1905,7 +1905,12 @@ static int grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double
     wave = next;
   }
   if ((rc = cores_of(true, 0, nullptr, false))) return rc;
-  return qtt_hip_check(ctx, hipStreamSynchronize(ctx->stream), "grad sync");
+  rc = qtt_hip_check(ctx, hipStreamSynchronize(ctx->stream), "grad sync");
+  if (!rc) {  // what it made, and what it waited for in tree_enter, is done: nothing to order by an event
+    S.making = false;
+    S.ev_stream = nullptr;
+  }
+  return rc;
 }
 
 int launch_grad_chain(qtt_ctx* ctx, qtt_net* net, const double* xs, const double* ybar, int64_t npts, double* grad,
